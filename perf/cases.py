@@ -215,8 +215,8 @@ def tolerance(case):
     op = case["op"]
     if op in ("transpose", "nw"):
         return "exact"
-    if op == "stencil":      # fp32 sums of up to 343 products: rel 6e-8 to 2e-7
-        return {"rel": 1e-6, "max": 4e-6}
+    if op == "stencil":      # fp32 sums of up to 344 products one after another: rel 3.3e-7, max 2.2e-6
+        return {"rel": 1.3e-6, "max": 8.7e-6}
     if op == "lud":          # n = 4096: rel 3.9e-7, max 1.2e-6
         return {"rel": 1.6e-6, "max": 4.6e-6}
     out = {"gemm": case.get("out"), "grouped": "f16"}.get(op) or case["dtype"]
