@@ -223,3 +223,97 @@ def tolerance(case):
     if out == "f32":         # softmax rel 8e-8, max 3.6e-7; gradients of LayerNorm over 1216 rows rel 2.2e-7, max 1.0e-6
         return {"rel": 1e-6, "max": 4e-6}
     return {"rel": 8.3e-4, "max": 2.1e-3} if out == "f16" else {"rel": 6.6e-3, "max": 1.6e-2}
+
+
+def _rows(x):
+    """64-bit slices of a matrix, few enough rows at a time for the temporaries to stay small."""
+    step = max(1, (1 << 25) // x.shape[1])
+    return [(slice(i, i + step), x[i:i + step].double()) for i in range(0, x.shape[0], step)]
+
+
+def _exact_layernorm(s):
+    x, w, b, dy = (s[k].detach() for k in ("x", "w", "b", "dy"))
+    wd, bd = w.double(), b.double()
+    y, dx = torch.empty_like(x, dtype=torch.float64), torch.empty_like(x, dtype=torch.float64)
+    dw, db = torch.zeros_like(wd), torch.zeros_like(bd)
+    for rows, xd in _rows(x):
+        d = dy[rows].double()
+        mean = xd.mean(1, keepdim=True)
+        rstd = (xd.var(1, unbiased=False, keepdim=True) + 1e-5).rsqrt()
+        xhat, g = (xd - mean) * rstd, d * wd
+        y[rows] = xhat * wd + bd
+        dx[rows] = (g - g.mean(1, keepdim=True) - xhat * (g * xhat).mean(1, keepdim=True)) * rstd
+        dw += (d * xhat).sum(0)
+        db += d.sum(0)
+    return y, dx, dw, db
+
+
+def _exact_product(a, b):
+    return a.to(torch.float64) @ b.to(torch.float64)
+
+
+def _exact_stencil(case, x, c):
+    n, r = case["n"], case["radius"]
+    x, c = x.double(), c.double().tolist()
+    if case["bricks"]:       # 8 x 8 x 8 points after one another, the bricks row-major
+        x = x.view(n // 8, n // 8, n // 8, 8, 8, 8).permute(0, 3, 1, 4, 2, 5).reshape(n, n, n)
+    out = torch.zeros_like(x)
+    core = out[r:n - r, r:n - r, r:n - r]
+
+    def at(di, dj, dk):
+        return x[r + di:n - r + di, r + dj:n - r + dj, r + dk:n - r + dk]
+
+    if case["kind"] == "f3d":     # the centre counts once on its own and once more in the window
+        core.add_(at(0, 0, 0), alpha=c[r][r][r])
+        span = range(-r, r + 1)
+        for di in span:
+            for dj in span:
+                for dk in span:
+                    core.add_(at(di, dj, dk), alpha=c[di + r][dj + r][dk + r])
+    else:
+        core.add_(at(0, 0, 0), alpha=c[0])
+        for d in range(1, r + 1):
+            for step in ((d, 0, 0), (-d, 0, 0), (0, d, 0), (0, -d, 0), (0, 0, d), (0, 0, -d)):
+                core.add_(at(*step), alpha=c[d])
+    if case["bricks"]:
+        out = out.view(n // 8, 8, n // 8, 8, n // 8, 8).permute(0, 2, 4, 1, 3, 5).reshape(n, n, n)
+    return out
+
+
+def _exact_lu(m):
+    """L and U in one matrix, no pivoting: panels of 64 columns, the rest by matrix products."""
+    m, n = m.double(), m.shape[0]
+    for k in range(0, n, 64):
+        e = min(k + 64, n)
+        panel = m[k:, k:e]
+        for j in range(e - k - 1 if e == n else e - k):
+            panel[j + 1:, j] /= panel[j, j]
+            panel[j + 1:, j + 1:].addr_(panel[j + 1:, j], panel[j, j + 1:], alpha=-1)
+        if e < n:
+            lower = m[k:e, k:e].tril(-1) + torch.eye(e - k, device=m.device, dtype=m.dtype)
+            m[k:e, e:] = torch.linalg.solve_triangular(lower, m[k:e, e:], upper=False, unitriangular=True)
+            m[e:, e:] -= m[e:, k:e] @ m[k:e, e:]
+    return m
+
+
+def exact(case, seed):
+    """What ``run`` returns for these inputs, from plain torch operations in 64 bits (None: bits moved or whole numbers)."""
+    op = case["op"]
+    if op in ("transpose", "nw"):
+        return None
+    s = prepare(case, seed)
+    if op == "softmax":
+        out = torch.empty_like(s["x"], dtype=torch.float64)
+        for rows, xd in _rows(s["x"]):
+            out[rows] = torch.softmax(xd, 1)
+        return out
+    if op == "layernorm":
+        return _exact_layernorm(s)
+    if op == "gemm":
+        c = _exact_product(s["a"], s["b"])
+        return torch.where(c >= 0, c, 0.01 * c) if case["activation"] else c
+    if op == "grouped":
+        return [_exact_product(a, b) for a, b in zip(s["a"], s["b"])]
+    if op == "stencil":
+        return _exact_stencil(case, s["x"], s["c"])
+    return _exact_lu(s["m"])
