@@ -206,6 +206,14 @@ int lego_hip_nw_i32(const int* reference, int* matrix, int n, int penalty, void*
  * pointers; sizes3 is a HOST array of groups*3 ints (M, N, K per problem).  Any number of
  * groups: one launch carries up to 64 problems (their pointers and sizes travel as kernel arguments), a
  * call with more is enqueued as runs of 64 in order of decreasing K, one launch after the other on
+/* The same with device memory for the columns that its workgroups hand to one another, *bytes of it (0 up to n = 256),
+ * 16-byte aligned, its contents undefined before and after: the matrix is then filled by one launch (and a small one that
+ * clears the workspace) where lego_hip_nw_i32 enqueues n/32 - 1 dependent ones.  Without a workspace, or with too small
+ * a one, it is lego_hip_nw_i32. */
+int lego_hip_nw_i32_workspace_bytes(int n, unsigned long long* bytes);
+int lego_hip_nw_i32_ws(const int* reference, int* matrix, int n, int penalty, void* workspace,
+                       unsigned long long workspace_bytes, void* stream);
+
  * `stream`.  One launch per run when every N and K is a multiple of 8 and every base 16-byte aligned (any M;
  * ragged tiles and last k-tiles are masked); otherwise one launch per problem, as lego_hip_gemm_f16
  * would take it.  Replaces

@@ -292,6 +292,8 @@ def collect():
           f"#define LEGO_GEMM_BK_8BIT {GEMM_BK['e5m2']}",
           f"#define LEGO_GROUPED_MAX_GROUPS {mg['MAX_GROUPS']}", ""]
     h += ["hipError_t lego_nw_i32_launch(const int*, int*, int, int, hipStream_t);",
+          "unsigned long long lego_nw_i32_strips_words(int);",
+          "hipError_t lego_nw_i32_strips_launch(const int*, int*, int, int, unsigned long long*, hipStream_t);",
           f"#define LEGO_NW_TILE {mnw['B']}", "",
           "hipError_t lego_stencil_f32_launch(const float*, float*, const float*, int, int, int, int, hipStream_t);",
           f"#define LEGO_STENCIL_BRICK {mst['B']}", f"#define LEGO_STENCIL_MAX_RADIUS {mst['MAX_RADIUS']}",

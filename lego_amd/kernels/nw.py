@@ -29,6 +29,9 @@ from ..lego import GenP, OrderBy, Row, antidiag
 from .common import BANNER, Emitted, code, idx, size, template, tidy
 
 B = 64
+# the single launch: strips of STRIP columns, STRIPS of them per workgroup, in phases of P steps; an LDS ring of RING blocks of
+# P slots per strip, scores requested AHEAD blocks before they are needed, the column to the left WEST_AHEAD blocks before
+STRIP, STRIPS, P, RING, AHEAD, WEST_AHEAD, LAG = 128, 2, 16, 9, 4, 2, 6
 
 
 def tile_layout(b=B):
@@ -39,6 +42,11 @@ def tile_layout(b=B):
 def rotation_layout(b=B):
     """The LDS tile of the kernel: row-major, a lane's column in one bank."""
     return OrderBy(Row(b, b)).TileBy([b, b])
+
+
+def slot_layout(slots=RING * P, strip=STRIP):
+    """A strip's LDS in the single launch: a slot holds one cell pair per lane, a lane's pairs in the same two banks."""
+    return OrderBy(Row(slots, strip)).TileBy([slots, strip])
 
 
 def emit():
@@ -55,11 +63,14 @@ def emit():
         raise ValueError(f"cell offset {cell} does not split into a row part and a lane part")
     i, j = sp.symbols("i j", integer=True, nonnegative=True)
     lds = sp.simplify(rotation_layout()[i, j])
+    slot, lane = idx("slot"), idx("lane")
+    slot_expr = tidy(slot_layout()[slot, 2 * lane], {slot: (0, RING * P), lane: (0, STRIP // 2)})
     params = dict(
-        banner=BANNER, B=B,
+        banner=BANNER, B=B, STRIP=STRIP, STRIPS=STRIPS, P=P, RING=RING, AHEAD=AHEAD, WEST_AHEAD=WEST_AHEAD, LAG=LAG,
+        slot=code(slot_expr), slot_layout=f"OrderBy(Row({RING * P}, {STRIP})).TileBy([{RING * P}, {STRIP}])[slot, 2*lane]",
         tile_layout=f"OrderBy(Row({B}, {B})).TileBy([{B}, {B}])[i, j]",
         matrix_layout=f"OrderBy(Row(cols, cols)).TileBy([cols, cols])[{B}*by + 1 + ty, {B}*bx + 1 + tx]",
         cell_row=code(cell_row), cell_lane=code(cell_lane), lds=code(lds),
     )
     text = template("nw.hip.j2").render(**params)
-    return Emitted("nw_i32.hip", text, ["lego_nw_i32_launch"]), dict(B=B)
+    return Emitted("nw_i32.hip", text, ["lego_nw_i32_launch", "lego_nw_i32_strips_launch", "lego_nw_i32_strips_words"]), dict(B=B)

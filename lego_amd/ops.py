@@ -280,7 +280,12 @@ def needleman_wunsch(reference: torch.Tensor, matrix: torch.Tensor, penalty: int
     _check(matrix, torch.int32, "matrix")
     if reference.shape != matrix.shape or matrix.shape[0] != matrix.shape[1]:
         raise ValueError("reference and matrix must be square and of the same shape")
-    runtime.call("lego_hip_nw_i32", _ptr(reference), _ptr(matrix), matrix.shape[0] - 1, int(penalty), _stream())
+    n = matrix.shape[0] - 1
+    size = ctypes.c_ulonglong(0)
+    runtime.call("lego_hip_nw_i32_workspace_bytes", n, ctypes.byref(size))
+    workspace = torch.empty(size.value // 8, dtype=torch.int64, device=matrix.device) if size.value else None
+    runtime.call("lego_hip_nw_i32_ws", _ptr(reference), _ptr(matrix), n, int(penalty),
+                 None if workspace is None else _ptr(workspace), size.value, _stream())
     return matrix
 
 

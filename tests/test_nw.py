@@ -81,6 +81,30 @@ def test_gpu_matches_oracle(n, penalty):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 128, 192, 256, 320, 384, 448, 576, 1088, 4160])
+def test_gpu_single_launch_agrees_with_a_launch_per_anti_diagonal(n):
+    """Strips of 128 columns, two per workgroup, the last one half empty or missing; any borders and scores, down to half
+    the type's lowest value.  Up to n = 256 (one workgroup, which both entry points take) the oracle's borders are used."""
+    from lego_amd import ops, runtime
+    print(f"needleman-wunsch n={n}, one launch", flush=True)
+    g = torch.Generator().manual_seed(n)
+    ref = torch.randint(-40, 60, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    ref[torch.rand(n + 1, n + 1, generator=g) < 0.01] = -(1 << 30)
+    m = torch.randint(-1000, 1000, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    m[5, 0] = m[0, 7] = -(1 << 30)
+    if n <= 256:
+        m[:, 0] = m[0, :] = -3 * torch.arange(n + 1, dtype=torch.int32)
+        want = torch.from_numpy(ok.needleman_wunsch(ref.numpy(), 3))
+    else:
+        mat, r = m.cuda(), ref.cuda()
+        runtime.call("lego_hip_nw_i32", r.data_ptr(), mat.data_ptr(), n, 3, None)
+        want = mat.cpu()
+    for _ in range(2):      # the second call finds the first one's workspace in the allocator
+        got = ops.needleman_wunsch(ref.cuda(), m.cuda(), 3).cpu()
+        assert torch.equal(got, want)
+
+
+@pytest.mark.gpu
 def test_gpu_rejects_bad_sizes():
     from lego_amd import ops
     from lego_amd.runtime import LegoHipError
