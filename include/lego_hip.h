@@ -167,6 +167,10 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_stencil_f3d_f32(const float* in, float* out, const float* c, int n, int radius, int bricks, void* stream);
 int lego_hip_stencil_laplacian_f32(const float* in, float* out, const float* c, int n, int radius, int bricks,
                                    void* stream);
+/* The same with zeros written to the points closer than radius to the boundary: every element of out is written. */
+int lego_hip_stencil_f3d_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks, void* stream);
+int lego_hip_stencil_laplacian_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks,
+                                         void* stream);
 
 /* LU decomposition without pivoting of an n x n fp32 row-major matrix, in place: on return the
  * strict lower triangle holds L (unit diagonal implied) and the upper triangle holds U, as
@@ -202,10 +206,6 @@ int lego_hip_lud_f32_plan(int n, int* records, int capacity, int* count);
  * matrix[i-1][j] - penalty) for i, j >= 1.  n a multiple of 64, at most 32768. */
 int lego_hip_nw_i32(const int* reference, int* matrix, int n, int penalty, void* stream);
 
-/* groups independent GEMMs in one launch.  a, b, c are HOST arrays of `groups` device
- * pointers; sizes3 is a HOST array of groups*3 ints (M, N, K per problem).  Any number of
- * groups: one launch carries up to 64 problems (their pointers and sizes travel as kernel arguments), a
- * call with more is enqueued as runs of 64 in order of decreasing K, one launch after the other on
 /* The same with device memory for the columns that its workgroups hand to one another, *bytes of it (0 up to n = 256),
  * 16-byte aligned, its contents undefined before and after: the matrix is then filled by one launch (and a small one that
  * clears the workspace) where lego_hip_nw_i32 enqueues n/32 - 1 dependent ones.  Without a workspace, or with too small
@@ -214,6 +214,10 @@ int lego_hip_nw_i32_workspace_bytes(int n, unsigned long long* bytes);
 int lego_hip_nw_i32_ws(const int* reference, int* matrix, int n, int penalty, void* workspace,
                        unsigned long long workspace_bytes, void* stream);
 
+/* groups independent GEMMs in one launch.  a, b, c are HOST arrays of `groups` device
+ * pointers; sizes3 is a HOST array of groups*3 ints (M, N, K per problem).  Any number of
+ * groups: one launch carries up to 64 problems (their pointers and sizes travel as kernel arguments), a
+ * call with more is enqueued as runs of 64 in order of decreasing K, one launch after the other on
  * `stream`.  One launch per run when every N and K is a multiple of 8 and every base 16-byte aligned (any M;
  * ragged tiles and last k-tiles are masked); otherwise one launch per problem, as lego_hip_gemm_f16
  * would take it.  Replaces

@@ -868,24 +868,35 @@ int lego_hip_gemm_f16(const void* a, const void* b, void* c, int M, int N, int K
 }
 
 namespace {
-int stencil(const float* in, float* out, const float* c, int n, int radius, int kind, int bricks, void* stream)
+int stencil(const float* in, float* out, const float* c, int n, int radius, int kind, int bricks, int keep, void* stream)
 {
   if (!usable(in) || !usable(out) || c == nullptr || in == out) return kInvalid;
   if (n <= 0 || n % LEGO_STENCIL_BRICK || n > 1024 || radius < 1 || radius > (kind == 1 ? LEGO_STENCIL_STAR_MAX_RADIUS : LEGO_STENCIL_MAX_RADIUS) || 2 * radius >= n)
     return kInvalid;
-  return ok_or(lego_stencil_f32_launch(in, out, c, n, radius, kind, bricks ? 1 : 0, as_stream(stream)));
+  return ok_or(lego_stencil_f32_launch(in, out, c, n, radius, kind, bricks ? 1 : 0, keep, as_stream(stream)));
 }
 }  // namespace
 
 int lego_hip_stencil_f3d_f32(const float* in, float* out, const float* c, int n, int radius, int bricks, void* stream)
 {
-  return stencil(in, out, c, n, radius, 0, bricks, stream);
+  return stencil(in, out, c, n, radius, 0, bricks, 1, stream);
 }
 
 int lego_hip_stencil_laplacian_f32(const float* in, float* out, const float* c, int n, int radius, int bricks,
                                    void* stream)
 {
-  return stencil(in, out, c, n, radius, 1, bricks, stream);
+  return stencil(in, out, c, n, radius, 1, bricks, 1, stream);
+}
+
+int lego_hip_stencil_f3d_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks, void* stream)
+{
+  return stencil(in, out, c, n, radius, 0, bricks, 0, stream);
+}
+
+int lego_hip_stencil_laplacian_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks,
+                                         void* stream)
+{
+  return stencil(in, out, c, n, radius, 1, bricks, 0, stream);
 }
 
 int lego_hip_lud_f32(float* m, int n, void* stream)
@@ -906,24 +917,13 @@ int lego_hip_nw_i32(const int* reference, int* matrix, int n, int penalty, void*
 {
   if (!usable(reference) || !usable(matrix)) return kInvalid;
   if (n <= 0 || n % LEGO_NW_TILE || n > 32768) return kInvalid;
-  return ok_or(lego_nw_i32_launch(reference, matrix, n, penalty, as_stream(stream)));
-}
-
-namespace {
-// Time of a grouped launch: list scheduling of its workgroups, in launch order, on `slots` workgroups
-// that run at once (a workgroup goes to the slot that frees up first).  The launch is a sequence of
-// batches of count[i] workgroups that take cost[i] each.  The slot loads are kept as a sorted list of
-// (load, how many slots) levels, so a batch of equal workgroups costs a few steps.
-double grouped_makespan(const long* count, const double* cost, int batches, long slots)
-{
-  struct Level { double load; long count; };
   // one workgroup needs no room for handing columns over; a single tile (n = 64) is one launch of the tile kernel, which
   // has no ring to fill and drain: 5.8 us against 8.8
   if (n > LEGO_NW_TILE && lego_nw_i32_strips_words(n) == 0)
     return ok_or(lego_nw_i32_strips_launch(reference, matrix, n, penalty, nullptr, as_stream(stream)));
-  Level lv[8 * LEGO_GROUPED_MAX_GROUPS + 8];
-  int n = 1;
-  lv[0] = {0.0, slots};
+  return ok_or(lego_nw_i32_launch(reference, matrix, n, penalty, as_stream(stream)));
+}
+
 int lego_hip_nw_i32_workspace_bytes(int n, unsigned long long* bytes)
 {
   if (bytes == nullptr || n <= 0 || n % LEGO_NW_TILE || n > 32768) return kInvalid;
@@ -940,6 +940,17 @@ int lego_hip_nw_i32_ws(const int* reference, int* matrix, int n, int penalty, vo
   return ok_or(lego_nw_i32_strips_launch(reference, matrix, n, penalty, static_cast<unsigned long long*>(workspace), as_stream(stream)));
 }
 
+namespace {
+// Time of a grouped launch: list scheduling of its workgroups, in launch order, on `slots` workgroups
+// that run at once (a workgroup goes to the slot that frees up first).  The launch is a sequence of
+// batches of count[i] workgroups that take cost[i] each.  The slot loads are kept as a sorted list of
+// (load, how many slots) levels, so a batch of equal workgroups costs a few steps.
+double grouped_makespan(const long* count, const double* cost, int batches, long slots)
+{
+  struct Level { double load; long count; };
+  Level lv[8 * LEGO_GROUPED_MAX_GROUPS + 8];
+  int n = 1;
+  lv[0] = {0.0, slots};
   for (int g = 0; g < batches; ++g) {
     long left = count[g];
     const double d = cost[g];

@@ -26,6 +26,7 @@ to one row of every lane is the whole 2 KiB brick (bricks storage) or 64 runs of
 from __future__ import annotations
 
 from ..lego import OrderBy, Row
+from .lud import XCDS, xcd_remap
 from .common import BANNER, Emitted, code, idx, size, template, tidy
 
 B = 8
@@ -33,6 +34,7 @@ MAX_RADIUS = 3        # the coefficient cube is 8 x 8 x 8: offsets -3..3 plus on
 STAR_MAX_RADIUS = 4   # the star stencil has radius + 1 coefficients; the reference runs it up to 4 (result/cuda/bricks-laplace.txt)
 WAVES = 4             # bricks per workgroup, dense stencil (its shell fills the 64 KiB of LDS at radius 3)
 STAR_WAVES = 8        # and star stencil: the more bricks in a row, the fewer row ends come from memory
+LANES_Y, LANES_Z = 4, 16   # the marching kernels: a wavefront is four DPP rows of sixteen lanes
 # words per row of the shell in LDS: 16 hold a row (3 + 8 + 3 points, 16-byte aligned), 20 spread the
 # 16-byte reads of eight neighbouring lanes over different banks
 ROW_WORDS = 20
@@ -82,7 +84,15 @@ def emit():
     SPLANE = size("PLANE")
     star = OrderBy(Row(H, SPLANE)).TileBy([H, SPLANE])
     star_row = code(tidy(star[hx, B * hy], {hx: (0, H), hy: (0, H)}))
+    # the marching kernels: columns of the field, one per wavefront, numbered chunk by chunk along the first axis
+    pid, lane, zt, yt, per, chunks = idx("id"), idx("lane"), size("zt"), size("yt"), size("per"), size("chunks")
+    order = OrderBy(Row(chunks, yt, zt)).TileBy([chunks, yt, zt]).inv(pid)
+    lanes = OrderBy(Row(LANES_Y, LANES_Z)).TileBy([LANES_Y, LANES_Z]).inv(lane)
     params = dict(
+        LANES_Y=LANES_Y, LANES_Z=LANES_Z, XCDS=XCDS, xcd_pid=code(tidy(xcd_remap(per, wg), {wg: (0, per * XCDS)})),
+        march_order=[code(tidy(e, {pid: (0, chunks * yt * zt)})) for e in order],
+        march_lane=[code(tidy(e, {lane: (0, LANES_Y * LANES_Z)})) for e in lanes],
+        march_layout=f"OrderBy(Row({LANES_Y}, {LANES_Z})).TileBy([{LANES_Y}, {LANES_Z}])",
         star_layout=f"OrderBy(Row(H, PLANE)).TileBy([H, PLANE])[hx, {B}*hy + word]", star_row=star_row,
         shell_layout=f"OrderBy(Row(H, PLANE)).TileBy([H, PLANE])[hx, {ROW_WORDS}*hy + word]",
         shell_inv=shell_inv, shell_row=shell_row, ROW_WORDS=ROW_WORDS,

@@ -198,6 +198,39 @@ def test_gpu_stencils_full_size_agree_between_layouts():
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("kind,radius,n", [("f3d", 1, 128), ("f3d", 1, 136), ("f3d", 2, 200), ("f3d", 3, 264), ("laplacian", 1, 128),
+                                           ("laplacian", 2, 152), ("laplacian", 3, 200), ("laplacian", 4, 136), ("laplacian", 4, 192)])
+def test_gpu_stencil_columns_and_bricks_agree(kind, radius, n):
+    """From these sizes on row-major fields are walked column by column, in sizes that leave lanes, rows and planes over;
+    the bricks storage (radius 4: its columns too) gives the same bits, an `out` of the caller's keeps its boundary and the
+    default one has zeros there.  The field around the smallest such column agrees with the oracle."""
+    from lego_amd import ops
+    print(f"{kind} n={n} radius={radius}", flush=True)
+    x = torch.rand(n, n, n, generator=torch.Generator().manual_seed(n)) * 2 - 1
+    c = torch.from_numpy(_coefficients(radius)) if kind == "f3d" else torch.tensor([-6.0, 1.0, 0.5, 0.25, 0.125])[:radius + 1].contiguous()
+    call, oracle = (ops.stencil_f3d, ok.stencil_f3d) if kind == "f3d" else (ops.stencil_laplacian, ok.stencil_laplacian)
+    order = ok.bricks_order(n)
+    a = call(x.cuda(), c.cuda(), radius, False).cpu()
+    b = _from_bricks(call(_to_bricks(x, order).cuda(), c.cuda(), radius, True).cpu(), order)
+    assert torch.equal(a, b)
+    inner = (slice(radius, n - radius),) * 3
+    want = torch.full((n, n, n), 7.0)
+    want[inner] = a[inner]
+    for bricks in (False, True):
+        out = torch.full((n, n, n), 7.0, device="cuda")
+        got = call(_to_bricks(x, order).cuda() if bricks else x.cuda(), c.cuda(), radius, bricks, out=out).cpu()
+        assert torch.equal(_from_bricks(got, order) if bricks else got, want)
+    a[inner] = 0
+    assert a.abs().max().item() == 0
+    for lo in (0, n - 24):      # the oracle of a corner, away from the cuts
+        s = slice(lo, lo + 24)
+        ref = torch.from_numpy(oracle(x[s, s, s].contiguous().numpy(), c.numpy(), radius)).float()
+        k = slice(radius, 24 - radius)
+        full = slice(lo + radius, lo + 24 - radius)
+        assert (want[full, full, full] - ref[k, k, k]).abs().max().item() <= 2e-5 * (2 * radius + 1) ** 3
+
+
+@pytest.mark.gpu
 def test_gpu_stencil_rejects_bad_arguments():
     from lego_amd import ops
     from lego_amd.runtime import LegoHipError
