@@ -22,6 +22,7 @@ from ..lego import Col, OrderBy, Row, le_constraint
 from .common import BANNER, Emitted, code, idx, size, template, tidy
 
 B, T, R = 64, 16, 4
+STEPS = 4      # elimination steps of a diagonal block between two exchanges among its wavefronts
 # side (in blocks) of the trailing square from which the next panels are solved on a second stream meanwhile
 AHEAD_MIN = 72
 # the trailing square is walked in groups of GROUP block rows, column by column inside a group (the grouped launch
@@ -71,7 +72,7 @@ def emit():
     j = idx("j")
     k_of_lane = tidy(OrderBy(Row(2, B // 2)).TileBy([2, B // 2])[l // 32, j], {l: (0, 64), j: (0, B // 2)})
     params = dict(
-        banner=BANNER, B=B, T=T, R=R, AHEAD_MIN=AHEAD_MIN,
+        banner=BANNER, B=B, T=T, R=R, STEPS=STEPS, AHEAD_MIN=AHEAD_MIN,
         matrix_layout=f"OrderBy(Row(n, n)).TileBy([n/{B}, n/{B}], [{B}, {B}])[bi, bj, r, c]",
         thread_layout=f"OrderBy(Row({R * T}, {R * T})).GroupBy([({R}, {R}), ({T}, {T})]).inv((ii*{R} + jj)*{T * T} + tid)",
         elem=code(elem), ci=code(i_e), cj=code(j_e), cty=code(ty_e), ctx=code(tx_e),

@@ -246,3 +246,31 @@ def test_gpu_call_with_second_stream_replays_from_a_hip_graph():
             torch.cuda.synchronize()
             del other
         del graph
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [64, 128, 192])
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30, 2.0 ** -130])
+def test_gpu_pivots_of_any_magnitude(n, scale):
+    """Pivots near the ends of the exponent range take true divisions (2^-130: denormal ones); the rounding of the
+    elements themselves, n of them summed, bounds L - L' and (U - U') / scale."""
+    from lego_amd import ops
+    print(f"lud n={n} scale={scale}", flush=True)
+    a = (_dominant(n, n + 1) * scale).astype(np.float32)
+    got = ops.lud(torch.from_numpy(a).cuda()).cpu().numpy().astype(np.float64)
+    want = ok.lud(a.astype(np.float64))
+    spacing = max(2.0 ** -24, 2.0 ** -149 / (scale * n))      # of the pivots, which are about n * scale
+    assert np.abs(np.tril(got - want, -1)).max() <= 4 * n * spacing
+    assert np.abs(np.triu(got - want)).max() / scale <= 4 * n * n * spacing
+
+
+@pytest.mark.gpu
+def test_gpu_non_finite_elements_stay_where_elimination_takes_them():
+    """A NaN reaches the blocks that depend on it and no other: the first block row and column of a matrix whose last block
+    has one are the factors of the matrix without it."""
+    from lego_amd import ops
+    a = torch.from_numpy(_dominant(192, 3).astype(np.float32))
+    want = ops.lud(a.clone().cuda()).cpu()
+    a[150, 160] = float("nan")
+    got = ops.lud(a.cuda()).cpu()
+    assert torch.equal(got[:128, :128], want[:128, :128]) and got[150, 160].isnan()
