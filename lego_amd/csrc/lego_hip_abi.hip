@@ -718,11 +718,15 @@ int splitk_parts(int M, int N, int K, int bk)
 }
 typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int, int, int, int, float*, hipStream_t);
 
-// 8-bit operands: the small tile only where both operands are k-major (A as given, B transposed)
-#define LEGO_GEMM_KERNELS_SMALL_NT(DT)                                                                 \
+// 8-bit operands: both tile sizes in all four layouts, one MFMA shape.  The rule between the tiles is that of the 16-bit
+// operands; us on big / small tiles, e5m2 A*B: 512 x 512 x 2048 19.5 / 8.6, 1000 x 2048 x 2048 22.1 / 13.6 (32 and 128
+// workgroups), 2048^3 22.0 / 14.1, 2048 x 4096 x 4096 39.4 / 31.0, 4352 x 4096 x 4096 78.4 / 73.7, 4608^3 88.3 / 84.6.
+#define LEGO_GEMM_KERNELS_8BIT(DT)                                                                     \
   {{lego_gemm_##DT##_nn_launch, lego_gemm_##DT##_nt_launch, lego_gemm_##DT##_tn_launch,              \
     lego_gemm_##DT##_tt_launch},                                                                       \
-   {nullptr, lego_gemm_##DT##_nt_t128x128_launch, nullptr, nullptr}}
+   {lego_gemm_##DT##_nn_t128x128_launch, lego_gemm_##DT##_nt_t128x128_launch,                         \
+    lego_gemm_##DT##_tn_t128x128_launch, lego_gemm_##DT##_tt_t128x128_launch},                         \
+   {nullptr, nullptr, nullptr, nullptr}}
 #define LEGO_GEMM_KERNELS(DT)                                                                          \
   {{lego_gemm_##DT##_nn_launch, lego_gemm_##DT##_nt_launch, lego_gemm_##DT##_tn_launch,              \
     lego_gemm_##DT##_tt_launch},                                                                       \
@@ -840,8 +844,8 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
 int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                          int activation, int format, void* stream)
 {
-  static const GemmKernels e4m3 = LEGO_GEMM_KERNELS_SMALL_NT(e4m3);
-  static const GemmKernels e5m2 = LEGO_GEMM_KERNELS_SMALL_NT(e5m2);
+  static const GemmKernels e4m3 = LEGO_GEMM_KERNELS_8BIT(e4m3);
+  static const GemmKernels e5m2 = LEGO_GEMM_KERNELS_8BIT(e5m2);
   if (format != 0 && format != 1) return kInvalid;
   return gemm_ex(format == 0 ? e4m3 : e5m2, format == 0 ? 2 : 3, a, b, c, M, N, K, trans_a, trans_b, activation,
                  stream, LEGO_GEMM_BK_8BIT, 16);

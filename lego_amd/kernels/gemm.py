@@ -54,14 +54,19 @@ def lds_b_layout(bk, bn, period=4, groups_by_k=False):
     A transposing read of 2-byte elements touches four consecutive k-rows, 64 bytes of each;
     rotating the 64-byte chunk index by ``k % 4`` puts the four rows on four different quarters
     of the banks.  One of 1-byte elements touches eight k-rows, 32 bytes of each (32 elements
-    again): ``period = 8``.  Bits 0-4 of ``n`` are untouched, so 16-byte stores and 8-byte reads
-    stay whole.  ``groups_by_k`` (16 x 16 MFMA blocks, 2-byte elements): the two 16-lane groups that an 8-byte read
+    again): ``period = 8``; where a row has four such chunks only (``bn = 128``), two rows fill the banks once and the
+    key goes up with every other row, ``32*((k // 2) % 4)``: eight rows, eight different chunks again.  Bits 0-4 of
+    ``n`` are untouched, so 16-byte stores and 8-byte reads stay whole.  ``groups_by_k`` (16 x 16 MFMA blocks, 2-byte elements): the two 16-lane groups that an 8-byte read
     serves together read the same 16 columns of k-rows eight apart, 32 of the 64 bytes of each quarter; the key
     also flips bit 4 of ``n`` (32 bytes) with bit 3 of ``k``, which sends the second group to the other 32 bytes
     (bits 0-3 stay, so 16-byte stores and 8-byte reads are still whole)."""
-    assert not groups_by_k or period == 4
+    assert not groups_by_k or (period == 4 and bn >= 128)
+
+    rows_per_key = max(1, 32 * period // bn)      # rows of under `period` chunks share a key
 
     def key(k):
+        if rows_per_key > 1:
+            return (k // rows_per_key % (period // rows_per_key)) * 32
         return (k % period) * 32 + (((k // 8) % 2) * 16 if groups_by_k else 0)
 
     def forward(kn):

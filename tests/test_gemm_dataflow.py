@@ -49,7 +49,7 @@ def _args(call):
 
 
 @pytest.mark.parametrize("dtype,bk,tile,block", [("f16", 64, 256, 32), ("f16", 64, 256, 16), ("e5m2", 128, 256, 32),
-                                                 ("f16", 64, 128, 32)])
+                                                 ("f16", 64, 128, 32), ("e5m2", 128, 128, 32)])
 @pytest.mark.parametrize("variant", ["nn", "tt"])
 def test_fragments_receive_the_right_elements(dtype, bk, tile, block, variant):
     ta, tb = variant[0] == "t", variant[1] == "t"

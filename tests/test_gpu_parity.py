@@ -1308,6 +1308,25 @@ def test_gemm_fp8_integer_exact(ops):
                 assert torch.equal(ops.matmul(ad, bd).cpu().double(), want)
 
 
+@pytest.mark.parametrize("M,N,K", [(16, 16, 16), (128, 128, 128), (144, 272, 400), (1008, 1040, 2064)])
+@pytest.mark.parametrize("fp8", [torch.float8_e5m2, torch.float8_e4m3fn])
+def test_gemm_fp8_small_tiles_ragged(ops, fp8, M, N, K):
+    """Products of few tiles go to the 128 x 128 tiles in all four layouts: a part of a tile, one tile, remainders in
+    every direction.  Operands in {-1..1}: sums are whole numbers of magnitude below 2048 at 2064 products (variance 4/9
+    each: 48 standard deviations), exact in fp32 and fp16."""
+    g = _gen(15)
+    a = torch.randint(-1, 2, (M, K), generator=g).float()
+    b = torch.randint(-1, 2, (K, N), generator=g).float()
+    want = a.double() @ b.double()
+    a8, b8 = a.to(fp8), b.to(fp8)
+    for ta in (False, True):
+        for tb in (False, True):
+            print(f"gemm {fp8} small tiles ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
+            ad = a8.t().contiguous().cuda().t() if ta else a8.cuda()
+            bd = b8.t().contiguous().cuda().t() if tb else b8.cuda()
+            assert torch.equal(ops.matmul(ad, bd).cpu().double(), want)
+
+
 def test_gemm_leaky_relu_epilogue(ops):
     print("gemm leaky_relu", flush=True)
     g = _gen(8)

@@ -122,9 +122,10 @@ def test_gemm_lds_layout_for_16_column_blocks_is_bijective_and_conflict_free():
                 assert conflicts([tp[k, n] // 2 for k, n in rows_cols], 2) == 2
 
 
-def test_gemm_lds_layouts_8bit_are_bijective_and_conflict_free():
+@pytest.mark.parametrize("tile", [256, 128])
+def test_gemm_lds_layouts_8bit_are_bijective_and_conflict_free(tile):
     """One-byte operands: 128 k-values per tile, 32 per lane and MFMA."""
-    bm, bn, bk = 256, 256, 128
+    bm, bn, bk = tile, tile, 128
     a = gemm.lds_a_layout(bm, bk // 16)
     b = gemm.lds_b_layout(bk, bn, 8)
     ta = np.array([[int(a.apply(r, c)) for c in range(bk // 16)] for r in range(bm)])
