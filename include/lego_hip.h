@@ -153,6 +153,13 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
  * element; shapes as for fp16, a 16-byte chunk being 16 elements and a k-tile 128. */
 int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                          int activation, int format, void* stream);
+/* The same product with room for partial sums: a product of few tiles is split along K as lego_hip_gemm_ex_ws does it.
+ * lego_hip_gemm_fp8_workspace_bytes gives the size the call uses for a shape (0: it stays whole); the workspace as
+ * there.  With a null or short workspace, or a layout whose rows are not whole 16-byte chunks, the call is
+ * lego_hip_gemm_fp8_ex. */
+int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes);
+int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
+                            int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream);
 
 /* 3-D stencils on an n x n x n fp32 array (the reference's bricks benchmarks:
  * benchmarks/cuda/bricks_f3d.py:8-22 with bricks/main_tmp.cu:24-104, and bricks_laplasian.py:8-33

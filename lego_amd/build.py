@@ -94,7 +94,6 @@ ROWWISE_MAX_N = rowwise.MAX_N
 GEMM = dict(bm=256, bn=256, bk=64, waves=(2, 2), max_group_m=8)
 GEMM_SMALL_TILE = 128
 GEMM_WAVES_TWO_PER_SIMD = (2, 4)
-GEMM_SPLITK_DTYPES = ("f16", "bf16", "bf16h")     # element types whose 128 x 128 tiles are also built with a split along K
 GEMM_DTYPES = ("f16", "bf16", "bf16h", "e4m3", "e5m2")     # bf16h: bfloat16 operands, fp16 result
 GEMM_SPARSE_ROUND_DTYPES = ("f16", "bf16", "bf16h")   # 16-bit operands: also built on the 32x32x16 MFMA (see collect())
 # The MFMA of the 256 x 256 tiles: v_mfma_f32_16x16x32 for 16-bit operands (the same matrix-core cycles per flop as
@@ -158,7 +157,7 @@ def collect():
                 # 256x256 tiles to fill the chip
                 gs, _ = gemm.emit(**dict(GEMM, bk=GEMM_BK[dtype], bm=GEMM_SMALL_TILE, bn=GEMM_SMALL_TILE),
                                   trans_a=ta, trans_b=tb, dtype=dtype,
-                                  with_grouped=dtype == "f16" and not (ta or tb), with_splitk=dtype in GEMM_SPLITK_DTYPES)
+                                  with_grouped=dtype == "f16" and not (ta or tb), with_splitk=True)
                 units.append(gs)
     # The 256 x 256 tile on 32 x 32 accumulator blocks (v_mfma_f32_32x32x16), four waves of 128 x 128: behind at the
     # socket's power limit (8192^3: 1.29 against 1.36 PFLOP/s) and ahead away from it, so launches of one round that
@@ -264,7 +263,7 @@ def collect():
           for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")
           for t in ("", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}")]
     h += [f"hipError_t lego_gemm_{d}_{v}_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_splitk_launch(const void*, const void*, void*, int, int, int, int, "
-          "int, float*, hipStream_t);" for d in GEMM_SPLITK_DTYPES for v in ("nn", "nt", "tn", "tt")]
+          "int, float*, hipStream_t);" for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")]
     h += [
           "hipError_t lego_grouped_gemm_f16_launch(const void* const*, const void* const*, void* const*, "
           "const int*, int, hipStream_t);",

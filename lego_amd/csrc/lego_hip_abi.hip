@@ -717,6 +717,8 @@ int splitk_parts(int M, int N, int K, int bk)
   return parts < 2 ? 1 : static_cast<int>(parts);
 }
 typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int, int, int, int, float*, hipStream_t);
+#define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_splitk_launch, lego_gemm_##DT##_nt_t128x128_splitk_launch, \
+                         lego_gemm_##DT##_tn_t128x128_splitk_launch, lego_gemm_##DT##_tt_t128x128_splitk_launch}
 
 // 8-bit operands: both tile sizes in all four layouts, one MFMA shape.  The rule between the tiles is that of the 16-bit
 // operands; us on big / small tiles, e5m2 A*B: 512 x 512 x 2048 19.5 / 8.6, 1000 x 2048 x 2048 22.1 / 13.6 (32 and 128
@@ -777,10 +779,7 @@ int lego_hip_gemm_workspace_bytes(int M, int N, int K, unsigned long long* bytes
 int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                         int activation, void* workspace, unsigned long long workspace_bytes, void* stream)
 {
-#define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_splitk_launch, lego_gemm_##DT##_nt_t128x128_splitk_launch, \
-                         lego_gemm_##DT##_tn_t128x128_splitk_launch, lego_gemm_##DT##_tt_t128x128_splitk_launch}
   static const splitk_launcher f16[4] = LEGO_SPLITK(f16), bf16[4] = LEGO_SPLITK(bf16), bf16h[4] = LEGO_SPLITK(bf16h);
-#undef LEGO_SPLITK
   if (element != 0 && element != 1 && element != 4) return kInvalid;
   unsigned long long need = 0;
   if (lego_hip_gemm_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
@@ -849,6 +848,44 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
   if (format != 0 && format != 1) return kInvalid;
   return gemm_ex(format == 0 ? e4m3 : e5m2, format == 0 ? 2 : 3, a, b, c, M, N, K, trans_a, trans_b, activation,
                  stream, LEGO_GEMM_BK_8BIT, 16);
+}
+
+// Parts along K of an 8-bit product: the rule of the 16-bit operands with k-tiles of 128 elements (the same bytes and the
+// same matrix-core time each), but whole where the tiles outnumber two per k-tile: the sums of about 512 parts, 64 KiB
+// each, then cost more than the shorter chains give.  us whole (small tile, A*B^T) / in parts: 16 x 8192 x 8192 (64 tiles,
+// 64 k-tiles) 41.4 / 18.0, 64 x 4096 x 4096 (32, 32) 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8, 1024 x 1024 x 4096 (64, 32)
+// 21.7 / 18.8, 1152 x 1280 x 5888 (90, 46) 32.9 / 32.2, 256 x 8192 x 8192 (128, 64) 40.2 / 33.4; 1408 x 1408 x 4096 (121, 32) 23.3 / 30.2.
+static int splitk_parts_8bit(int M, int N, int K)
+{
+  const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128);
+  const long depth = (K + LEGO_GEMM_BK_8BIT - 1) / LEGO_GEMM_BK_8BIT;
+  return tiles > 2 * depth ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT);
+}
+
+// Room for the sums of a split product; none where gemm_ex would not take the tiled kernels in any layout.
+int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
+{
+  if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
+  const int parts = N % 16 ? 1 : splitk_parts_8bit(M, N, K);
+  const unsigned long long tiles = static_cast<unsigned long long>((M + 127) / 128) * ((N + 127) / 128);
+  *bytes = parts > 1 ? parts * tiles * 128ull * 128ull * sizeof(float) : 0ull;
+  return 0;
+}
+
+int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
+                            int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream)
+{
+  static const splitk_launcher e4m3[4] = LEGO_SPLITK(e4m3), e5m2[4] = LEGO_SPLITK(e5m2);
+  unsigned long long need = 0;
+  if ((format != 0 && format != 1) || lego_hip_gemm_fp8_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
+  const bool tiled = usable(a) && usable(b) && usable(c) && N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) &&
+                     (!trans_b || K % 16 == 0);
+  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need)
+    return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
+  if (activation != 0 && activation != 1) return kInvalid;
+  const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
+  return ok_or((format == 0 ? e4m3 : e5m2)[layout](a, b, c, M, N, K, activation, splitk_parts_8bit(M, N, K),
+                                                   static_cast<float*>(workspace), as_stream(stream)));
 }
 
 int lego_hip_gemm_f16_variant(const void* a, const void* b, void* c, int M, int N, int K, int variant, void* stream)

@@ -1,4 +1,5 @@
 """GPU parity tests: the HIP path, called through the C ABI, against the CPU oracle."""
+import ctypes
 import math
 
 import pytest
@@ -1325,6 +1326,33 @@ def test_gemm_fp8_small_tiles_ragged(ops, fp8, M, N, K):
             ad = a8.t().contiguous().cuda().t() if ta else a8.cuda()
             bd = b8.t().contiguous().cuda().t() if tb else b8.cuda()
             assert torch.equal(ops.matmul(ad, bd).cpu().double(), want)
+
+
+@pytest.mark.parametrize("M,N,K", [(16, 8192, 8192), (1, 64, 4096), (144, 272, 4112), (256, 256, 16384), (112, 144, 8016)])
+@pytest.mark.parametrize("fp8", [torch.float8_e5m2, torch.float8_e4m3fn])
+def test_gemm_fp8_split_along_k(ops, fp8, M, N, K):
+    """Few tiles and a long K go in parts: whole tiles, a single row, ragged sides and a ragged last k-tile, a last part
+    that is shorter than the others.  Operands in {-1, 0, 1}, an eighth of A's non-zero: sums are whole numbers of
+    magnitude below 2048 (variance 1/12 a product, 55 standard deviations at K = 16384), exact in fp32 and fp16."""
+    from lego_amd import runtime
+    need = ctypes.c_ulonglong(0)
+    runtime.call("lego_hip_gemm_fp8_workspace_bytes", M, N, K, ctypes.byref(need))
+    assert need.value > 0
+    g = _gen(16)
+    a = torch.randint(-1, 2, (M, K), generator=g).float() * (torch.randint(0, 8, (M, K), generator=g) == 0)
+    b = torch.randint(-1, 2, (K, N), generator=g).float()
+    want = a @ b            # whole numbers below 2^24: exact
+    assert want.abs().max() < 2048
+    a8, b8 = a.to(fp8), b.to(fp8)
+    for ta in (False, True):
+        for tb in (False, True):
+            print(f"gemm {fp8} split ta={ta} tb={tb} {M}x{N}x{K}", flush=True)
+            ad = a8.t().contiguous().cuda().t() if ta else a8.cuda()
+            bd = b8.t().contiguous().cuda().t() if tb else b8.cuda()
+            got = ops.matmul(ad, bd)
+            assert torch.equal(got.cpu().float(), want)
+            leaky = torch.where(want >= 0, want, 0.01 * want)
+            assert (ops.matmul(ad, bd, activation="leaky_relu").cpu().float() - leaky).abs().max() <= 2048 * 0.01 * 2 ** -11
 
 
 def test_gemm_leaky_relu_epilogue(ops):
