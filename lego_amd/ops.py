@@ -184,18 +184,17 @@ def _operand(t, name):
     raise ValueError(f"{name} must be contiguous or the transpose of a contiguous tensor")
 
 
-_gemm_workspace = {}      # (entry point, M, N, K) -> bytes of workspace that the product uses
+_gemm_workspace, _fp8_workspace = {}, {}      # (M, N, K) -> bytes of workspace that the product uses
 
 
-def _workspace_bytes(entry, M, N, K):
-    need = _gemm_workspace.get((entry, M, N, K))
-    if need is None:      # asked once per shape
-        size = ctypes.c_ulonglong(0)
-        runtime.call(entry, M, N, K, ctypes.byref(size))
-        if len(_gemm_workspace) >= 4096:
-            _gemm_workspace.clear()
-        need = _gemm_workspace[(entry, M, N, K)] = size.value
-    return need
+def _ask_workspace(entry, known, shape):
+    """The size for a shape seen for the first time, kept in ``known``."""
+    size = ctypes.c_ulonglong(0)
+    runtime.call(entry, *shape, ctypes.byref(size))
+    if len(known) >= 4096:
+        known.clear()
+    known[shape] = size.value
+    return size.value
 
 
 def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=torch.float16) -> torch.Tensor:
@@ -215,7 +214,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
         raise ValueError("a and b must have the same dtype")
     if a.dtype in _FP8_FORMAT:
         c = torch.empty((M, N), device=a.device, dtype=torch.float16)
-        need = _workspace_bytes("lego_hip_gemm_fp8_workspace_bytes", M, N, K)
+        need = _fp8_workspace.get((M, N, K))
+        if need is None:
+            need = _ask_workspace("lego_hip_gemm_fp8_workspace_bytes", _fp8_workspace, (M, N, K))
         if need:
             workspace = torch.empty(need // 4, dtype=torch.float32, device=a.device)
             runtime.call("lego_hip_gemm_fp8_ex_ws", _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
@@ -234,7 +235,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     c = torch.empty((M, N), device=a.device, dtype=out_dtype)
     # products of few tiles (a skinny operand, a long K) are split along K when there is room for the partial sums;
     # shapes whose operand rows are not whole 16-byte chunks run on zero-padded copies in the workspace
-    need = _workspace_bytes("lego_hip_gemm_workspace_bytes", M, N, K)
+    need = _gemm_workspace.get((M, N, K))
+    if need is None:
+        need = _ask_workspace("lego_hip_gemm_workspace_bytes", _gemm_workspace, (M, N, K))
     if need:
         workspace = torch.empty(need // 4, dtype=torch.float32, device=a.device)
         element = 0 if a.dtype == torch.float16 else 4 if out_dtype == torch.float16 else 1
