@@ -706,11 +706,18 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
 // Parts along K for a product of few tiles (1: one workgroup per tile does it all): enough parts for two
 // workgroups of 128 x 128 tiles per CU, at least four k-tiles each.  The second launch and the partial sums cost
 // about what 16 k-tiles take, so shallower products stay whole (1024^3: 8.6 us whole, 11.7 in four parts;
-// 512 x 512 x 2048: 13.7 whole, 8.2 in eight).
+// 512 x 512 x 2048: 13.7 whole, 8.2 in eight).  Whole too where the result is more than two tiles' worth of elements per
+// k-tile: about 512 parts of sums then cost more than the shorter chains give (M counts in eights, as padded copies do).
+// us whole / in parts, fp16: 1152 x 1152 x 2048 (81 tiles' worth, 32 k-tiles) 23.3 / 26.7, 1408 x 1408 x 2048 (121, 32)
+// 23.6 / 30.5, 256 x 8192 x 2048 (128, 32) 21.7 / 26.6, 1408 x 1408 x 3072 (121, 48) 34.1 / 37.7; 1024 x 1024 x 2048 (64, 32)
+// 21.3 / 19.7, 1024 x 1152 x 2304 (72, 36) 23.6 / 23.1, 64 x 8192 x 2048 (32, 32) 22.5 / 18.8, 16 x 16384 x 2048 22.9 / 17.1.
+// e5m2, k-tiles of 128: 16 x 8192 x 8192 41.4 / 18.0, 64 x 4096 x 4096 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8, 1024 x 1024 x
+// 4096 (64, 32) 21.7 / 18.8, 256 x 8192 x 8192 (128, 64) 40.2 / 33.4; 1408 x 1408 x 4096 (121, 32) 23.3 / 30.2.
 int splitk_parts(int M, int N, int K, int bk)
 {
   const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
   if (tiles > 128 || depth < 32) return 1;
+  if ((M + 7l) / 8 * 8 * N > 2 * depth * 128 * 128) return 1;
   long parts = (512 + tiles - 1) / tiles;
   if (parts > depth / 4) parts = depth / 4;
   if (parts > 64) parts = 64;
@@ -850,23 +857,11 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
                  stream, LEGO_GEMM_BK_8BIT, 16);
 }
 
-// Parts along K of an 8-bit product: the rule of the 16-bit operands with k-tiles of 128 elements (the same bytes and the
-// same matrix-core time each), but whole where the tiles outnumber two per k-tile: the sums of about 512 parts, 64 KiB
-// each, then cost more than the shorter chains give.  us whole (small tile, A*B^T) / in parts: 16 x 8192 x 8192 (64 tiles,
-// 64 k-tiles) 41.4 / 18.0, 64 x 4096 x 4096 (32, 32) 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8, 1024 x 1024 x 4096 (64, 32)
-// 21.7 / 18.8, 1152 x 1280 x 5888 (90, 46) 32.9 / 32.2, 256 x 8192 x 8192 (128, 64) 40.2 / 33.4; 1408 x 1408 x 4096 (121, 32) 23.3 / 30.2.
-static int splitk_parts_8bit(int M, int N, int K)
-{
-  const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128);
-  const long depth = (K + LEGO_GEMM_BK_8BIT - 1) / LEGO_GEMM_BK_8BIT;
-  return tiles > 2 * depth ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT);
-}
-
 // Room for the sums of a split product; none where gemm_ex would not take the tiled kernels in any layout.
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
-  const int parts = N % 16 ? 1 : splitk_parts_8bit(M, N, K);
+  const int parts = N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT);
   const unsigned long long tiles = static_cast<unsigned long long>((M + 127) / 128) * ((N + 127) / 128);
   *bytes = parts > 1 ? parts * tiles * 128ull * 128ull * sizeof(float) : 0ull;
   return 0;
@@ -884,7 +879,7 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
-  return ok_or((format == 0 ? e4m3 : e5m2)[layout](a, b, c, M, N, K, activation, splitk_parts_8bit(M, N, K),
+  return ok_or((format == 0 ? e4m3 : e5m2)[layout](a, b, c, M, N, K, activation, splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT),
                                                    static_cast<float*>(workspace), as_stream(stream)));
 }
 

@@ -88,5 +88,12 @@ def test_workspace_sizes_follow_the_launch_rules():
         r8 = lambda v: (v + 7) // 8 * 8
         assert need.value >= 2 * (r8(M) * r8(K) + r8(K) * r8(N) + r8(M) * r8(N)), (M, N, K)
         assert need.value % 16 == 0
+    for fn, bk in ((lib.lego_hip_gemm_workspace_bytes, 64), (lib.lego_hip_gemm_fp8_workspace_bytes, 128)):
+        for M, N in ((1, 64), (16, 16384), (1024, 1024), (1017, 1024), (1024, 1040), (1408, 1408), (2048, 2048)):
+            for depth in (31, 32, 64, 65):
+                assert fn(M, N, depth * bk, ctypes.byref(need)) == 0
+                tiles = -(-M // 128) * -(-N // 128)
+                split = tiles <= 128 and depth >= 32 and (M + 7) // 8 * 8 * N <= 2 * depth * 128 * 128
+                assert (need.value > 0) == split and need.value % (tiles * 65536) == 0, (M, N, depth, need.value)
     for M, N, K in ((4096, 4096, 4096), (1001, 264, 200), (2048, 1024, 64)):     # M alone never asks for copies
         assert lib.lego_hip_gemm_workspace_bytes(M, N, K, ctypes.byref(need)) == 0 and need.value == 0, (M, N, K)
