@@ -12,9 +12,10 @@ Here a block is 64 x 64, ``T = 16`` and ``R = 4`` (256 lanes per trailing block)
 inverse places the lanes that stage the two panels in LDS, and the offsets of a block's elements
 in the ``n x n`` matrix are those of ``OrderBy(Row(n, n)).TileBy([n/64, n/64], [64, 64])``.  The
 product itself runs on the fp32 matrix cores, whose accumulator layout is one more LEGO
-expression (``Row(4, 2, 4)``).  The diagonal block is eliminated by one wavefront with row ``t`` in
-lane ``t``'s registers; a panel block is solved by one wavefront, a lane per column (row panel) or
-per row (column panel), with the diagonal block's elements read across lanes.
+expression (``Row(4, 2, 4)``).  The diagonal block is eliminated by four wavefronts, sixteen columns each,
+row ``t`` in lane ``t``'s registers; a panel block is solved by four wavefronts, sixteen columns (row
+panel) or rows (column panel) each, in 16 x 16 tiles: products of tiles on the matrix cores, substitution
+inside a diagonal tile.
 """
 from __future__ import annotations
 

@@ -248,16 +248,22 @@ def test_gpu_call_with_second_stream_replays_from_a_hip_graph():
         del graph
 
 
+def _factored(a):
+    from lego_amd import ops
+    return ops.lud(torch.from_numpy(a.astype(np.float32)).cuda()).cpu().numpy().astype(np.float64)
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [64, 128, 192])
-@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30, 2.0 ** -130])
+@pytest.mark.parametrize("scale", [1.0, 1e-30, 1e30, 2.0 ** -130, 2.0 ** -136])
 def test_gpu_pivots_of_any_magnitude(n, scale):
-    """Pivots near the ends of the exponent range take true divisions (2^-130: denormal ones); the rounding of the
-    elements themselves, n of them summed, bounds L - L' and (U - U') / scale."""
-    from lego_amd import ops
+    """Pivots near the ends of the exponent range take true divisions; the last scale makes them subnormal, below 2^-128,
+    where a reciprocal overflows.  The rounding of the elements themselves, n of them summed, bounds L - L' and
+    (U - U') / scale."""
     print(f"lud n={n} scale={scale}", flush=True)
     a = (_dominant(n, n + 1) * scale).astype(np.float32)
-    got = ops.lud(torch.from_numpy(a).cuda()).cpu().numpy().astype(np.float64)
+    assert scale > 2.0 ** -136 or np.abs(np.diagonal(a)).max() < 2.0 ** -128
+    got = _factored(a)
     want = ok.lud(a.astype(np.float64))
     spacing = max(2.0 ** -24, 2.0 ** -149 / (scale * n))      # of the pivots, which are about n * scale
     assert np.abs(np.tril(got - want, -1)).max() <= 4 * n * spacing
@@ -265,12 +271,55 @@ def test_gpu_pivots_of_any_magnitude(n, scale):
 
 
 @pytest.mark.gpu
-def test_gpu_non_finite_elements_stay_where_elimination_takes_them():
-    """A NaN reaches the blocks that depend on it and no other: the first block row and column of a matrix whose last block
-    has one are the factors of the matrix without it."""
-    from lego_amd import ops
-    a = torch.from_numpy(_dominant(192, 3).astype(np.float32))
-    want = ops.lud(a.clone().cuda()).cpu()
-    a[150, 160] = float("nan")
-    got = ops.lud(a.cuda()).cpu()
-    assert torch.equal(got[:128, :128], want[:128, :128]) and got[150, 160].isnan()
+@pytest.mark.parametrize("n", [128, 192])
+def test_gpu_upper_triangle_is_its_own_decomposition(n):
+    """Ones above a small diagonal: L = I and U the matrix itself, exactly, though the inverse of a 16 x 16 tile of it is beyond
+    the range of floats."""
+    a = np.triu(np.ones((n, n)), 1) + np.float64(np.float32(0.003)) * np.eye(n)
+    assert np.array_equal(_factored(a), a)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["normal", "uniform"])
+@pytest.mark.parametrize("n", [128, 256])
+def test_gpu_residual_is_that_of_elimination(n, kind):
+    """Matrices that no diagonal dominates, whose blocks and tiles may be ill-conditioned: A - L U against |L| |U| stays within
+    twice that of the elimination done in float32, element by element, on the host."""
+    print(f"lud n={n} {kind}", flush=True)
+
+    def residual(a, w):
+        low, up = np.tril(w, -1) + np.eye(n), np.triu(w)
+        return np.linalg.norm(a - low @ up) / np.linalg.norm(np.abs(low) @ np.abs(up))
+
+    for seed in range(6):
+        rng = np.random.default_rng(seed)
+        a = (rng.standard_normal((n, n)) if kind == "normal" else rng.uniform(0, 1, (n, n))).astype(np.float32)
+        host = a.copy()
+        for k in range(n - 1):
+            host[k + 1:, k] /= host[k, k]
+            host[k + 1:, k + 1:] -= np.outer(host[k + 1:, k], host[k, k + 1:])
+        a = a.astype(np.float64)
+        assert residual(a, _factored(a)) <= 2 * residual(a, host.astype(np.float64)), seed
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("at,value", [((10, 100), np.inf), ((100, 10), np.inf), ((10, 100), np.nan), ((100, 40), np.nan),
+                                      ((63, 64), -np.inf), ((64, 63), np.inf), ((0, 190), np.inf), ((150, 160), np.nan), ((40, None), 0.0)])
+def test_gpu_non_finite_elements_stay_where_elimination_takes_them(at, value):
+    """An infinity or NaN in a panel of the first step, in a later block, or a zero pivot (a row of zeros): what elimination
+    leaves finite is finite and the same, but for diagonal blocks that have other elements: rows that are done take
+    the multiplier 0 there, and 0 times an infinity is none."""
+    print(f"lud {value} at {at}", flush=True)
+    a = _dominant(192, 3).astype(np.float32)
+    a[at[0], slice(None) if at[1] is None else at[1]] = value
+    with np.errstate(all="ignore"):
+        want = ok.lud(a.astype(np.float64))
+    got = _factored(a)
+    finite = np.isfinite(want)
+    assert not np.isfinite(got[~finite]).any()
+    for k in range(0, 192, 64):
+        block = finite[k:k + 64, k:k + 64]
+        block &= block.all()
+    assert want.size // 4 < np.count_nonzero(finite) < want.size
+    assert np.isfinite(got[finite]).all()
+    assert np.abs(got[finite] - want[finite]).max() <= 2e-5 * np.abs(want[finite]).max()
