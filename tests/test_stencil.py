@@ -230,6 +230,57 @@ def test_gpu_stencil_columns_and_bricks_agree(kind, radius, n):
         assert (want[full, full, full] - ref[k, k, k]).abs().max().item() <= 2e-5 * (2 * radius + 1) ** 3
 
 
+def _fused(a, b, c):
+    """a * b + c with one rounding to float32 (64 bits hold the product; the sum is rounded twice in one of 2^29 cases)."""
+    return (a.double() * b.double() + c.double()).float()
+
+
+def _shifted(x, r, di, dj, dk):
+    n = x.shape[0]
+    return x[r + di:n - r + di, r + dj:n - r + dj, r + dk:n - r + dk]
+
+
+def _in_order(kind, x, c, r):
+    """The interior points, rounded as the kernels are meant to: the centre's product inside the first sum."""
+    if kind == "laplacian":
+        acc = None
+        for a in range(1, r + 1):
+            six = _shifted(x, r, a, 0, 0)
+            for step in ((0, a, 0), (0, 0, a), (0, 0, -a), (0, -a, 0), (-a, 0, 0)):
+                six = six + _shifted(x, r, *step)
+            acc = _fused(_shifted(x, r, 0, 0, 0), c[0], c[1] * six) if a == 1 else _fused(six, c[a], acc)
+        return acc
+    acc, span = None, range(-r, r + 1)
+    for di in span:
+        for dj in span:
+            for dk in span:
+                v, w = _shifted(x, r, di, dj, dk), c[di + r, dj + r, dk + r]
+                acc = _fused(_shifted(x, r, 0, 0, 0), c[r, r, r], v * w) if acc is None else _fused(v, w, acc)
+    return acc
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [24, 136, 192])
+@pytest.mark.parametrize("kind,radius", [("laplacian", 1), ("laplacian", 2), ("laplacian", 4), ("f3d", 1), ("f3d", 2)])
+def test_gpu_stencil_rounds_the_centre_with_the_first_sum(kind, radius, n):
+    """Both kernels and storages, and the precision that goes with the order: the distance of a Laplacian's results from 64 bits is
+    up to a third larger when the product of its centre, the largest one, is rounded by itself."""
+    from lego_amd import ops
+    print(f"{kind} n={n} radius={radius}", flush=True)
+    x = torch.rand(n, n, n, generator=torch.Generator().manual_seed(n)) * 2 - 1
+    if kind == "f3d":
+        call, c = ops.stencil_f3d, torch.from_numpy(_coefficients(radius))
+    else:
+        call, c = ops.stencil_laplacian, torch.tensor([-6.1, 1.1, 0.53, 0.27, 0.129])[:radius + 1].contiguous()
+    want = _in_order(kind, x, c, radius)
+    order = ok.bricks_order(n)
+    inner = (slice(radius, n - radius),) * 3
+    for bricks in (False, True):
+        got = call(_to_bricks(x, order).cuda() if bricks else x.cuda(), c.cuda(), radius, bricks).cpu()
+        got = (_from_bricks(got, order) if bricks else got)[inner]
+        assert (got != want).sum().item() <= 2 + want.numel() // 10 ** 7
+
+
 @pytest.mark.gpu
 def test_gpu_stencil_rejects_bad_arguments():
     from lego_amd import ops
