@@ -198,10 +198,12 @@ def test_gpu_stencils_full_size_agree_between_layouts():
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("kind,radius,n", [("f3d", 1, 128), ("f3d", 1, 136), ("f3d", 2, 200), ("f3d", 3, 264), ("laplacian", 1, 128),
+@pytest.mark.parametrize("kind,radius,n", [("f3d", 1, 128), ("f3d", 1, 136), ("f3d", 2, 200), ("f3d", 2, 248),
+                                           ("f3d", 2, 280), ("f3d", 3, 264), ("f3d", 3, 320), ("laplacian", 1, 128),
                                            ("laplacian", 2, 152), ("laplacian", 3, 200), ("laplacian", 4, 136), ("laplacian", 4, 192)])
 def test_gpu_stencil_columns_and_bricks_agree(kind, radius, n):
-    """From these sizes on row-major fields are walked column by column, in sizes that leave lanes, rows and planes over;
+    """Row-major fields of about these sizes are walked column by column, also where lanes, rows and planes are left over (the
+    dense stencils of radius 2 and 3 where few are);
     the bricks storage (radius 4: its columns too) gives the same bits, an `out` of the caller's keeps its boundary and the
     default one has zeros there.  The field around the smallest such column agrees with the oracle."""
     from lego_amd import ops
