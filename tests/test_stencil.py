@@ -232,6 +232,21 @@ def test_gpu_stencil_columns_and_bricks_agree(kind, radius, n):
         assert (want[full, full, full] - ref[k, k, k]).abs().max().item() <= 2e-5 * (2 * radius + 1) ** 3
 
 
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,radius", [(520, 1), (520, 3), (728, 2)])
+def test_gpu_star_columns_of_large_fields_agree_with_bricks(n, radius):
+    """Beyond n = 512 a star's columns are cut into shorter chunks; on bricks up to radius 3 a wavefront has a brick."""
+    from lego_amd import ops
+    print(f"laplacian n={n} radius={radius}", flush=True)
+    m = n // 8
+    x = torch.rand(n, n, n, device="cuda", generator=torch.Generator(device="cuda").manual_seed(n)) * 2 - 1
+    c = torch.tensor([-6.0, 1.0, 0.5, 0.25], device="cuda")[:radius + 1].contiguous()
+    a = ops.stencil_laplacian(x, c, radius, False)
+    b = ops.stencil_laplacian(x.view(m, 8, m, 8, m, 8).permute(0, 2, 4, 1, 3, 5).contiguous().view(n, n, n), c, radius, True)
+    assert torch.equal(a, b.view(m, m, m, 8, 8, 8).permute(0, 3, 1, 4, 2, 5).reshape(n, n, n))
+    assert a[radius:-radius, radius:-radius, radius:-radius].abs().max().item() > 0
+
+
 def _fused(a, b, c):
     """a * b + c with one rounding to float32 (64 bits hold the product; the sum is rounded twice in one of 2^29 cases)."""
     return (a.double() * b.double() + c.double()).float()
