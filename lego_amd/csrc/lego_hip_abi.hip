@@ -706,18 +706,20 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
 // Parts along K for a product of few tiles (1: one workgroup per tile does it all): enough parts for two
 // workgroups of 128 x 128 tiles per CU, at least four k-tiles each.  The second launch and the partial sums cost
 // about what 16 k-tiles take, so shallower products stay whole (1024^3: 8.6 us whole, 11.7 in four parts;
-// 512 x 512 x 2048: 13.7 whole, 8.2 in eight).  Whole too where the result is more than two tiles' worth of elements per
-// k-tile: about 512 parts of sums then cost more than the shorter chains give (M counts in eights, as padded copies do).
-// us whole / in parts, fp16: 1152 x 1152 x 2048 (81 tiles' worth, 32 k-tiles) 23.3 / 26.7, 1408 x 1408 x 2048 (121, 32)
-// 23.6 / 30.5, 256 x 8192 x 2048 (128, 32) 21.7 / 26.6, 1408 x 1408 x 3072 (121, 48) 34.1 / 37.7; 1024 x 1024 x 2048 (64, 32)
-// 21.3 / 19.7, 1024 x 1152 x 2304 (72, 36) 23.6 / 23.1, 64 x 8192 x 2048 (32, 32) 22.5 / 18.8, 16 x 16384 x 2048 22.9 / 17.1.
-// e5m2, k-tiles of 128: 16 x 8192 x 8192 41.4 / 18.0, 64 x 4096 x 4096 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8, 1024 x 1024 x
-// 4096 (64, 32) 21.7 / 18.8, 256 x 8192 x 8192 (128, 64) 40.2 / 33.4; 1408 x 1408 x 4096 (121, 32) 23.3 / 30.2.
+// 512 x 512 x 2048: 13.7 whole, 8.2 in eight).  More workgroups also keep more loads in flight, so parts gain most where operands come
+// from memory, whatever the size of the result.  us whole / in parts, fp16, operands from memory, and in brackets from the
+// caches: 1024 x 1536 x 2048 27.5 / 26.2 (21.3 / 24.0), 1024 x 2048 x 3584 49.4 / 32.7 (34.8 / 30.8), 384 x 5120 x 3072 43.3 / 39.1 (30.6 /
+// 34.1), 256 x 8192 x 2304 33.2 / 28.1 (24.3 / 25.3), 8192 x 256 x 3584 49.1 / 34.5 (36.0 / 28.7), 1496 x 1144 x 3024 50.6 / 36.9 (38.9 / 35.7);
+// over 87 products of 2 to 4 tiles' worth of result per k-tile parts take 0.86 of the time from memory, 1.01 from the caches.
+// 8-bit operands are half as many bytes beside the same sums: a product whose result is more than two tiles' worth of
+// elements per k-tile stays whole, 21.6 against 24.3 from the caches at 384 x 4096 x 4096 with B transposed (28.4 / 26.7 from memory),
+// 24.1 / 27.6 at 4608 deep; below, k-tiles of 128: 16 x 8192 x 8192 41.4 / 18.0, 64 x 4096 x 4096 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8,
+// 1024 x 1024 x 4096 21.7 / 18.8.
 int splitk_parts(int M, int N, int K, int bk)
 {
   const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
   if (tiles > 128 || depth < 32) return 1;
-  if ((M + 7l) / 8 * 8 * N > 2 * depth * 128 * 128) return 1;
+  if (bk == LEGO_GEMM_BK_8BIT && static_cast<long>(M) * N > 2 * depth * 128 * 128) return 1;
   long parts = (512 + tiles - 1) / tiles;
   if (parts > depth / 4) parts = depth / 4;
   if (parts > 64) parts = 64;
