@@ -217,7 +217,8 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
         need = _fp8_workspace.get((M, N, K))
         if need is None:
             need = _ask_workspace("lego_hip_gemm_fp8_workspace_bytes", _fp8_workspace, (M, N, K))
-        if need:
+        # the size is for any layout: one whose rows are not whole 16-byte chunks runs without
+        if need and (M if ta else K) % 16 == 0 and not (tb and K % 16):
             workspace = torch.empty(need // 4, dtype=torch.float32, device=a.device)
             runtime.call("lego_hip_gemm_fp8_ex_ws", _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
                          1 if activation else 0, _FP8_FORMAT[a.dtype], _ptr(workspace), need, _stream())

@@ -1355,6 +1355,25 @@ def test_gemm_fp8_split_along_k(ops, fp8, M, N, K):
             assert (ops.matmul(ad, bd, activation="leaky_relu").cpu().float() - leaky).abs().max() <= 2048 * 0.01 * 2 ** -11
 
 
+@pytest.mark.parametrize("M,N,K,ta,tb,split", [(16, 64, 4096, 0, 0, True), (24, 64, 4096, 0, 1, True), (24, 64, 4096, 1, 0, False),
+                                               (32, 64, 4104, 0, 0, False), (32, 64, 4104, 1, 0, True), (32, 64, 4104, 1, 1, False)])
+def test_gemm_fp8_brings_a_workspace_only_where_it_is_used(ops, monkeypatch, M, N, K, ta, tb, split):
+    """Layouts whose rows are not whole 16-byte chunks stay whole: no workspace is allocated for them."""
+    from lego_amd import runtime
+    print(f"gemm e5m2 {M}x{N}x{K} ta={ta} tb={tb}", flush=True)
+    g = _gen(17)
+    a = torch.randint(-1, 2, (M, K), generator=g).float() * (torch.randint(0, 4, (M, K), generator=g) == 0)
+    b = torch.randint(-1, 2, (K, N), generator=g).float()
+    a8, b8 = a.to(torch.float8_e5m2), b.to(torch.float8_e5m2)
+    ad = a8.t().contiguous().cuda().t() if ta else a8.cuda()
+    bd = b8.t().contiguous().cuda().t() if tb else b8.cuda()
+    calls, call = [], runtime.call
+    monkeypatch.setattr(runtime, "call", lambda name, *args: (calls.append(name), call(name, *args))[1])
+    got = ops.matmul(ad, bd)
+    assert ("lego_hip_gemm_fp8_ex_ws" in calls) == split
+    assert torch.equal(got.cpu().float(), a @ b)
+
+
 def test_gemm_leaky_relu_epilogue(ops):
     print("gemm leaky_relu", flush=True)
     g = _gen(8)
