@@ -48,6 +48,11 @@ def lds_a_layout(bm, chunks):
     return OrderBy(GenP((bm, chunks), forward, backward)).TileBy([bm, chunks])
 
 
+def _rows_per_key(bn, period):
+    """Consecutive k-rows of a ``[bk][bn]`` tile that share a key: rows of under ``period`` chunks."""
+    return max(1, 32 * period // bn)
+
+
 def lds_b_layout(bk, bn, period=4, groups_by_k=False):
     """B tile in elements, rows of ``bn``: ``k*bn + (n ^ 32*(k % period))``.
 
@@ -62,7 +67,7 @@ def lds_b_layout(bk, bn, period=4, groups_by_k=False):
     (bits 0-3 stay, so 16-byte stores and 8-byte reads are still whole)."""
     assert not groups_by_k or (period == 4 and bn >= 128)
 
-    rows_per_key = max(1, 32 * period // bn)      # rows of under `period` chunks share a key
+    rows_per_key = _rows_per_key(bn, period)
 
     def key(k):
         if rows_per_key > 1:
@@ -454,7 +459,9 @@ def _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped,
     tag = ("" if (bm, bn) == (256, 256) else f"_t{bm}x{bn}") + ("" if tuple(waves) == (2, 2) else f"_w{WAVES_M}x{WAVES_N}") + suffix
     chunk_params = dict(WAVES=WAVES, variant=variant, tag=tag, with_grouped=with_grouped, **operand("a"), **operand("b"))
 
+    shared = _rows_per_key(bn, 4 if esize == 2 else 8)
     params = dict(
+        KEY="k%8" if shared == 1 else f"(k/{shared})%{8 // shared}",      # of an 8-bit [bk][bn] tile (lds_b_layout)
         banner=BANNER, elt=elt, out_elt=out_elt, ESIZE=esize, EPC=EPC, MFMA_K=mfma_k, NPH=NPH,
         FMT={"e4m3": 0, "e5m2": 1}.get(dtype, 0), dt=dtype, mfma_dt={"bf16h": "bf16"}.get(dtype, dtype), BM=bm, BN=bn, BK=bk, THREADS=THREADS, WAVES_M=WAVES_M, WAVES_N=WAVES_N,
         WM=WM, WN=WN, TM=TM, TN=TN, A_ITERS=A_ITERS, B_ITERS=B_ITERS, DMA_LAST=DMA_LAST,
