@@ -12,9 +12,8 @@
  *     entry points (*_wpr, *_split) ask for 16 bytes.  Nothing is allocated, freed or
  *     synchronised: the kernel is enqueued on `stream` (a hipStream_t; NULL = the default
  *     stream) and the call returns;
- *   - re-entrant: safe from several host threads on distinct streams.  Two entry points keep state between
- *     calls, both described where they are declared: lego_hip_lud_f32 (a side stream per caller's stream) and
- *     lego_hip_layernorm_bwd_f16_noalloc (a built-in scratch array per device).
+ *   - re-entrant: safe from several host threads on distinct streams.  One entry point keeps state between
+ *     calls, described where it is declared: lego_hip_layernorm_bwd_f16_noalloc (a built-in scratch array per device).
  *
  * The reference has no FFI: its kernels are reached through generated Python host
  * functions.  Each entry point below names the reference host function it stands behind.
@@ -183,26 +182,17 @@ int lego_hip_stencil_laplacian_f32_zeros(const float* in, float* out, const floa
  * strict lower triangle holds L (unit diagonal implied) and the upper triangle holds U, as
  * Rodinia's lud (the reference's thread-coarsening benchmark: benchmarks/cuda/lud.py:5-12,
  * kernels lud/lud_kernel_temp.cu:14-352, host loop :358-390).  n a multiple of 64, at most 32768.
- * From n = 4928 on, part of the work is enqueued on a second stream, forked from and joined back into
- * `stream` with events inside the call, so the caller sees ordinary stream order (captured into a graph,
- * the fork and join become graph edges).  The library makes that stream and its two events on the first
- * such call for a given (device, `stream`) pair -- the device of `stream` must be current -- and keeps
- * them until the process ends: callers on distinct streams share nothing.  After 32 such pairs, and for a
- * `stream` that is under capture the first time it is seen (nothing is created during a capture), the
- * call stays on `stream` alone (same results, less overlap).  Concurrent calls on the SAME `stream` from
- * several threads are not supported, as for any stream-ordered work. */
+ * Two block steps of 64 per pair of launches, all on `stream`; nothing is kept between calls. */
 int lego_hip_lud_f32(float* m, int n, void* stream);
 
-/* The launches that lego_hip_lud_f32 enqueues for an n x n matrix, in order, without touching a device: six
- * ints per launch, {kind, stream, a, b, c, d}, stream 0 = the caller's, 1 = the library's second one.
- *   kind 0 panels of step a (b workgroups);  1 strip: block row and column a+1 against step a (b = blocks left in
- *   a block row);  2 the two block rows and columns at the top and left of the square of side c from block b on,
- *   against steps a, a+1;  3 trailing update of the square of side c from block b on against d/16 steps from a on,
- *   d%16 blocks per workgroup;  4 fork (stream 1 waits for stream 0);  5 join (stream 0 waits for stream 1);
+/* What lego_hip_lud_f32 does to an n x n matrix in blocks of 64, in order, without touching a device: six ints per
+ * record, {kind, 0, a, b, c, d}; a launch does one or more of them.
+ *   kind 0 panels of step a (b blocks each);  1 block row and column a+1 against step a (b = blocks left in
+ *   a block row);  3 trailing update of the square of side c from block b on against d/16 steps from a on (d%16 is 1);
  *   6 factors of the a diagonal blocks written.
  * At most `capacity` records are written; *count receives how many there are.  No counterpart in the
  * reference (its host loop, lud_kernel_temp.cu:358-390, is three launches per step on one stream): it is
- * there so that the order and the overlap of the launches can be checked on the host. */
+ * there so that the order of the work can be checked on the host. */
 int lego_hip_lud_f32_plan(int n, int* records, int capacity, int* count);
 
 /* Needleman-Wunsch score matrix (Rodinia's needle, the reference's anti-diagonal layout

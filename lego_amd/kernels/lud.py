@@ -23,14 +23,13 @@ from ..lego import Col, OrderBy, Row, le_constraint
 from .common import BANNER, Emitted, code, idx, size, template, tidy
 
 B, T, R = 64, 16, 4
-STEPS = 4      # elimination steps of a diagonal block between two exchanges among its wavefronts
-# side (in blocks) of the trailing square from which the next panels are solved on a second stream meanwhile
-AHEAD_MIN = 72
-# the trailing square is walked in groups of GROUP block rows, column by column inside a group (the grouped launch
+P = 2 * B      # two block steps between two passes over the trailing square
+# side (in blocks) of the trailing square from which the next panels are solved on a second stream meanwhile: none, the
+# trailing launch itself factors ahead (a matrix has at most 512 blocks a side)
+AHEAD_MIN = 512
+# the trailing square is walked in groups of up to GROUP block rows, column by column inside a group (the grouped launch
 # order of the reference's matmul, matmul_sympy.py:57-65), and each of the XCDS L2 caches gets a contiguous run of it
-GROUP, XCDS = 8, 8
-# a workgroup takes a run of up to GROUP blocks of a column as long as that leaves this many workgroups (two per CU, twice)
-MIN_WGS = 1024
+GROUP, XCDS, CUS = 8, 8, 256
 
 
 def block_order(ng, q, nsub, pid):
@@ -65,21 +64,20 @@ def emit():
     # the matrix core's accumulator: register q of lane l holds row Row(4, 2, 4)[q/4, l/32, q%4] of its 32 x 32 result
     q, l = idx("q"), idx("l")
     acc_row = tidy(OrderBy(Row(4, 2, 4)).TileBy([4, 2, 4])[q // 4, l // 32, q % 4], {q: (0, 16), l: (0, 64)})
-    ng, qq, per, pid, wg = size("ng"), size("q"), size("per"), idx("pid"), idx("wg")
-    nsub = size("nsub")
-    og, oc, osub = (tidy(e, {pid: (0, ng * qq * nsub)}) for e in block_order(ng, qq, nsub, pid))
+    ng, q2, per, pid, wg = size("ng"), size("q2"), size("per"), idx("pid"), idx("wg")
+    og, oc, _ = (tidy(e, {pid: (0, ng * q2)}) for e in block_order(ng, q2, 1, pid))     # a workgroup takes all rows of its group
     xcd_pid = tidy(xcd_remap(per, wg), {wg: (0, per * XCDS)})
     # k of the j-th matrix-core instruction in lane l: Row(2, 32)[l/32, j] (halves of the wavefront take halves of k)
     j = idx("j")
     k_of_lane = tidy(OrderBy(Row(2, B // 2)).TileBy([2, B // 2])[l // 32, j], {l: (0, 64), j: (0, B // 2)})
     params = dict(
-        banner=BANNER, B=B, T=T, R=R, STEPS=STEPS, AHEAD_MIN=AHEAD_MIN,
+        banner=BANNER, B=B, T=T, R=R, P=P,
         matrix_layout=f"OrderBy(Row(n, n)).TileBy([n/{B}, n/{B}], [{B}, {B}])[bi, bj, r, c]",
         thread_layout=f"OrderBy(Row({R * T}, {R * T})).GroupBy([({R}, {R}), ({T}, {T})]).inv((ii*{R} + jj)*{T * T} + tid)",
         elem=code(elem), ci=code(i_e), cj=code(j_e), cty=code(ty_e), ctx=code(tx_e),
-        acc_row=code(acc_row), k_of_lane=code(k_of_lane), k_layout=f"Row(2, {B // 2})[l/32, j]", GROUP=GROUP, XCDS=XCDS,
-        order_g=code(og), order_c=code(oc), order_sub=code(osub), xcd_pid=code(xcd_pid), MIN_WGS=MIN_WGS,
-        order_layout="OrderBy(Row(ng, q, nsub)).TileBy([ng, q, nsub]).inv(pid) -> (group, column, part)",
+        acc_row=code(acc_row), k_of_lane=code(k_of_lane), k_layout=f"Row(2, {B // 2})[l/32, j]", GROUP=GROUP, XCDS=XCDS, CUS=CUS,
+        order_g=code(og), order_c=code(oc), xcd_pid=code(xcd_pid),
+        order_layout="OrderBy(Row(ng, q2, 1)).TileBy([ng, q2, 1]).inv(pid) -> (group, column, 0)",
         xcd_layout=f"OrderBy(Col(per, {XCDS})).TileBy([per, {XCDS}])[Row(per, {XCDS}).inv(wg)]",
     )
     text = template("lud.hip.j2").render(**params)

@@ -185,6 +185,20 @@ def test_gpu_matches_oracle(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n", [192, 320, 576, 1088, 1152])
+def test_gpu_odd_block_counts_and_run_lengths(n):
+    """A last block that is no pair, a second column of blocks past the matrix, runs of one and more block rows with a short
+    last one: the factors against the oracle's, each rounded some n times at the size of the pivots."""
+    from lego_amd import ops
+    print(f"lud n={n}", flush=True)
+    a = _dominant(n, 300 + n).astype(np.float32)
+    want = ok.lud(a)
+    got = ops.lud(torch.from_numpy(a.copy()).cuda()).cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(got - want) <= n * 2.0 ** -24 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+@pytest.mark.gpu
 def test_gpu_rejects_bad_sizes():
     from lego_amd import ops
     from lego_amd.runtime import LegoHipError
