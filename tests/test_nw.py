@@ -105,6 +105,22 @@ def test_gpu_single_launch_agrees_with_a_launch_per_anti_diagonal(n):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("n,penalty", [(320, 2 ** 31 - 1), (384, -(2 ** 31)), (576, -7)])
+def test_gpu_single_launch_wraps_as_the_tiles_do(n, penalty):
+    """Scores, borders and penalties over the whole range of the type: sums are modulo 2^32 in both forms of the recurrence,
+    and what is compared has the same bits."""
+    from lego_amd import ops, runtime
+    print(f"needleman-wunsch n={n}, whole range", flush=True)
+    g = torch.Generator().manual_seed(n + 1)
+    lo, hi = -(2 ** 31), 2 ** 31 - 1
+    ref = torch.randint(lo, hi, (n + 1, n + 1), generator=g, dtype=torch.int32).cuda()
+    m = torch.randint(lo, hi, (n + 1, n + 1), generator=g, dtype=torch.int32).cuda()
+    want = m.clone()
+    runtime.call("lego_hip_nw_i32", ref.data_ptr(), want.data_ptr(), n, penalty, None)
+    assert torch.equal(ops.needleman_wunsch(ref, m, penalty), want)
+
+
+@pytest.mark.gpu
 def test_gpu_rejects_bad_sizes():
     from lego_amd import ops
     from lego_amd.runtime import LegoHipError
