@@ -21,6 +21,7 @@ from .lego_hip import HIPCC_FLAGS, hipcc_path
 ROOT = Path(__file__).resolve().parents[1]
 LIB_DIR = Path(__file__).resolve().parent / "lib"
 LIB_PATH = LIB_DIR / "liblego_hip.so"
+NODE_PATH = LIB_DIR / "layernorm_node.so"
 OBJ_DIR = LIB_DIR / "obj"
 
 # the tilings the library is built with
@@ -376,8 +377,30 @@ def _compile(src: Path, incremental: bool = False) -> Path:
     return obj
 
 
+def build_node(incremental: bool = False) -> Path:
+    """Compile the LayerNorm node (C++ over torch's headers) beside liblego_hip.so, which it is linked with."""
+    import sysconfig
+
+    import torch
+    from torch.utils import cpp_extension
+    src = CSRC / f"{NODE_PATH.stem}.cpp"
+    if incremental and NODE_PATH.exists() and NODE_PATH.stat().st_mtime > max(p.stat().st_mtime for p in (src, ROOT / "include" / "lego_hip.h")):
+        return NODE_PATH
+    includes = [str(ROOT / "include"), *cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
+    libs = cpp_extension.library_paths()
+    cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DTORCH_EXTENSION_NAME={NODE_PATH.stem}",
+           *[a for i in includes for a in ("-I", i)], str(src), "-o", str(NODE_PATH),
+           *[a for d in libs for a in ("-L", d, f"-Wl,-rpath,{d}")], "-L", str(LIB_DIR), "-Wl,-rpath,$ORIGIN", f"-l:{LIB_PATH.name}",
+           "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-ltorch_hip"]
+    res = subprocess.run(cmd, capture_output=True, text=True)
+    if res.returncode != 0:
+        raise RuntimeError(f"g++ failed on {src.name}:\n{res.stderr}")
+    return NODE_PATH
+
+
 def build(verbose=True, incremental=False):
-    """Generate, compile every translation unit for gfx950 and link liblego_hip.so.  With
+    """Generate, compile every translation unit for gfx950 and link liblego_hip.so, then the LayerNorm node.  With
     ``incremental`` a translation unit whose object file is newer than its source is kept."""
     sources = generate() + [CSRC / "lego_hip_abi.hip"]
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
@@ -387,6 +410,7 @@ def build(verbose=True, incremental=False):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
+    build_node(incremental)
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} translation units")
     return LIB_PATH

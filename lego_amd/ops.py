@@ -146,8 +146,7 @@ def layer_norm_bwd(dy, x, weight, mean, rstd):
 
 
 class LEGOLayerNorm(torch.autograd.Function):
-    """``lego_layer_norm = LEGOLayerNorm.apply`` with the reference's signature and gradients
-    (triton_generated/layernorm/layernorm.py:323-405)."""
+    """The node of ``lego_layer_norm`` in Python, for calls that the one in C++ leaves to it."""
 
     @staticmethod
     def forward(ctx, x, normalized_shape, weight, bias, eps):
@@ -165,7 +164,15 @@ class LEGOLayerNorm(torch.autograd.Function):
         return dx, None, dw, db, None
 
 
-lego_layer_norm = LEGOLayerNorm.apply
+def lego_layer_norm(x, normalized_shape, weight, bias, eps):
+    """LayerNorm with the reference's signature and gradients (triton_generated/layernorm/layernorm.py:323-407).  Plain GPU
+    tensors go through the node in C++ (csrc/layernorm_node.cpp); subclasses, dual tensors, calls under a tracer, a mode or a
+    transform, and calls that are refused, through the one above."""
+    if not torch.compiler.is_compiling():
+        y = runtime.layernorm_node().apply(x, normalized_shape, weight, bias, eps)
+        if y is not None:
+            return y
+    return LEGOLayerNorm.apply(x, normalized_shape, weight, bias, eps)
 
 
 _GEMM_ENTRY = {torch.float16: "lego_hip_gemm_f16_ex", torch.bfloat16: "lego_hip_gemm_bf16_ex"}

@@ -10,6 +10,7 @@ import ctypes
 from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "liblego_hip.so"
+NODE_PATH = LIB_PATH.with_name("layernorm_node.so")
 
 _c_int, _c_void_p, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_float
 _PTR_ARRAY = ctypes.POINTER(ctypes.c_void_p)
@@ -110,6 +111,25 @@ def load_library(path=None):
     if path is None:
         _lib = lib
     return lib
+
+
+_node = None
+
+
+def layernorm_node():
+    """The extension module with LayerNorm's autograd node, prebuilt beside the library."""
+    global _node
+    if _node is None:
+        import importlib.machinery
+        import importlib.util
+        if not NODE_PATH.exists():
+            raise FileNotFoundError(
+                f"{NODE_PATH} is missing: build it with `python -m lego_amd.build` (there is no fallback path)")
+        loader = importlib.machinery.ExtensionFileLoader("layernorm_node", str(NODE_PATH))
+        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("layernorm_node", loader))
+        loader.exec_module(module)
+        _node = module
+    return _node
 
 
 _entry_points = {}
