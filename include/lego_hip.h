@@ -159,6 +159,12 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes);
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream);
+/* The product on zero-padded copies for operand rows that are not whole 16-byte chunks (lego_hip_gemm_fp8_padded_bytes gives the
+ * size of the workspace, 0 where copies gain nothing): one launch for the copies, the product, one that copies the result back.
+ * Without it (or 16-byte alignment of it) the call is lego_hip_gemm_fp8_ex. */
+int lego_hip_gemm_fp8_padded_bytes(int M, int N, int K, int trans_a, int trans_b, unsigned long long* bytes);
+int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
+                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream);
 
 /* 3-D stencils on an n x n x n fp32 array (the reference's bricks benchmarks:
  * benchmarks/cuda/bricks_f3d.py:8-22 with bricks/main_tmp.cu:24-104, and bricks_laplasian.py:8-33
@@ -224,6 +230,12 @@ int lego_hip_nw_i32_ws(const int* reference, int* matrix, int n, int penalty, vo
 int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* const* c,
                               const int* sizes3, int groups, void* stream);
 
+/* lego_hip_grouped_gemm_f16 with room for zero-padded copies of the problems whose N or K is no multiple of 8: one launch for the
+ * copies, the grouped one for all problems, and one that copies results back.  lego_hip_grouped_gemm_f16_workspace_bytes gives the
+ * size for a list of problems (0: none is needed); without it (or 16-byte alignment of it) the call is lego_hip_grouped_gemm_f16. */
+int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes);
+int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
+                                 void* workspace, unsigned long long workspace_bytes, void* stream);
 /* What lego_hip_grouped_gemm_f16 launches for these sizes, without touching a device: plan3[0] = tile
  * size (256: 256 x 256 tiles, or 128: 128 x 128 tiles), plan3[1] = number of 256 x 256 tiles of all
  * problems, plan3[2] = how many of them, the last ones of the launch order, are computed as two

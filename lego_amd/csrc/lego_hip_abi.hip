@@ -12,6 +12,7 @@
 
 #include <algorithm>
 #include <mutex>
+#include <new>
 #include <vector>
 
 #include "lego_hip.h"
@@ -265,70 +266,92 @@ __global__ void __launch_bounds__(256) lego_mfma_probe_8bit_16x16_kernel(const p
 }
 
 typedef unsigned u32x4w __attribute__((ext_vector_type(4)));
-typedef unsigned u32x4w_any __attribute__((ext_vector_type(4), aligned(2)));     // the same 16 bytes at any 2-byte element
+typedef unsigned u32x4w_any __attribute__((ext_vector_type(4), aligned(1)));     // the same 16 bytes at any byte
 
-// Zero-padded copy of a rows x cols matrix of 2-byte elements (rows at any element alignment) into a
-// rows_to x cols_to one with cols_to a multiple of 8 on a 16-byte aligned base: one lane per 16-byte chunk of
-// the destination, a source chunk that lies inside its row as a whole is one 16-byte access.
-__global__ void __launch_bounds__(256) lego_pad2d_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                         unsigned rows, unsigned cols, unsigned rows_to, unsigned cols_to)
+// Matrices on their way into, or out of, copies whose rows are whole 16-byte chunks on a 16-byte aligned base: up to kCopies of them
+// in one launch, told apart by the running total of workgroups (a launch of its own for each took 2-3 us, more than most of the
+// copies themselves).  One lane per 16-byte chunk; a chunk that lies inside the matrix as a whole is one access on either side.
+constexpr int kCopies = 64;
+struct Copy {
+  const void* from;
+  void* to;
+  unsigned rows, row_bytes;        // of the matrix as it is
+  unsigned rows_to, pitch;         // of the copy: rows beyond `rows` and bytes beyond `row_bytes` are zeros
+  unsigned end;                    // workgroups up to and including this one
+};
+struct Copies {
+  Copy of[kCopies];
+  int count;
+};
+
+template <bool PAD>
+__global__ void __launch_bounds__(256) lego_copies_kernel(const Copies copies)
 {
-  const unsigned per_row = cols_to / 8;
-  const size_t chunk = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
+  int i = 0;
+  while (i + 1 < copies.count && blockIdx.x >= copies.of[i].end) ++i;      // the same for the whole workgroup
+  const Copy c = copies.of[i];
+  const size_t chunk = static_cast<size_t>(blockIdx.x - (i ? copies.of[i - 1].end : 0u)) * 256 + threadIdx.x;
+  const unsigned per_row = c.pitch / 16, at = static_cast<unsigned>(chunk % per_row) * 16;
   const size_t r = chunk / per_row;
-  const unsigned c = static_cast<unsigned>(chunk % per_row) * 8;
-  if (r >= rows_to) return;
-  u32x4w v = {0u, 0u, 0u, 0u};
-  if (r < rows) {
-    const uint16_t* p = src + r * cols + c;
-    if (c + 8 <= cols) {
-      v = *reinterpret_cast<const u32x4w_any*>(p);
+  if (PAD) {
+    if (r >= c.rows_to) return;
+    u32x4w v = {0u, 0u, 0u, 0u};
+    if (r < c.rows && at < c.row_bytes) {
+      const uint8_t* p = static_cast<const uint8_t*>(c.from) + r * c.row_bytes + at;
+      if (at + 16 <= c.row_bytes) {
+        v = *reinterpret_cast<const u32x4w_any*>(p);
+      } else {
+#pragma unroll
+        for (unsigned e = 0; e < 16; ++e)
+          if (at + e < c.row_bytes) v[e / 4] |= static_cast<uint32_t>(p[e]) << (8 * (e % 4));
+      }
+    }
+    *reinterpret_cast<u32x4w*>(static_cast<uint8_t*>(c.to) + r * c.pitch + at) = v;
+  } else {
+    if (r >= c.rows || at >= c.row_bytes) return;
+    const u32x4w v = *reinterpret_cast<const u32x4w*>(static_cast<const uint8_t*>(c.from) + r * c.pitch + at);
+    uint8_t* q = static_cast<uint8_t*>(c.to) + r * c.row_bytes + at;
+    if (at + 16 <= c.row_bytes) {
+      *reinterpret_cast<u32x4w_any*>(q) = v;
     } else {
 #pragma unroll
-      for (unsigned e = 0; e < 8; ++e)
-        if (c + e < cols) v[e / 2] |= static_cast<uint32_t>(p[e]) << (16 * (e % 2));
+      for (unsigned e = 0; e < 16; e += 2)       // two-byte elements
+        if (at + e < c.row_bytes) *reinterpret_cast<uint16_t*>(q + e) = static_cast<uint16_t>(v[e / 4] >> (8 * (e % 4)));
     }
   }
-  *reinterpret_cast<u32x4w*>(dst + r * cols_to + c) = v;
 }
 
-// The way back for the result: rows x cols elements out of a matrix whose rows are cols_from elements apart.
-__global__ void __launch_bounds__(256) lego_unpad2d_kernel(const uint16_t* __restrict__ src, uint16_t* __restrict__ dst,
-                                                           unsigned rows, unsigned cols, unsigned cols_from)
-{
-  const unsigned per_row = (cols + 7) / 8;
-  const size_t chunk = static_cast<size_t>(blockIdx.x) * 256 + threadIdx.x;
-  const size_t r = chunk / per_row;
-  const unsigned c = static_cast<unsigned>(chunk % per_row) * 8;
-  if (r >= rows) return;
-  const u32x4w v = *reinterpret_cast<const u32x4w*>(src + r * cols_from + c);
-  uint16_t* q = dst + r * cols + c;
-  if (c + 8 <= cols) {
-    *reinterpret_cast<u32x4w_any*>(q) = v;
-  } else {
-#pragma unroll
-    for (unsigned e = 0; e < 8; ++e)
-      if (c + e < cols) q[e] = static_cast<uint16_t>(v[e / 2] >> (16 * (e % 2)));
+// Collects copies of matrices that lie one after the other in a workspace and enqueues them, kCopies at a time.
+class Copier {
+ public:
+  Copier(bool pad, hipStream_t stream) : pad_(pad), stream_(stream) { copies_.count = 0; }
+  // rows x cols elements of `bytes` bytes each, copied to (pad) or from (otherwise) rows of cols_to elements
+  void add(const void* from, void* to, long rows, long cols, long rows_to, long cols_to, int bytes)
+  {
+    if (copies_.count == kCopies) (void)flush();      // its error is kept
+    const unsigned long long chunks = static_cast<unsigned long long>(pad_ ? rows_to : rows) * (cols_to * bytes / 16);
+    const unsigned before = copies_.count ? copies_.of[copies_.count - 1].end : 0u;
+    copies_.of[copies_.count++] = {from, to, static_cast<unsigned>(rows), static_cast<unsigned>(cols * bytes), static_cast<unsigned>(rows_to),
+                                   static_cast<unsigned>(cols_to * bytes), before + static_cast<unsigned>((chunks + 255) / 256)};
   }
-}
+  hipError_t flush()
+  {
+    if (copies_.count == 0) return err_;
+    const dim3 grid(copies_.of[copies_.count - 1].end);
+    if (pad_) hipLaunchKernelGGL(lego_copies_kernel<true>, grid, dim3(256), 0, stream_, copies_);
+    else hipLaunchKernelGGL(lego_copies_kernel<false>, grid, dim3(256), 0, stream_, copies_);
+    copies_.count = 0;
+    const hipError_t e = hipGetLastError();
+    if (err_ == hipSuccess) err_ = e;
+    return err_;
+  }
 
-hipError_t pad2d(const void* src, void* dst, int rows, int cols, int rows_to, int cols_to, hipStream_t stream)
-{
-  const size_t chunks = static_cast<size_t>(rows_to) * (cols_to / 8);
-  hipLaunchKernelGGL(lego_pad2d_kernel, dim3(static_cast<unsigned>((chunks + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), static_cast<unsigned>(rows),
-                     static_cast<unsigned>(cols), static_cast<unsigned>(rows_to), static_cast<unsigned>(cols_to));
-  return hipGetLastError();
-}
-
-hipError_t unpad2d(const void* src, void* dst, int rows, int cols, int cols_from, hipStream_t stream)
-{
-  const size_t chunks = static_cast<size_t>(rows) * ((cols + 7) / 8);
-  hipLaunchKernelGGL(lego_unpad2d_kernel, dim3(static_cast<unsigned>((chunks + 255) / 256)), dim3(256), 0, stream,
-                     static_cast<const uint16_t*>(src), static_cast<uint16_t*>(dst), static_cast<unsigned>(rows),
-                     static_cast<unsigned>(cols), static_cast<unsigned>(cols_from));
-  return hipGetLastError();
-}
+ private:
+  bool pad_;
+  hipStream_t stream_;
+  Copies copies_;
+  hipError_t err_ = hipSuccess;
+};
 
 // Scratch of lego_hip_layernorm_bwd_f16_noalloc: the fp32 dw/db partial rows that the other
 // LayerNorm backward entry points take from the caller.  One copy per device, held until the process
@@ -729,6 +752,53 @@ typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int,
 #define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_splitk_launch, lego_gemm_##DT##_nt_t128x128_splitk_launch, \
                          lego_gemm_##DT##_tn_t128x128_splitk_launch, lego_gemm_##DT##_tt_t128x128_splitk_launch}
 
+// Operand rows that are not whole 16-byte chunks: the tiled kernels run on zero-padded copies (every side a multiple of `chunk`
+// elements; the padding adds zeros to the sums) and the result is copied back: two more launches and three more passes over
+// the matrices, against the kernel that moves one element per access and whose chain of k-tiles is long.  8-bit operands, us by
+// elements / on copies: 320 x 1984 x 7959 829 / 35, 2000 x 2000 x 2001 276 / 27, 5000 x 3001 x 136 93 / 32, 6902 x 192 x 296 31 / 28, 1000 x
+// 1000 x 264 27 / 25, 33 x 100 x 200 16 / 23, 1000 x 1000 x 136 16 / 22: copies from K = 256 on, or from as many 64 x 64 tiles of the
+// result as keep the one-element kernel busy for 30 us.
+inline bool copies_gain_8bit(int M, int N, int K)
+{
+  const double tiles = static_cast<double>((M + 63) / 64) * ((N + 63) / 64);
+  return K >= 256 || tiles * K >= 150000.0;
+}
+inline int round_up(int v, int to) { return (v + to - 1) / to * to; }
+inline unsigned long long padded_bytes(int M, int N, int K, int chunk, int bytes)
+{
+  const unsigned long long m = round_up(M, chunk), n = round_up(N, chunk), k = round_up(K, chunk);
+  return bytes * (m * k + k * n) + 2ull * m * n;
+}
+inline unsigned long long parts_bytes(int M, int N, int parts)
+{
+  const unsigned long long tiles = static_cast<unsigned long long>((M + 127) / 128) * ((N + 127) / 128);
+  return parts > 1 ? parts * tiles * 128ull * 128ull * sizeof(float) : 0ull;
+}
+
+// `product(a, b, c, M, N, K, sums)` on padded copies in the workspace, whose part for sums follows them.
+extern "C++" template <class Product>
+int on_padded_copies(int chunk, int bytes, const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
+                     void* workspace, void* stream, const Product& product)
+{
+  const int Mr = round_up(M, chunk), Nr = round_up(N, chunk), Kr = round_up(K, chunk);
+  const int Mp = trans_a ? Mr : M;                 // rows of the padded product: a transposed A has rows of M elements
+  uint8_t* ap = static_cast<uint8_t*>(workspace);
+  uint8_t* bp = ap + static_cast<size_t>(Mr) * Kr * bytes;
+  uint8_t* cp = bp + static_cast<size_t>(Kr) * Nr * bytes;
+  void* sums = cp + static_cast<size_t>(Mr) * Nr * 2;
+  const bool copy_a = Kr != K || Mp != M || !usable(a), copy_b = Kr != K || Nr != N || !usable(b), copy_c = Nr != N || Mp != M || !usable(c);
+  Copier pads(true, as_stream(stream));
+  if (copy_a) trans_a ? pads.add(a, ap, K, M, Kr, Mr, bytes) : pads.add(a, ap, M, K, M, Kr, bytes);
+  if (copy_b) trans_b ? pads.add(b, bp, N, K, Nr, Kr, bytes) : pads.add(b, bp, K, N, Kr, Nr, bytes);
+  const hipError_t err = pads.flush();
+  if (err != hipSuccess) return ok_or(err);
+  const int rc = product(copy_a ? ap : a, copy_b ? bp : b, copy_c ? cp : c, Mp, Nr, Kr, sums);
+  if (rc != 0 || !copy_c) return rc;
+  Copier back(false, as_stream(stream));
+  back.add(cp, c, M, N, M, Nr, 2);
+  return ok_or(back.flush());
+}
+
 // 8-bit operands: both tile sizes in all four layouts, one MFMA shape.  The rule between the tiles is that of the 16-bit
 // operands; us on big / small tiles, e5m2 A*B: 512 x 512 x 2048 19.5 / 8.6, 1000 x 2048 x 2048 22.1 / 13.6 (32 and 128
 // workgroups), 2048^3 22.0 / 14.1, 2048 x 4096 x 4096 39.4 / 31.0, 4352 x 4096 x 4096 78.4 / 73.7, 4608^3 88.3 / 84.6.
@@ -771,17 +841,14 @@ int lego_hip_gemm_bf16_f16_ex(const void* a, const void* b, void* c, int M, int 
 int lego_hip_gemm_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
-  // N or K not a multiple of 8: room for zero-padded copies of both operands and of the result (2-byte elements).
+  // N or K not a multiple of 8: room for zero-padded copies of both operands and of the result.
   // (M only matters as the row length of a transposed A; that case alone stays with the one-element kernel.)
   unsigned long long copies = 0;
   if (N % 8 || K % 8) {
-    const unsigned long long m8 = (M + 7ull) / 8 * 8, n8 = (N + 7ull) / 8 * 8, k8 = (K + 7ull) / 8 * 8;
-    copies = 2ull * (m8 * k8 + k8 * n8 + m8 * n8);
-    M = static_cast<int>(m8); N = static_cast<int>(n8); K = static_cast<int>(k8);     // the product that then runs
+    copies = padded_bytes(M, N, K, 8, 2);
+    M = round_up(M, 8); N = round_up(N, 8); K = round_up(K, 8);     // the product that then runs
   }
-  const int parts = splitk_parts(M, N, K, LEGO_GEMM_BK);
-  const unsigned long long tiles = static_cast<unsigned long long>((M + 127) / 128) * ((N + 127) / 128);
-  *bytes = copies + (parts > 1 ? parts * tiles * 128ull * 128ull * sizeof(float) : 0ull);
+  *bytes = copies + parts_bytes(M, N, splitk_parts(M, N, K, LEGO_GEMM_BK));
   return 0;
 }
 
@@ -790,63 +857,30 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
 {
   static const splitk_launcher f16[4] = LEGO_SPLITK(f16), bf16[4] = LEGO_SPLITK(bf16), bf16h[4] = LEGO_SPLITK(bf16h);
   if (element != 0 && element != 1 && element != 4) return kInvalid;
+  const splitk_launcher parts_by_layout = (element == 0 ? f16 : element == 1 ? bf16 : bf16h)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)];
+  const auto whole = [&](const void* aa, const void* bb, void* cc, int m, int n, int k) {
+    switch (element) {
+      case 0: return lego_hip_gemm_f16_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, stream);
+      case 1: return lego_hip_gemm_bf16_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, stream);
+      default: return lego_hip_gemm_bf16_f16_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, stream);
+    }
+  };
   unsigned long long need = 0;
   if (lego_hip_gemm_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
-  // what the tiled kernels ask of shapes and bases (gemm_ex): anything else, and every product that gains nothing
-  // from parts, takes the plain entry point
+  if (need == 0 || workspace_bytes < need || !usable(workspace)) return whole(a, b, c, M, N, K);
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 8 == 0 && (trans_a ? M % 8 == 0 : K % 8 == 0) &&
                      (!trans_b || K % 8 == 0);
-  const bool have_workspace = need != 0 && workspace != nullptr && workspace_bytes >= need && usable(workspace);
-  if (have_workspace && (N % 8 || K % 8)) {
-    // Operand rows that are not whole 16-byte chunks: the tiled kernels run on zero-padded copies (every side a
-    // multiple of 8; the padding adds zeros to the sums) and the result is copied back.  Three more passes over
-    // the matrices, against the tenfold cost of the kernel that moves one element per access.
-    if (a == nullptr || b == nullptr || c == nullptr || (activation != 0 && activation != 1)) return kInvalid;
-    if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
-    const int M8 = (M + 7) / 8 * 8, N8 = (N + 7) / 8 * 8, K8 = (K + 7) / 8 * 8;
-    const int Mp = trans_a ? M8 : M;                 // rows of the padded product: a transposed A has rows of M elements
-    uint16_t* ap = static_cast<uint16_t*>(workspace);
-    uint16_t* bp = ap + static_cast<size_t>(M8) * K8;
-    uint16_t* cp = bp + static_cast<size_t>(K8) * N8;
-    const bool copy_a = K8 != K || (trans_a && M8 != M) || !usable(a);
-    const bool copy_b = K8 != K || N8 != N || !usable(b);
-    const bool copy_c = N8 != N || Mp != M || !usable(c);
-    hipError_t err = hipSuccess;
-    if (copy_a) err = trans_a ? pad2d(a, ap, K, M, K8, M8, as_stream(stream)) : pad2d(a, ap, M, K, M, K8, as_stream(stream));
-    if (err != hipSuccess) return ok_or(err);
-    if (copy_b) err = trans_b ? pad2d(b, bp, N, K, N8, K8, as_stream(stream)) : pad2d(b, bp, K, N, K8, N8, as_stream(stream));
-    if (err != hipSuccess) return ok_or(err);
-    const void* aa = copy_a ? ap : a;
-    const void* bb = copy_b ? bp : b;
-    void* cc = copy_c ? cp : c;
-    int rc;
-    const int parts = splitk_parts(Mp, N8, K8, LEGO_GEMM_BK);
-    if (parts > 1) {      // few tiles: parts along K, their sums behind the copies (the size asked for covers M8 rows)
-      const splitk_launcher* by_layout = element == 0 ? f16 : element == 1 ? bf16 : bf16h;
-      rc = ok_or(by_layout[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](aa, bb, cc, Mp, N8, K8, activation, parts,
-                                                                 reinterpret_cast<float*>(cp + static_cast<size_t>(M8) * N8),
-                                                                 as_stream(stream)));
-    } else {
-      switch (element) {
-        case 0: rc = lego_hip_gemm_f16_ex(aa, bb, cc, Mp, N8, K8, trans_a, trans_b, activation, stream); break;
-        case 1: rc = lego_hip_gemm_bf16_ex(aa, bb, cc, Mp, N8, K8, trans_a, trans_b, activation, stream); break;
-        default: rc = lego_hip_gemm_bf16_f16_ex(aa, bb, cc, Mp, N8, K8, trans_a, trans_b, activation, stream); break;
-      }
-    }
-    if (rc != 0 || !copy_c) return rc;
-    return ok_or(unpad2d(cp, c, M, N, N8, as_stream(stream)));
-  }
-  if (!have_workspace || !tiled) {
-    switch (element) {
-      case 0: return lego_hip_gemm_f16_ex(a, b, c, M, N, K, trans_a, trans_b, activation, stream);
-      case 1: return lego_hip_gemm_bf16_ex(a, b, c, M, N, K, trans_a, trans_b, activation, stream);
-      default: return lego_hip_gemm_bf16_f16_ex(a, b, c, M, N, K, trans_a, trans_b, activation, stream);
-    }
-  }
+  const bool copies = N % 8 || K % 8;      // and room for them
+  if (!tiled && !copies) return whole(a, b, c, M, N, K);
   if (a == nullptr || b == nullptr || c == nullptr || (activation != 0 && activation != 1)) return kInvalid;
-  const splitk_launcher* by_layout = element == 0 ? f16 : element == 1 ? bf16 : bf16h;
-  return ok_or(by_layout[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](a, b, c, M, N, K, activation, splitk_parts(M, N, K, LEGO_GEMM_BK),
-                                                             static_cast<float*>(workspace), as_stream(stream)));
+  if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
+  const auto product = [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
+    const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK);
+    if (parts < 2) return whole(aa, bb, cc, m, n, k);
+    return ok_or(parts_by_layout(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
+  };
+  if (tiled) return product(a, b, c, M, N, K, workspace);
+  return on_padded_copies(8, 2, a, b, c, M, N, K, trans_a, trans_b, workspace, stream, product);
 }
 
 int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
@@ -863,16 +897,21 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
-  const int parts = N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT);
-  const unsigned long long tiles = static_cast<unsigned long long>((M + 127) / 128) * ((N + 127) / 128);
-  *bytes = parts > 1 ? parts * tiles * 128ull * 128ull * sizeof(float) : 0ull;
+  *bytes = parts_bytes(M, N, N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT));
   return 0;
 }
+
+namespace {
+const splitk_launcher* fp8_parts(int format)
+{
+  static const splitk_launcher e4m3[4] = LEGO_SPLITK(e4m3), e5m2[4] = LEGO_SPLITK(e5m2);
+  return format == 0 ? e4m3 : e5m2;
+}
+}  // namespace
 
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream)
 {
-  static const splitk_launcher e4m3[4] = LEGO_SPLITK(e4m3), e5m2[4] = LEGO_SPLITK(e5m2);
   unsigned long long need = 0;
   if ((format != 0 && format != 1) || lego_hip_gemm_fp8_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) &&
@@ -881,8 +920,39 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
-  return ok_or((format == 0 ? e4m3 : e5m2)[layout](a, b, c, M, N, K, activation, splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT),
-                                                   static_cast<float*>(workspace), as_stream(stream)));
+  return ok_or(fp8_parts(format)[layout](a, b, c, M, N, K, activation, splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT),
+                                         static_cast<float*>(workspace), as_stream(stream)));
+}
+
+// Whether a product whose rows are not whole 16-byte chunks gains from copies that are; room for these and for the sums of their product.
+int lego_hip_gemm_fp8_padded_bytes(int M, int N, int K, int trans_a, int trans_b, unsigned long long* bytes)
+{
+  if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
+  const bool tiled = N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) && (!trans_b || K % 16 == 0);
+  if (tiled || !copies_gain_8bit(M, N, K)) { *bytes = 0; return 0; }
+  const int Mp = trans_a ? round_up(M, 16) : M, Nr = round_up(N, 16), Kr = round_up(K, 16);
+  *bytes = padded_bytes(M, N, K, 16, 1) + parts_bytes(Mp, Nr, splitk_parts(Mp, Nr, Kr, LEGO_GEMM_BK_8BIT));
+  return 0;
+}
+
+int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
+                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream)
+{
+  unsigned long long need = 0;
+  if ((format != 0 && format != 1) || lego_hip_gemm_fp8_padded_bytes(M, N, K, trans_a, trans_b, &need) != 0) return kInvalid;
+  const auto whole = [&](const void* aa, const void* bb, void* cc, int m, int n, int k) {
+    return lego_hip_gemm_fp8_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, format, stream);
+  };
+  if (need == 0 || !usable(workspace) || workspace_bytes < need) return whole(a, b, c, M, N, K);
+  if (a == nullptr || b == nullptr || c == nullptr || (activation != 0 && activation != 1)) return kInvalid;
+  if (reinterpret_cast<uintptr_t>(c) & 1u) return kInvalid;
+  return on_padded_copies(16, 1, a, b, c, M, N, K, trans_a, trans_b, workspace, stream,
+                          [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
+    const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK_8BIT);
+    if (parts < 2) return whole(aa, bb, cc, m, n, k);
+    return ok_or(fp8_parts(format)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums),
+                                                                         as_stream(stream)));
+  });
 }
 
 int lego_hip_gemm_f16_variant(const void* a, const void* b, void* c, int M, int N, int K, int variant, void* stream)
@@ -1194,6 +1264,55 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
   if (plan.kind == 1) return ok_or(lego_grouped_gemm_f16_t128x128_launch(a, b, c, sizes3, groups, as_stream(stream)));
   if (plan.split == 0) return ok_or(lego_grouped_gemm_f16_launch(a, b, c, sizes3, groups, as_stream(stream)));
   return ok_or(lego_grouped_gemm_f16_split_launch(a, b, c, sizes3, groups, plan.split, as_stream(stream)));
+}
+
+// Room for zero-padded copies of the problems whose N or K is no multiple of 8.
+int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes)
+{
+  if (sizes3 == nullptr || bytes == nullptr || groups <= 0 || groups > kGroupedMaxProblems) return kInvalid;
+  unsigned long long total = 0;
+  for (int g = 0; g < groups; ++g) {
+    const int m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
+    if (m <= 0 || n <= 0 || k <= 0) return kInvalid;
+    if (n % 8 || k % 8) total += padded_bytes(m, n, k, 8, 2);
+  }
+  *bytes = total;
+  return 0;
+}
+
+int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
+                                 void* workspace, unsigned long long workspace_bytes, void* stream) try
+{
+  const int checked = grouped_check(a, b, c, sizes3, groups);
+  unsigned long long need = 0;
+  if (checked != 2 || lego_hip_grouped_gemm_f16_workspace_bytes(sizes3, groups, &need) != 0 || need == 0 || workspace_bytes < need || !usable(workspace))
+    return lego_hip_grouped_gemm_f16(a, b, c, sizes3, groups, stream);
+  std::vector<const void*> aa(a, a + groups), bb(b, b + groups);
+  std::vector<void*> cc(c, c + groups);
+  std::vector<int> sizes(sizes3, sizes3 + 3 * static_cast<size_t>(groups));
+  Copier pads(true, as_stream(stream)), back(false, as_stream(stream));
+  uint8_t* at = static_cast<uint8_t*>(workspace);
+  std::vector<int> copied;
+  for (int g = 0; g < groups; ++g) {
+    const int m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
+    if (n % 8 == 0 && k % 8 == 0) continue;
+    const int mr = round_up(m, 8), nr = round_up(n, 8), kr = round_up(k, 8);
+    uint8_t *ap = at, *bp = ap + 2 * static_cast<size_t>(mr) * kr, *cp = bp + 2 * static_cast<size_t>(kr) * nr;
+    at = cp + 2 * static_cast<size_t>(mr) * nr;
+    if (kr != k || !usable(a[g])) { pads.add(a[g], ap, m, k, m, kr, 2); aa[g] = ap; }
+    if (kr != k || nr != n || !usable(b[g])) { pads.add(b[g], bp, k, n, kr, nr, 2); bb[g] = bp; }
+    if (nr != n || !usable(c[g])) { cc[g] = cp; copied.push_back(g); }
+    sizes[3 * g + 1] = nr;
+    sizes[3 * g + 2] = kr;
+  }
+  const hipError_t err = pads.flush();
+  if (err != hipSuccess) return ok_or(err);
+  const int rc = lego_hip_grouped_gemm_f16(aa.data(), bb.data(), cc.data(), sizes.data(), groups, stream);
+  if (rc != 0) return rc;
+  for (const int g : copied) back.add(cc[g], c[g], sizes3[3 * g], sizes3[3 * g + 1], sizes3[3 * g], sizes[3 * g + 1], 2);
+  return ok_or(back.flush());
+} catch (const std::bad_alloc&) {
+  return ok_or(hipErrorOutOfMemory);
 }
 
 int lego_hip_rows_f16_plan(int M, int N, int* waves_per_row)

@@ -191,7 +191,7 @@ def _operand(t, name):
     raise ValueError(f"{name} must be contiguous or the transpose of a contiguous tensor")
 
 
-_gemm_workspace, _fp8_workspace = {}, {}      # (M, N, K) -> bytes of workspace that the product uses
+_gemm_workspace, _fp8_workspace, _fp8_padded = {}, {}, {}      # (M, N, K, ...) -> bytes of workspace that the product uses
 
 
 def _ask_workspace(entry, known, shape):
@@ -221,13 +221,20 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
         raise ValueError("a and b must have the same dtype")
     if a.dtype in _FP8_FORMAT:
         c = torch.empty((M, N), device=a.device, dtype=torch.float16)
-        need = _fp8_workspace.get((M, N, K))
-        if need is None:
-            need = _ask_workspace("lego_hip_gemm_fp8_workspace_bytes", _fp8_workspace, (M, N, K))
-        # the size is for any layout: one whose rows are not whole 16-byte chunks runs without
-        if need and (M if ta else K) % 16 == 0 and not (tb and K % 16):
-            workspace = torch.empty(need // 4, dtype=torch.float32, device=a.device)
-            runtime.call("lego_hip_gemm_fp8_ex_ws", _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
+        if N % 16 or (M if ta else K) % 16 or (tb and K % 16):
+            # rows that are not whole 16-byte chunks: zero-padded copies where they gain
+            need = _fp8_padded.get((M, N, K, ta, tb))
+            if need is None:
+                need = _ask_workspace("lego_hip_gemm_fp8_padded_bytes", _fp8_padded, (M, N, K, ta, tb))
+            entry = "lego_hip_gemm_fp8_padded"
+        else:
+            need = _fp8_workspace.get((M, N, K))
+            if need is None:
+                need = _ask_workspace("lego_hip_gemm_fp8_workspace_bytes", _fp8_workspace, (M, N, K))
+            entry = "lego_hip_gemm_fp8_ex_ws"
+        if need:
+            workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
+            runtime.call(entry, _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
                          1 if activation else 0, _FP8_FORMAT[a.dtype], _ptr(workspace), need, _stream())
             return c
         runtime.call("lego_hip_gemm_fp8_ex", _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
@@ -236,9 +243,10 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     if out_dtype not in (torch.float16, a.dtype):
         raise ValueError("out_dtype must be float16 or the operands' type")
     entry = "lego_hip_gemm_bf16_f16_ex" if (a.dtype, out_dtype) == (torch.bfloat16, torch.float16) else _GEMM_ENTRY[a.dtype]
-    if ta and M % 8 and M * K >= 65536:
+    if ta and M % 8 and (M * K >= 65536 or K >= 384):
         # a column-major A whose columns (M elements) are not whole 16-byte chunks is outside the tiled kernels whatever
-        # the workspace: store it row-major first (one pass with the transpose kernels)
+        # the workspace: store it row-major first (one pass with the transpose kernels; by elements / row-major first:
+        # 33 x 256 x 256 13 / 15 us, 7 x 512 x 512 22 / 16, 3 x 1024 x 8192 323 / 19)
         a_store, ta = transpose(a_store), 0
     c = torch.empty((M, N), device=a.device, dtype=out_dtype)
     # products of few tiles (a skinny operand, a long K) are split along K when there is room for the partial sums;
@@ -265,24 +273,24 @@ def lego_group_gemm_fn(group_A, group_B):
         _check(b, torch.float16, "B")
         if a.shape[1] != b.shape[0]:
             raise ValueError("Incompatible dimensions")
-    # Problems whose rows are not whole 16-byte chunks would take the whole call to one launch per problem with the
-    # one-element kernel: those few go through ``matmul`` (zero-padded copies, a workspace from torch), the rest in
-    # one launch.
-    odd = [i for i, b in enumerate(group_B) if b.shape[0] % 8 or b.shape[1] % 8]
-    if odd:
-        rest = [i for i in range(len(group_A)) if i not in set(odd)]
+    # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace.  Those that a single product
+    # splits along K (32 k-tiles of 64 and more) would be one long workgroup after another's end: they go through `matmul`.
+    deep = [i for i, b in enumerate(group_B) if b.shape[0] > 31 * 64 and (b.shape[0] % 8 or b.shape[1] % 8)]
+    if deep:
+        rest = [i for i in range(len(group_A)) if i not in set(deep)]
         out = [None] * len(group_A)
         if rest:
             for i, c in zip(rest, lego_group_gemm_fn([group_A[i] for i in rest], [group_B[i] for i in rest])):
                 out[i] = c
-        for i in odd:
+        for i in deep:
             out[i] = matmul(group_A[i], group_B[i])
         return out
     groups = len(group_A)
-    group_C, sizes = [], []
+    group_C, sizes, padded = [], [], False
     for a, b in zip(group_A, group_B):
         M, K = a.shape
         N = b.shape[1]
+        padded = padded or N % 8 != 0 or K % 8 != 0
         group_C.append(torch.empty((M, N), device=a.device, dtype=a.dtype))
         sizes += [M, N, K]
     arr = ctypes.c_void_p * groups
@@ -290,6 +298,12 @@ def lego_group_gemm_fn(group_A, group_B):
     pb = arr(*[t.data_ptr() for t in group_B])
     pc = arr(*[t.data_ptr() for t in group_C])
     sz = (ctypes.c_int * (3 * groups))(*sizes)
+    if padded:
+        size = ctypes.c_ulonglong(0)
+        runtime.call("lego_hip_grouped_gemm_f16_workspace_bytes", sz, groups, ctypes.byref(size))
+        workspace = torch.empty(size.value // 2, dtype=torch.float16, device=group_C[0].device)
+        runtime.call("lego_hip_grouped_gemm_f16_ws", pa, pb, pc, sz, groups, _ptr(workspace), size.value, _stream())
+        return group_C
     runtime.call("lego_hip_grouped_gemm_f16", pa, pb, pc, sz, groups, _stream())
     return group_C
 

@@ -49,6 +49,8 @@ SIGNATURES = {
     "lego_hip_gemm_fp8_workspace_bytes": [_c_int, _c_int, _c_int, ctypes.POINTER(ctypes.c_ulonglong)],
     "lego_hip_gemm_fp8_ex_ws": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                 _c_void_p, ctypes.c_ulonglong, _c_void_p],
+    "lego_hip_gemm_fp8_padded_bytes": [_c_int] * 5 + [ctypes.POINTER(ctypes.c_ulonglong)],
+    "lego_hip_gemm_fp8_padded": [_c_void_p] * 3 + [_c_int] * 7 + [_c_void_p, ctypes.c_ulonglong, _c_void_p],
     "lego_hip_gemm_fp8_ex": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                              _c_int, _c_void_p],
     "lego_hip_stencil_f3d_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
@@ -61,6 +63,8 @@ SIGNATURES = {
     "lego_hip_nw_i32_workspace_bytes": [_c_int, ctypes.POINTER(ctypes.c_ulonglong)],
     "lego_hip_nw_i32_ws": [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p, ctypes.c_ulonglong, _c_void_p],
     "lego_hip_grouped_gemm_f16": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_void_p],
+    "lego_hip_grouped_gemm_f16_workspace_bytes": [_INT_ARRAY, _c_int, ctypes.POINTER(ctypes.c_ulonglong)],
+    "lego_hip_grouped_gemm_f16_ws": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_void_p, ctypes.c_ulonglong, _c_void_p],
     "lego_hip_grouped_gemm_f16_plan": [_INT_ARRAY, _c_int, _INT_ARRAY],
     "lego_hip_grouped_gemm_f16_split": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_int, _c_void_p],
     "lego_hip_softmax_f16_wpr": [_c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],

@@ -1,0 +1,68 @@
+"""Products whose operand rows are not whole 16-byte chunks, on zero-padded copies: 8-bit ones, and grouped calls with such problems
+among others.  Small whole numbers: every sum is exact, whatever the workspace held."""
+import ctypes
+
+import pytest
+import torch
+
+
+def _size(entry, *args):
+    from lego_amd import runtime
+    need = ctypes.c_ulonglong(0)
+    runtime.call(entry, *args, ctypes.byref(need))
+    return need.value
+
+
+def test_padded_sizes_hold_the_copies():
+    for M, N, K, ta, tb in ((17, 65, 4000, 0, 0), (320, 1984, 7959, 0, 1), (33, 64, 512, 1, 0), (5000, 3001, 100, 0, 0)):
+        r = lambda v: (v + 15) // 16 * 16
+        need = _size("lego_hip_gemm_fp8_padded_bytes", M, N, K, ta, tb)
+        assert need >= r(M) * r(K) + r(K) * r(N) + 2 * r(M) * r(N) and need % 16 == 0
+    for M, N, K, ta, tb in ((33, 64, 512, 0, 0), (64, 64, 512, 1, 1), (32, 64, 4104, 1, 0), (100, 100, 100, 0, 0)):     # whole chunks, or too little work
+        assert _size("lego_hip_gemm_fp8_padded_bytes", M, N, K, ta, tb) == 0
+    sizes = (ctypes.c_int * 9)(64, 64, 64, 5, 9, 17, 100, 64, 63)
+    assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 3) == 2 * (8 * 24 + 24 * 16 + 8 * 16 + 104 * 64 + 64 * 64 + 104 * 64)
+    assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 1) == 0
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("fp8", [torch.float8_e5m2, torch.float8_e4m3fn])
+@pytest.mark.parametrize("M,N,K", [(1, 65, 257), (17, 64, 4097), (33, 100, 264), (128, 129, 256), (1000, 1001, 271), (2500, 3001, 72)])
+def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
+    from lego_amd import ops, runtime
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M, K), generator=g).float() * (torch.randint(0, 4, (M, K), generator=g) == 0)
+    b = torch.randint(-1, 2, (K, N), generator=g).float()
+    want = a @ b
+    assert want.abs().max() < 2048
+    for ta in (0, 1):
+        for tb in (0, 1):
+            print(f"8-bit on copies {fp8} {M}x{N}x{K} ta={ta} tb={tb}", flush=True)
+            a8 = a.to(fp8).t().contiguous().cuda() if ta else a.to(fp8).cuda()
+            b8 = b.to(fp8).t().contiguous().cuda() if tb else b.to(fp8).cuda()
+            assert torch.equal(ops.matmul(a8.t() if ta else a8, b8.t() if tb else b8).cpu().float(), want)
+            need = _size("lego_hip_gemm_fp8_padded_bytes", M, N, K, ta, tb)
+            if not need:
+                continue
+            # a workspace full of NaN, operands and result at any element, nothing written around the result
+            ws = torch.full((need,), 0x7f, dtype=torch.uint8, device="cuda")
+            ad, bd = (torch.cat([t.view(torch.uint8).new_zeros(3), t.view(torch.uint8).reshape(-1)])[3:] for t in (a8, b8))
+            c = torch.full((M * N + 64,), 7.0, dtype=torch.float16, device="cuda")
+            runtime.call("lego_hip_gemm_fp8_padded", ad.data_ptr(), bd.data_ptr(), c.data_ptr() + 2 * 29, M, N, K, ta, tb, 0,
+                         0 if fp8 == torch.float8_e4m3fn else 1, ws.data_ptr(), need, None)
+            assert torch.equal(c[29:29 + M * N].view(M, N).cpu().float(), want)
+            assert (c[:29] == 7).all() and (c[29 + M * N:] == 7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("problems", [[(1, 65, 64), (64, 64, 64), (33, 72, 63)], [(5, 9, 2111), (64, 64, 64), (130, 1, 1)],
+                                      [(16 + i, 63 + i, 65 + i) for i in range(70)]])
+def test_gpu_grouped_with_ragged_problems(problems):
+    """Problems of whole chunks and others, deep ones, and more than the launches of the copies and of the products carry."""
+    from lego_amd import ops
+    print(f"grouped, {len(problems)} problems", flush=True)
+    g = torch.Generator().manual_seed(len(problems))
+    a = [torch.randint(-2, 3, (m, k), generator=g).half() * (torch.rand(m, k, generator=g) < 200.0 / k).half() for m, _, k in problems]
+    b = [torch.randint(-2, 3, (k, n), generator=g).half() for _, n, k in problems]
+    for x, y, c in zip(a, b, ops.lego_group_gemm_fn([x.cuda() for x in a], [y.cuda() for y in b])):
+        assert torch.equal(c.cpu().double(), x.double() @ y.double())
