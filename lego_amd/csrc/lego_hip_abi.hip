@@ -298,12 +298,16 @@ __global__ void __launch_bounds__(256) lego_copies_kernel(const Copies copies)
     u32x4w v = {0u, 0u, 0u, 0u};
     if (r < c.rows && at < c.row_bytes) {
       const uint8_t* p = static_cast<const uint8_t*>(c.from) + r * c.row_bytes + at;
-      if (at + 16 <= c.row_bytes) {
+      const unsigned valid = c.row_bytes - at;
+      if ((c.rows - r) * c.row_bytes - at >= 16) {      // the matrix has sixteen bytes from here on, this row's or the next one's
         v = *reinterpret_cast<const u32x4w_any*>(p);
+#pragma unroll
+        for (unsigned e = 0; e < 4; ++e)
+          v[e] = valid >= 4 * e + 4 ? v[e] : valid > 4 * e ? v[e] & ((1u << (8 * (valid - 4 * e))) - 1u) : 0u;
       } else {
 #pragma unroll
         for (unsigned e = 0; e < 16; ++e)
-          if (at + e < c.row_bytes) v[e / 4] |= static_cast<uint32_t>(p[e]) << (8 * (e % 4));
+          if (e < valid) v[e / 4] |= static_cast<uint32_t>(p[e]) << (8 * (e % 4));
       }
     }
     *reinterpret_cast<u32x4w*>(static_cast<uint8_t*>(c.to) + r * c.pitch + at) = v;
@@ -700,6 +704,15 @@ inline int gemm_choice(int M, int N, bool has_small, bool has_sparse)
   return has_sparse && tiles < kSparseRoundBelow ? 2 : 0;
 }
 
+// Few rows against a k-major B: the kernel that reads B once, straight into registers.  Us, tiles / this, 16 rows of bf16: 1024 x 1024
+// 11.3 / 10.5, 2048 x 4096 16.0 / 12.2, 4096 x 4096 16.0 / 12.3, 6144 x 4096 22.0 / 14.2, 8192 x 8192 33.2 / 25.8, 16384 x 4096 33.2 / 31.6; 1024 x
+// 8192 16.0 / 16.8 and 64 x 8192 14.2 / 16.7, where a workgroup's K is long and there are few of them; of 32 rows, which read A
+// twice as often, 8192 x 8192 34.3 / 34.5.
+inline bool takes_rows(int M, int N, int K, int trans_a, int trans_b, int bytes)
+{
+  return M <= 16 && !trans_a && trans_b && N >= 1024 && (N <= 4096 || N >= 6144) && K <= 4l * N && static_cast<long>(K) * bytes * 32 < (1l << 31) && static_cast<long>(N) * K < (1l << 31);
+}
+
 int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, void* c, int M, int N, int K,
             int trans_a, int trans_b, int activation, void* stream, int bk = LEGO_GEMM_BK, int chunk = 8)
 {
@@ -720,6 +733,8 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
     return ok_or(lego_gemm_any_launch(a, b, c, M, N, K, trans_a ? 1 : 0, trans_b ? 1 : 0, activation, element,
                                       as_stream(stream)));
   }
+  if (takes_rows(M, N, K, trans_a, trans_b, element == 2 || element == 3 ? 1 : 2))
+    return ok_or(lego_gemm_rows_launch(a, b, c, M, N, K, activation, element, as_stream(stream)));
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
   const int choice = gemm_choice(M, N, k.small[layout] != nullptr, k.sparse[layout] != nullptr);
   const gemm_launcher* by_layout = choice == 1 ? k.small : choice == 2 ? k.sparse : k.big;
@@ -876,7 +891,7 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
   if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
   const auto product = [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK);
-    if (parts < 2) return whole(aa, bb, cc, m, n, k);
+    if (parts < 2 || takes_rows(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
     return ok_or(parts_by_layout(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
   };
   if (tiled) return product(a, b, c, M, N, K, workspace);
@@ -916,7 +931,7 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
   if ((format != 0 && format != 1) || lego_hip_gemm_fp8_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) &&
                      (!trans_b || K % 16 == 0);
-  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need)
+  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need || takes_rows(M, N, K, trans_a, trans_b, 1))
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
@@ -949,7 +964,7 @@ int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N
   return on_padded_copies(16, 1, a, b, c, M, N, K, trans_a, trans_b, workspace, stream,
                           [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK_8BIT);
-    if (parts < 2) return whole(aa, bb, cc, m, n, k);
+    if (parts < 2 || takes_rows(m, n, k, trans_a, trans_b, 1)) return whole(aa, bb, cc, m, n, k);
     return ok_or(fp8_parts(format)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums),
                                                                          as_stream(stream)));
   });

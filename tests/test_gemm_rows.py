@@ -1,0 +1,42 @@
+"""Products of up to sixteen rows against a transposed B, which a kernel of their own takes: every element type, ragged columns, a last
+line of k that is not whole, fewer lines than wavefronts.  Small whole numbers: sums are exact in any order."""
+import pytest
+import torch
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,out", [(torch.float16, torch.float16), (torch.bfloat16, torch.bfloat16), (torch.bfloat16, torch.float16),
+                                       (torch.float8_e4m3fn, torch.float16), (torch.float8_e5m2, torch.float16)])
+@pytest.mark.parametrize("M,N,K", [(1, 1024, 16), (16, 1024, 64), (3, 1040, 528), (16, 1032, 4096), (7, 4096, 1040), (15, 6160, 272), (16, 6176, 2064)])
+def test_gpu_few_rows_against_a_transposed_matrix(dtype, out, M, N, K):
+    from lego_amd import ops
+    print(f"gemm rows {dtype} {M}x{N}x{K}", flush=True)
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M, K), generator=g).float() * (torch.rand(M, K, generator=g) < 100.0 / K)
+    b = torch.randint(-1, 2, (K, N), generator=g).float()
+    want = a @ b
+    assert want.abs().max() <= 256
+    bd = b.t().contiguous().to(dtype).cuda().t()
+    got = ops.matmul(a.to(dtype).cuda(), bd, out_dtype=out)
+    assert got.dtype == out and torch.equal(got.cpu().float(), want)
+    leaky = torch.where(want >= 0, want, 0.01 * want)
+    got = ops.matmul(a.to(dtype).cuda(), bd, activation="leaky_relu", out_dtype=out).cpu().float()
+    assert (got - leaky).abs().max() <= 256 * 0.01 * 2.0 ** (-8 if out == torch.bfloat16 else -11)
+
+
+@pytest.mark.gpu
+def test_gpu_row_past_the_matrix_reaches_nothing():
+    """Infinities around the operands (the same storage, before and after) stay out of every sum; nothing is written past C."""
+    import ctypes
+    from lego_amd import runtime
+    print("gemm rows, infinities around the operands", flush=True)
+    M, N, K = 5, 1032, 72
+    def inside(t):
+        buf = torch.full((t.numel() + 256,), float("inf"), dtype=torch.float16, device="cuda")
+        buf[128:128 + t.numel()] = t.reshape(-1).cuda()
+        return buf, buf.data_ptr() + 256
+    a, b = torch.ones(M, K).half(), torch.ones(N, K).half()
+    (ab, ap), (bb, bp) = inside(a), inside(b)
+    c = torch.full((M * N + 256,), 7.0, dtype=torch.float16, device="cuda")
+    runtime.call("lego_hip_gemm_f16_ex", ap, bp, c.data_ptr() + 256, M, N, K, 0, 1, 0, None)
+    assert (c[128:128 + M * N] == K).all() and (c[:128] == 7).all() and (c[128 + M * N:] == 7).all()
