@@ -3,9 +3,9 @@
 // The kernels of a training step over a short sequence take some 14 us; a node written in Python takes 120 us around them: its
 // bookkeeping, and a backward pass that waits for the interpreter on the engine's own thread.  This one asks for the same
 // tensors, saves the same ones and enqueues the same kernels on the current stream (a forward and backward over 512 x 768
-// bf16 elements 120 -> 69 us, over 4096 x 8192 fp16 ones 120 -> 68, what its kernels take).  It takes what needs nothing else: plain GPU tensors in the layouts that the kernels take, with
-// no dispatch mode, tracer or transform in between.  `apply` returns None for everything else, errors included, and the caller
-// goes through the node in Python.
+// bf16 elements 120 -> 69 us, over 4096 x 8192 fp16 ones 120 -> 68, what its kernels take).  It takes what needs nothing
+// else: plain GPU tensors in the layouts that the kernels take, with no dispatch mode, tracer or transform in between.
+// `apply` returns None for everything else, errors included, and the caller goes through the node in Python.
 #include <ATen/hip/impl/HIPStreamMasqueradingAsCUDA.h>
 #include <torch/csrc/autograd/python_variable.h>
 #include <torch/extension.h>

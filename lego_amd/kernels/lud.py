@@ -12,10 +12,9 @@ Here a block is 64 x 64, ``T = 16`` and ``R = 4`` (256 lanes per trailing block)
 inverse places the lanes that stage the two panels in LDS, and the offsets of a block's elements
 in the ``n x n`` matrix are those of ``OrderBy(Row(n, n)).TileBy([n/64, n/64], [64, 64])``.  The
 product itself runs on the fp32 matrix cores, whose accumulator layout is one more LEGO
-expression (``Row(4, 2, 4)``).  The diagonal block is eliminated by four wavefronts, sixteen columns each,
-row ``t`` in lane ``t``'s registers; a panel block is solved by four wavefronts, sixteen columns (row
-panel) or rows (column panel) each, in 16 x 16 tiles: products of tiles on the matrix cores, substitution
-inside a diagonal tile.
+expression (``Row(4, 2, 4)``).  Block steps go in pairs: one launch solves the panels of both against a factored 128 x 128
+diagonal block, the next one updates the trailing blocks while its first workgroup factors the diagonal block of the next
+pair, in 16 x 16 tiles.
 """
 from __future__ import annotations
 
