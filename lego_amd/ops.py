@@ -273,9 +273,10 @@ def lego_group_gemm_fn(group_A, group_B):
         _check(b, torch.float16, "B")
         if a.shape[1] != b.shape[0]:
             raise ValueError("Incompatible dimensions")
-    # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace.  Those that a single product
-    # splits along K (32 k-tiles of 64 and more) would be one long workgroup after another's end: they go through `matmul`.
-    deep = [i for i, b in enumerate(group_B) if b.shape[0] > 31 * 64 and (b.shape[0] % 8 or b.shape[1] % 8)]
+    # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace.  In a call of two or three, those that a
+    # single product splits along K (32 k-tiles of 64 and more) go through `matmul`: little else runs beside their chains (two
+    # problems, one 688 x 640 x 2577: 36 us, in the grouped launch 44; eleven with three such 107 us, in the launch 68).
+    deep = [i for i, b in enumerate(group_B) if b.shape[0] > 31 * 64 and (b.shape[0] % 8 or b.shape[1] % 8)] if len(group_B) <= 3 else []
     if deep:
         rest = [i for i in range(len(group_A)) if i not in set(deep)]
         out = [None] * len(group_A)

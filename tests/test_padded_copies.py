@@ -56,6 +56,7 @@ def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("problems", [[(1, 65, 64), (64, 64, 64), (33, 72, 63)], [(5, 9, 2111), (64, 64, 64), (130, 1, 1)],
+                                      [(9, 31, 2050), (64, 64, 64), (33, 72, 63), (3, 8, 8)],
                                       [(16 + i, 63 + i, 65 + i) for i in range(70)]])
 def test_gpu_grouped_with_ragged_problems(problems):
     """Problems of whole chunks and others, deep ones, and more than the launches of the copies and of the products carry."""
