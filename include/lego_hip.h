@@ -183,6 +183,10 @@ int lego_hip_stencil_laplacian_f32(const float* in, float* out, const float* c, 
 int lego_hip_stencil_f3d_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks, void* stream);
 int lego_hip_stencil_laplacian_f32_zeros(const float* in, float* out, const float* c, int n, int radius, int bricks,
                                          void* stream);
+/* How these walk a field, without touching a device: plan2[0] = planes that a wavefront takes, in columns along the first
+ * axis (0: a wavefront has a brick), plan2[1] = wavefronts that have any.  No counterpart in the reference; it is there
+ * so that the choice can be checked on the host. */
+int lego_hip_stencil_f32_plan(int n, int radius, int star, int bricks, int* plan2);
 
 /* LU decomposition without pivoting of an n x n fp32 row-major matrix, in place: on return the
  * strict lower triangle holds L (unit diagonal implied) and the upper triangle holds U, as

@@ -1022,6 +1022,14 @@ int lego_hip_stencil_laplacian_f32_zeros(const float* in, float* out, const floa
   return stencil(in, out, c, n, radius, 1, bricks, 0, stream);
 }
 
+int lego_hip_stencil_f32_plan(int n, int radius, int star, int bricks, int* plan2)
+{
+  if (plan2 == nullptr || n <= 0 || n % LEGO_STENCIL_BRICK || n > 1024 || radius < 1 || 2 * radius >= n ||
+      radius > (star ? LEGO_STENCIL_STAR_MAX_RADIUS : LEGO_STENCIL_MAX_RADIUS))
+    return kInvalid;
+  return ok_or(lego_stencil_f32_plan(n, radius, star ? 1 : 0, bricks ? 1 : 0, plan2));
+}
+
 int lego_hip_lud_f32(float* m, int n, void* stream)
 {
   if (!usable(m)) return kInvalid;

@@ -106,4 +106,4 @@ def emit():
         at_normal=at[0], at_bricks=at[1], coeff=code(coeff),
     )
     text = template("stencil.hip.j2").render(**params)
-    return Emitted("stencil_f32.hip", text, ["lego_stencil_f32_launch"]), dict(B=B, MAX_RADIUS=MAX_RADIUS, STAR_MAX_RADIUS=STAR_MAX_RADIUS)
+    return Emitted("stencil_f32.hip", text, ["lego_stencil_f32_launch", "lego_stencil_f32_plan"]), dict(B=B, MAX_RADIUS=MAX_RADIUS, STAR_MAX_RADIUS=STAR_MAX_RADIUS)

@@ -57,6 +57,7 @@ SIGNATURES = {
     "lego_hip_stencil_laplacian_f32": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "lego_hip_stencil_f3d_f32_zeros": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
     "lego_hip_stencil_laplacian_f32_zeros": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_void_p],
+    "lego_hip_stencil_f32_plan": [_c_int] * 4 + [_INT_ARRAY],
     "lego_hip_lud_f32": [_c_void_p, _c_int, _c_void_p],
     "lego_hip_lud_f32_plan": [_c_int, ctypes.POINTER(_c_int), _c_int, ctypes.POINTER(_c_int)],
     "lego_hip_nw_i32": [_c_void_p, _c_void_p, _c_int, _c_int, _c_void_p],

@@ -232,6 +232,38 @@ def test_gpu_stencil_columns_and_bricks_agree(kind, radius, n):
         assert (want[full, full, full] - ref[k, k, k]).abs().max().item() <= 2e-5 * (2 * radius + 1) ** 3
 
 
+@pytest.mark.parametrize("star,radius", [(0, 1), (1, 1), (1, 4)])
+def test_columns_of_large_fields_fill_the_chip(star, radius):
+    """2048 wavefronts run at once: beyond n = 512 the last round of them is at least four fifths full, or there are many rounds."""
+    import ctypes
+    from lego_amd import runtime
+    plan = (ctypes.c_int * 2)()
+    for n in range(520, 1025, 8):
+        runtime.call("lego_hip_stencil_f32_plan", n, radius, star, 0, plan)
+        planes, waves = plan
+        columns = -(-n // 64) * -(-n // 8)
+        assert planes >= 2 and waves == -(-n // planes) * columns
+        assert waves >= 0.8 * 2048 * -(-waves // 2048) and (waves <= 2048 or waves >= 5 * 2048), n
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [552, 592])
+def test_gpu_dense_columns_of_large_fields_agree_with_bricks(n):
+    """Beyond n = 512 columns that leave much of a round empty are cut into shorter chunks; on bricks a wavefront has a brick, and sums its
+    27 products in another order."""
+    from lego_amd import ops
+    print(f"f3d n={n}", flush=True)
+    m = n // 8
+    g = torch.Generator(device="cuda").manual_seed(n)
+    x = torch.rand(n, n, n, device="cuda", generator=g) * 2 - 1
+    c = torch.rand(8, 8, 8, device="cuda", generator=g)
+    a = ops.stencil_f3d(x, c, 1, False)
+    b = ops.stencil_f3d(x.view(m, 8, m, 8, m, 8).permute(0, 2, 4, 1, 3, 5).contiguous().view(n, n, n), c, 1, True)
+    b = b.view(m, m, m, 8, 8, 8).permute(0, 3, 1, 4, 2, 5).reshape(n, n, n)
+    assert (a - b).abs().max().item() <= 28 * 28 * 2.0 ** -24      # 28 products of at most 1, one rounding of at most half a unit of 28 each
+    assert a[1:-1, 1:-1, 1:-1].abs().max().item() > 0
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("n,radius", [(520, 1), (520, 3), (728, 2)])
 def test_gpu_star_columns_of_large_fields_agree_with_bricks(n, radius):
