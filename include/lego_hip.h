@@ -240,6 +240,10 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
 int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes);
 int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
                                  void* workspace, unsigned long long workspace_bytes, void* stream);
+/* Which problems of a grouped call are better apart, apart[g] = 1: those that need copies and that lego_hip_gemm_ex_ws would split
+ * along K, where the other problems do not fill the time of their chains.  Host only; lego_hip_grouped_gemm_f16_ws itself takes
+ * any of them. */
+int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart);
 /* What lego_hip_grouped_gemm_f16 launches for these sizes, without touching a device: plan3[0] = tile
  * size (256: 256 x 256 tiles, or 128: 128 x 128 tiles), plan3[1] = number of 256 x 256 tiles of all
  * problems, plan3[2] = how many of them, the last ones of the launch order, are computed as two

@@ -1117,6 +1117,7 @@ double grouped_makespan(const long* count, const double* cost, int batches, long
 // order as two 128 x 256 halves each (kind 0), or the kernel on 128 x 128 tiles (kind 1).
 struct GroupedPlan {
   int kind, tiles, split;
+  double time;      // the estimate that chose it, in the units below
 };
 
 // Costs in units of one k-tile step of a 256 x 256 tile that has its CU to itself (about 1.8 us for
@@ -1181,6 +1182,7 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
   plan.kind = t_small < best ? 1 : 0;
   plan.tiles = static_cast<int>(total);
   plan.split = plan.kind == 0 ? static_cast<int>(best_split) : 0;
+  plan.time = plan.kind == 1 ? t_small : best;
   return plan;
 }
 
@@ -1287,6 +1289,42 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
   if (plan.kind == 1) return ok_or(lego_grouped_gemm_f16_t128x128_launch(a, b, c, sizes3, groups, as_stream(stream)));
   if (plan.split == 0) return ok_or(lego_grouped_gemm_f16_launch(a, b, c, sizes3, groups, as_stream(stream)));
   return ok_or(lego_grouped_gemm_f16_split_launch(a, b, c, sizes3, groups, plan.split, as_stream(stream)));
+}
+
+// Ragged problems that a single product splits along K (more than 31 k-tiles): in the grouped launch they are chains of whole depth,
+// apart each is some four launches more.  Apart, then, where the launch without them is estimated shorter by more than 14 steps for
+// each, and 2.5 for each of up to eight others, whose calls are enqueued all the same.  Us, together / apart: 64 x 64 x 4095 beside three of 64^3
+// 44 / 32, 512 x 512 x 4095 beside four of 512^3 50 / 35; 64 x 64 x 4095 beside sixteen of 1024^3 68 / 64, which the estimate keeps
+// together as it does 512 x 512 x 2577 beside eight of 512^3, 42 / 44; four of 64 x 64 x 4095 48 / 61.  Over 4278 drawn calls of 2 to 16
+// problems the rule takes 1.013 times the better of the two, all apart 1.16, all together 1.19, by the number of problems 1.13.
+int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) try
+{
+  if (sizes3 == nullptr || apart == nullptr || groups <= 0 || groups > kGroupedMaxProblems) return kInvalid;
+  std::vector<int> order(static_cast<size_t>(groups));
+  for (int g = 0; g < groups; ++g) {
+    if (sizes3[3 * g] <= 0 || sizes3[3 * g + 1] <= 0 || sizes3[3 * g + 2] <= 0) return kInvalid;
+    order[static_cast<size_t>(g)] = g;
+    apart[g] = 0;
+  }
+  std::stable_sort(order.begin(), order.end(), [sizes3](int p, int q) { return sizes3[3 * p + 2] > sizes3[3 * q + 2]; });
+  // what the first launch carries: the deepest problems
+  const int count = groups < LEGO_GROUPED_MAX_GROUPS ? groups : LEGO_GROUPED_MAX_GROUPS;
+  int all[3 * LEGO_GROUPED_MAX_GROUPS], rest[3 * LEGO_GROUPED_MAX_GROUPS], deep[LEGO_GROUPED_MAX_GROUPS], others = 0, deeps = 0;
+  for (int i = 0; i < count; ++i) {
+    const int g = order[static_cast<size_t>(i)], m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
+    const bool ragged = n % 8 || k % 8;
+    const int size[3] = {m, ragged ? round_up(n, 8) : n, ragged ? round_up(k, 8) : k};
+    memcpy(all + 3 * i, size, sizeof(size));
+    if (ragged && k > 31 * LEGO_GEMM_BK) deep[deeps++] = g;
+    else memcpy(rest + 3 * others++, size, sizeof(size));
+  }
+  if (deeps == 0) return 0;
+  const double without = others ? grouped_plan(rest, others).time + 2.5 * (groups - 1 < 8 ? groups - 1 : 8) : 0.0;
+  if (grouped_plan(all, count).time > without + 14 * deeps)
+    for (int i = 0; i < deeps; ++i) apart[deep[i]] = 1;
+  return 0;
+} catch (const std::bad_alloc&) {
+  return ok_or(hipErrorOutOfMemory);
 }
 
 // Room for zero-padded copies of the problems whose N or K is no multiple of 8.

@@ -264,42 +264,63 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     return c
 
 
+_group_apart = {}      # sizes of a call's problems -> those that are products of their own
+
+
+def _problems_apart(sizes):
+    """Asked once for a list of sizes: the answer is a function of the sizes alone."""
+    groups = len(sizes) // 3
+    flags = (ctypes.c_int * groups)()
+    runtime.call("lego_hip_grouped_gemm_f16_apart", (ctypes.c_int * len(sizes))(*sizes), groups, flags)
+    if len(_group_apart) >= 1024:
+        _group_apart.clear()
+    apart = _group_apart[sizes] = frozenset(g for g in range(groups) if flags[g])
+    return apart
+
+
 def lego_group_gemm_fn(group_A, group_B):
     """One launch for a list of independent GEMMs; returns the list of results."""
     if len(group_A) != len(group_B):
         raise ValueError("group_A and group_B must have the same length")
+    # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace; those whose long chains the other
+    # problems leave alone run on their own.
+    sizes, ragged, deep = [], False, False
     for a, b in zip(group_A, group_B):
         _check(a, torch.float16, "A")
         _check(b, torch.float16, "B")
-        if a.shape[1] != b.shape[0]:
-            raise ValueError("Incompatible dimensions")
-    # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace.  In a call of two or three, those that a
-    # single product splits along K (32 k-tiles of 64 and more) go through `matmul`: little else runs beside their chains (two
-    # problems, one 688 x 640 x 2577: 36 us, in the grouped launch 44; eleven with three such 107 us, in the launch 68).
-    deep = [i for i, b in enumerate(group_B) if b.shape[0] > 31 * 64 and (b.shape[0] % 8 or b.shape[1] % 8)] if len(group_B) <= 3 else []
-    if deep:
-        rest = [i for i in range(len(group_A)) if i not in set(deep)]
-        out = [None] * len(group_A)
-        if rest:
-            for i, c in zip(rest, lego_group_gemm_fn([group_A[i] for i in rest], [group_B[i] for i in rest])):
-                out[i] = c
-        for i in deep:
-            out[i] = matmul(group_A[i], group_B[i])
-        return out
-    groups = len(group_A)
-    group_C, sizes, padded = [], [], False
-    for a, b in zip(group_A, group_B):
         M, K = a.shape
-        N = b.shape[1]
-        padded = padded or N % 8 != 0 or K % 8 != 0
-        group_C.append(torch.empty((M, N), device=a.device, dtype=a.dtype))
+        depth, N = b.shape
+        if K != depth:
+            raise ValueError("Incompatible dimensions")
         sizes += [M, N, K]
+        if N % 8 or K % 8:
+            ragged = True
+            deep = deep or K > 1984
+    if ragged and len(group_A) == 1:      # 1000 x 1001 x 1002 24 us, in a grouped launch 29
+        return [matmul(group_A[0], group_B[0])]
+    if deep:
+        key = tuple(sizes)
+        apart = _group_apart.get(key)
+        if apart is None:
+            apart = _problems_apart(key)
+        if apart:
+            rest = [g for g in range(len(group_A)) if g not in apart]
+            together = iter(_grouped([group_A[g] for g in rest], [group_B[g] for g in rest],
+                                     [s for g in rest for s in sizes[3 * g:3 * g + 3]]) if rest else ())
+            return [matmul(group_A[g], group_B[g]) if g in apart else next(together) for g in range(len(group_A))]
+    return _grouped(group_A, group_B, sizes)
+
+
+def _grouped(group_A, group_B, sizes):
+    """Checked problems, all in the grouped launch."""
+    groups = len(group_A)
+    group_C = [torch.empty((sizes[3 * g], sizes[3 * g + 1]), device=a.device, dtype=a.dtype) for g, a in enumerate(group_A)]
     arr = ctypes.c_void_p * groups
     pa = arr(*[t.data_ptr() for t in group_A])
     pb = arr(*[t.data_ptr() for t in group_B])
     pc = arr(*[t.data_ptr() for t in group_C])
     sz = (ctypes.c_int * (3 * groups))(*sizes)
-    if padded:
+    if any(s % 8 for s in sizes[1::3]) or any(s % 8 for s in sizes[2::3]):
         size = ctypes.c_ulonglong(0)
         runtime.call("lego_hip_grouped_gemm_f16_workspace_bytes", sz, groups, ctypes.byref(size))
         workspace = torch.empty(size.value // 2, dtype=torch.float16, device=group_C[0].device)

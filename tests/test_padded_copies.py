@@ -25,6 +25,25 @@ def test_padded_sizes_hold_the_copies():
     assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 1) == 0
 
 
+def _apart(*problems):
+    from lego_amd import runtime
+    flags = (ctypes.c_int * len(problems))()
+    runtime.call("lego_hip_grouped_gemm_f16_apart", (ctypes.c_int * (3 * len(problems)))(*sum(problems, ())), len(problems), flags)
+    return [i for i, f in enumerate(flags) if f]
+
+
+def test_deep_problems_leave_a_grouped_call_by_the_work_beside_them():
+    """A ragged problem's chain of k-tiles runs beside the others' work, however many they are, or in parts on its own."""
+    for few in (2, 3, 5):
+        assert _apart(*[(64, 64, 64)] * few, (64, 64, 4095)) == [few]              # next to nothing beside it
+        assert _apart((512, 512, 8191), *[(512, 512, 512)] * few) == [0]
+    assert _apart(*[(64, 64, 64)] * 15, (64, 64, 4095)) == [15]                     # many, and still nothing
+    assert _apart(*[(1024, 1024, 1024)] * 16, (64, 64, 2577)) == []                 # a chain beside rounds of tiles
+    assert _apart(*[(64, 64, 4095)] * 4) == []                                      # chains beside each other
+    assert _apart(*[(64, 64, 4096)] * 4) == [] and _apart((64, 65, 1984), (64, 64, 64)) == []      # whole chunks, or not split
+    assert _apart(*[(64, 64, 64)] * 100, (64, 64, 16383)) == [100]                  # more than a launch carries
+
+
 @pytest.mark.gpu
 @pytest.mark.parametrize("fp8", [torch.float8_e5m2, torch.float8_e4m3fn])
 @pytest.mark.parametrize("M,N,K", [(1, 65, 257), (17, 64, 4097), (33, 100, 264), (128, 129, 256), (1000, 1001, 271), (2500, 3001, 72)])
@@ -57,6 +76,7 @@ def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
 @pytest.mark.gpu
 @pytest.mark.parametrize("problems", [[(1, 65, 64), (64, 64, 64), (33, 72, 63)], [(5, 9, 2111), (64, 64, 64), (130, 1, 1)],
                                       [(9, 31, 2050), (64, 64, 64), (33, 72, 63), (3, 8, 8)],
+                                      [(64, 64, 64), (9, 31, 8190), (33, 72, 63), (3, 8, 8), (17, 8, 4100)], [(65, 63, 100)],
                                       [(16 + i, 63 + i, 65 + i) for i in range(70)]])
 def test_gpu_grouped_with_ragged_problems(problems):
     """Problems of whole chunks and others, deep ones, and more than the launches of the copies and of the products carry."""
