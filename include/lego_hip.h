@@ -235,7 +235,8 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
                               const int* sizes3, int groups, void* stream);
 
 /* lego_hip_grouped_gemm_f16 with room for zero-padded copies of the problems whose N or K is no multiple of 8: one launch for the
- * copies, the grouped one for all problems, and one that copies results back.  lego_hip_grouped_gemm_f16_workspace_bytes gives the
+ * copies, the grouped one for all problems, and one that copies results back; where the copies are more than 512 MiB, the same again for
+ * each run of problems whose copies are not (a run has one problem at least).  lego_hip_grouped_gemm_f16_workspace_bytes gives the
  * size for a list of problems (0: none is needed); without it (or 16-byte alignment of it) the call is lego_hip_grouped_gemm_f16. */
 int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes);
 int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,

@@ -1327,18 +1327,53 @@ int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) t
   return ok_or(hipErrorOutOfMemory);
 }
 
-// Room for zero-padded copies of the problems whose N or K is no multiple of 8.
-int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes)
+namespace {
+// Copies of the ragged problems of a call lie in the workspace together up to this much; what is beyond follows in further runs of the
+// same call, copies, launch and way back each, with no problem's own copies cut.  Sixteen products of 4095^3: 1.6 GB at once, 0.5 GB in runs
+// of five, whose 1280 tiles are five rounds of the chip.
+constexpr unsigned long long kCopyRoom = 512ull << 20;
+
+inline unsigned long long copies_of(const int* size) { return size[1] % 8 || size[2] % 8 ? padded_bytes(size[0], size[1], size[2], 8, 2) : 0ull; }
+
+// `run(problems, count, bytes)` for each run, as the call lists the problems where one run is all, otherwise deepest first.
+extern "C++" template <class Run>
+int grouped_copy_runs(const int* sizes3, int groups, const Run& run)
+{
+  unsigned long long total = 0;
+  std::vector<int> order(static_cast<size_t>(groups));
+  for (int g = 0; g < groups; ++g) {
+    order[static_cast<size_t>(g)] = g;
+    total += copies_of(sizes3 + 3 * g);
+  }
+  if (total > kCopyRoom) std::stable_sort(order.begin(), order.end(), [sizes3](int p, int q) { return sizes3[3 * p + 2] > sizes3[3 * q + 2]; });
+  for (int first = 0; first < groups;) {
+    unsigned long long used = 0;
+    int count = 0;
+    for (; first + count < groups; ++count) {
+      const unsigned long long more = copies_of(sizes3 + 3 * order[static_cast<size_t>(first + count)]);
+      if (used != 0 && used + more > kCopyRoom) break;
+      used += more;
+    }
+    const int rc = run(order.data() + first, count, used);
+    if (rc != 0) return rc;
+    first += count;
+  }
+  return 0;
+}
+}  // namespace
+
+// Room for zero-padded copies of the problems whose N or K is no multiple of 8: that of the largest run.
+int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes) try
 {
   if (sizes3 == nullptr || bytes == nullptr || groups <= 0 || groups > kGroupedMaxProblems) return kInvalid;
-  unsigned long long total = 0;
-  for (int g = 0; g < groups; ++g) {
-    const int m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
-    if (m <= 0 || n <= 0 || k <= 0) return kInvalid;
-    if (n % 8 || k % 8) total += padded_bytes(m, n, k, 8, 2);
-  }
-  *bytes = total;
+  for (int i = 0; i < 3 * groups; ++i)
+    if (sizes3[i] <= 0) return kInvalid;
+  unsigned long long most = 0;
+  grouped_copy_runs(sizes3, groups, [&](const int*, int, unsigned long long used) { most = std::max(most, used); return 0; });
+  *bytes = most;
   return 0;
+} catch (const std::bad_alloc&) {
+  return ok_or(hipErrorOutOfMemory);
 }
 
 int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
@@ -1348,30 +1383,33 @@ int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, voi
   unsigned long long need = 0;
   if (checked != 2 || lego_hip_grouped_gemm_f16_workspace_bytes(sizes3, groups, &need) != 0 || need == 0 || workspace_bytes < need || !usable(workspace))
     return lego_hip_grouped_gemm_f16(a, b, c, sizes3, groups, stream);
-  std::vector<const void*> aa(a, a + groups), bb(b, b + groups);
-  std::vector<void*> cc(c, c + groups);
-  std::vector<int> sizes(sizes3, sizes3 + 3 * static_cast<size_t>(groups));
-  Copier pads(true, as_stream(stream)), back(false, as_stream(stream));
-  uint8_t* at = static_cast<uint8_t*>(workspace);
-  std::vector<int> copied;
-  for (int g = 0; g < groups; ++g) {
-    const int m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
-    if (n % 8 == 0 && k % 8 == 0) continue;
-    const int mr = round_up(m, 8), nr = round_up(n, 8), kr = round_up(k, 8);
-    uint8_t *ap = at, *bp = ap + 2 * static_cast<size_t>(mr) * kr, *cp = bp + 2 * static_cast<size_t>(kr) * nr;
-    at = cp + 2 * static_cast<size_t>(mr) * nr;
-    if (kr != k || !usable(a[g])) { pads.add(a[g], ap, m, k, m, kr, 2); aa[g] = ap; }
-    if (kr != k || nr != n || !usable(b[g])) { pads.add(b[g], bp, k, n, kr, nr, 2); bb[g] = bp; }
-    if (nr != n || !usable(c[g])) { cc[g] = cp; copied.push_back(g); }
-    sizes[3 * g + 1] = nr;
-    sizes[3 * g + 2] = kr;
-  }
-  const hipError_t err = pads.flush();
-  if (err != hipSuccess) return ok_or(err);
-  const int rc = lego_hip_grouped_gemm_f16(aa.data(), bb.data(), cc.data(), sizes.data(), groups, stream);
-  if (rc != 0) return rc;
-  for (const int g : copied) back.add(cc[g], c[g], sizes3[3 * g], sizes3[3 * g + 1], sizes3[3 * g], sizes[3 * g + 1], 2);
-  return ok_or(back.flush());
+  std::vector<const void*> aa, bb;
+  std::vector<void*> cc;
+  std::vector<int> sizes, copied;
+  return grouped_copy_runs(sizes3, groups, [&](const int* problems, int count, unsigned long long) {
+    aa.clear(); bb.clear(); cc.clear(); sizes.clear(); copied.clear();
+    Copier pads(true, as_stream(stream)), back(false, as_stream(stream));
+    uint8_t* at = static_cast<uint8_t*>(workspace);
+    for (int i = 0; i < count; ++i) {
+      const int g = problems[i], m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
+      const bool ragged = n % 8 || k % 8;
+      const int mr = round_up(m, 8), nr = ragged ? round_up(n, 8) : n, kr = ragged ? round_up(k, 8) : k;
+      aa.push_back(a[g]); bb.push_back(b[g]); cc.push_back(c[g]);
+      sizes.insert(sizes.end(), {m, nr, kr});
+      if (!ragged) continue;
+      uint8_t *ap = at, *bp = ap + 2 * static_cast<size_t>(mr) * kr, *cp = bp + 2 * static_cast<size_t>(kr) * nr;
+      at = cp + 2 * static_cast<size_t>(mr) * nr;
+      if (kr != k || !usable(a[g])) { pads.add(a[g], ap, m, k, m, kr, 2); aa[i] = ap; }
+      if (kr != k || nr != n || !usable(b[g])) { pads.add(b[g], bp, k, n, kr, nr, 2); bb[i] = bp; }
+      if (nr != n || !usable(c[g])) { cc[i] = cp; copied.push_back(i); }
+    }
+    const hipError_t err = pads.flush();
+    if (err != hipSuccess) return ok_or(err);
+    const int rc = lego_hip_grouped_gemm_f16(aa.data(), bb.data(), cc.data(), sizes.data(), count, stream);
+    if (rc != 0) return rc;
+    for (const int i : copied) back.add(cc[i], c[problems[i]], sizes[3 * i], sizes3[3 * problems[i] + 1], sizes[3 * i], sizes[3 * i + 1], 2);
+    return ok_or(back.flush());
+  });
 } catch (const std::bad_alloc&) {
   return ok_or(hipErrorOutOfMemory);
 }

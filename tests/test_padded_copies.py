@@ -25,6 +25,16 @@ def test_padded_sizes_hold_the_copies():
     assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 1) == 0
 
 
+def test_copies_of_a_grouped_call_take_bounded_room():
+    """Sixteen ragged products of 4095 a side: copies of five of them at a time, not of all sixteen (1.6 GB)."""
+    one = 3 * 2 * 4096 * 4096
+    for count, need in ((1, one), (5, 5 * one), (16, 5 * one)):
+        sizes = (ctypes.c_int * (3 * count))(*[4095] * (3 * count))
+        assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, count) == need
+    sizes = (ctypes.c_int * 9)(20000, 20001, 64, 2000, 9999, 16, 64, 64, 64)       # one beyond the bound keeps its own room
+    assert _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 3) == 2 * (20000 * 64 + 64 * 20008 + 20000 * 20008)
+
+
 def _apart(*problems):
     from lego_amd import runtime
     flags = (ctypes.c_int * len(problems))()
@@ -71,6 +81,28 @@ def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
                          0 if fp8 == torch.float8_e4m3fn else 1, ws.data_ptr(), need, None)
             assert torch.equal(c[29:29 + M * N].view(M, N).cpu().float(), want)
             assert (c[:29] == 7).all() and (c[29 + M * N:] == 7).all()
+
+
+@pytest.mark.gpu
+def test_gpu_grouped_in_runs_of_bounded_copies():
+    """Copies of 680 MB in all, in two runs through the same room, with whole-chunk problems among them; nothing beyond the room is written."""
+    from lego_amd import ops, runtime
+    print("grouped, copies in runs", flush=True)
+    problems = [(90000, 1001, 9), (64, 64, 64), (90000, 1001, 17), (90000, 1999, 33), (8, 16, 8), (33, 72, 63)]
+    g = torch.Generator(device="cuda").manual_seed(5)
+    a = [torch.randint(-2, 3, (m, k), device="cuda", generator=g).half() for m, _, k in problems]
+    b = [torch.randint(-2, 3, (k, n), device="cuda", generator=g).half() for _, n, k in problems]
+    want = [(x.float() @ y.float()).half() for x, y in zip(a, b)]
+    for c, w in zip(ops.lego_group_gemm_fn(a, b), want):
+        assert torch.equal(c, w)
+    sizes = (ctypes.c_int * 18)(*sum(problems, ()))
+    need = _size("lego_hip_grouped_gemm_f16_workspace_bytes", sizes, 6)
+    assert need <= 512 << 20 < sum(2 * 8 * -(-m // 8) * 8 * -(-n // 8) for m, n, _ in problems if n % 8)
+    ws = torch.full((need + 64,), 0x5a, dtype=torch.uint8, device="cuda")
+    c = [torch.zeros_like(w) for w in want]
+    pointers = lambda ts: (ctypes.c_void_p * 6)(*[t.data_ptr() for t in ts])
+    runtime.call("lego_hip_grouped_gemm_f16_ws", pointers(a), pointers(b), pointers(c), sizes, 6, ws.data_ptr(), need, None)
+    assert all(torch.equal(x, w) for x, w in zip(c, want)) and (ws[need:] == 0x5a).all()
 
 
 @pytest.mark.gpu
