@@ -1293,10 +1293,11 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
 
 // Ragged problems that a single product splits along K (more than 31 k-tiles): in the grouped launch they are chains of whole depth,
 // apart each is some four launches more.  Apart, then, where the launch without them is estimated shorter by more than 14 steps for
-// each, and 2.5 for each of up to eight others, whose calls are enqueued all the same.  Us, together / apart: 64 x 64 x 4095 beside three of 64^3
+// each and twice what it is of a step of the whole chip, and 2.5 for each of up to eight others, whose calls are enqueued all the same.  Us, together / apart: 64 x 64 x 4095 beside three of 64^3
 // 44 / 32, 512 x 512 x 4095 beside four of 512^3 50 / 35; 64 x 64 x 4095 beside sixteen of 1024^3 68 / 64, which the estimate keeps
-// together as it does 512 x 512 x 2577 beside eight of 512^3, 42 / 44; four of 64 x 64 x 4095 48 / 61.  Over 4278 drawn calls of 2 to 16
-// problems the rule takes 1.013 times the better of the two, all apart 1.16, all together 1.19, by the number of problems 1.13.
+// together as it does 512 x 512 x 2577 beside eight of 512^3, 42 / 44; four of 64 x 64 x 4095 48 / 61, eight of 3001 x 2999 x
+// 3003 562 / 669.  Over 9831 drawn calls of 2 to 16 problems the rule takes 1.013 times the better of the two, all apart 1.19, all
+// together 1.11, by the number of problems 1.10.
 int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) try
 {
   if (sizes3 == nullptr || apart == nullptr || groups <= 0 || groups > kGroupedMaxProblems) return kInvalid;
@@ -1310,17 +1311,22 @@ int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) t
   // what the first launch carries: the deepest problems
   const int count = groups < LEGO_GROUPED_MAX_GROUPS ? groups : LEGO_GROUPED_MAX_GROUPS;
   int all[3 * LEGO_GROUPED_MAX_GROUPS], rest[3 * LEGO_GROUPED_MAX_GROUPS], deep[LEGO_GROUPED_MAX_GROUPS], others = 0, deeps = 0;
+  double alone = 0.0;
   for (int i = 0; i < count; ++i) {
     const int g = order[static_cast<size_t>(i)], m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
     const bool ragged = n % 8 || k % 8;
     const int size[3] = {m, ragged ? round_up(n, 8) : n, ragged ? round_up(k, 8) : k};
     memcpy(all + 3 * i, size, sizeof(size));
-    if (ragged && k > 31 * LEGO_GEMM_BK) deep[deeps++] = g;
-    else memcpy(rest + 3 * others++, size, sizeof(size));
+    if (ragged && k > 31 * LEGO_GEMM_BK) {
+      deep[deeps++] = g;
+      alone += 14.0 + 2.0 * m * n * k / (256.0 * 256 * 256 * LEGO_GEMM_BK);
+    } else {
+      memcpy(rest + 3 * others++, size, sizeof(size));
+    }
   }
   if (deeps == 0) return 0;
   const double without = others ? grouped_plan(rest, others).time + 2.5 * (groups - 1 < 8 ? groups - 1 : 8) : 0.0;
-  if (grouped_plan(all, count).time > without + 14 * deeps)
+  if (grouped_plan(all, count).time > without + alone)
     for (int i = 0; i < deeps; ++i) apart[deep[i]] = 1;
   return 0;
 } catch (const std::bad_alloc&) {

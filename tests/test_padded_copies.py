@@ -50,6 +50,7 @@ def test_deep_problems_leave_a_grouped_call_by_the_work_beside_them():
     assert _apart(*[(64, 64, 64)] * 15, (64, 64, 4095)) == [15]                     # many, and still nothing
     assert _apart(*[(1024, 1024, 1024)] * 16, (64, 64, 2577)) == []                 # a chain beside rounds of tiles
     assert _apart(*[(64, 64, 4095)] * 4) == []                                      # chains beside each other
+    assert _apart(*[(3001, 2999, 3003)] * 8) == []                                  # rounds of the whole chip
     assert _apart(*[(64, 64, 4096)] * 4) == [] and _apart((64, 65, 1984), (64, 64, 64)) == []      # whole chunks, or not split
     assert _apart(*[(64, 64, 64)] * 100, (64, 64, 16383)) == [100]                  # more than a launch carries
 
