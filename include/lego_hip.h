@@ -270,8 +270,12 @@ int lego_hip_layernorm_fwd_f16_wpr(const void* x, void* y, const void* w, const 
                                    float* mean, float* rstd, int M, int N, float eps,
                                    int waves_per_row, void* stream);
 
-/* What lego_hip_gemm_f16_ex and lego_hip_gemm_bf16*_ex launch for a product whose operands lie in whole 16-byte chunks,
- * without touching a device: plan2[0] = side of the workgroup's tile (256 or 128), plan2[1] = side of the MFMA's
+/* Whether a product whose operands lie in whole 16-byte chunks (of element_bytes = 1 or 2) is of so few rows that a kernel of its own reads
+ * a transposed B once: columns of the result per workgroup, or 0, and then tiles are launched.  Host only. */
+int lego_hip_gemm_rows_plan(int M, int N, int K, int trans_a, int trans_b, int element_bytes, int* columns);
+
+/* What lego_hip_gemm_f16_ex and lego_hip_gemm_bf16*_ex launch for a product whose operands lie in whole 16-byte chunks and for which
+ * lego_hip_gemm_rows_plan gives 0, without touching a device: plan2[0] = side of the workgroup's tile (256 or 128), plan2[1] = side of the MFMA's
  * accumulator block (16: v_mfma_f32_16x16x32, 32: v_mfma_f32_32x32x16).  No counterpart in the reference (its
  * autotuner picks among tile configurations at run time, matmul_sympy.py:98-165); it is there so that the choice can be
  * checked on the host. */

@@ -281,7 +281,7 @@ def collect():
           "const int*, int, int, hipStream_t);",
           "hipError_t lego_gemm_stamps_read(unsigned long long*, int);",
           "hipError_t lego_gemm_any_launch(const void*, const void*, void*, int, int, int, int, int, int, int, hipStream_t);",
-          "hipError_t lego_gemm_rows_launch(const void*, const void*, void*, int, int, int, int, int, hipStream_t);",
+          "hipError_t lego_gemm_rows_launch(const void*, const void*, void*, int, int, int, int, int, int, hipStream_t);",
           "hipError_t lego_grouped_gemm_f16_split_launch(const void* const*, const void* const*, void* const*, "
           "const int*, int, int, hipStream_t);",
           f"#define LEGO_GEMM_BM {mg['BM']}", f"#define LEGO_GEMM_BN {mg['BN']}", f"#define LEGO_GEMM_BK {mg['BK']}",

@@ -704,13 +704,30 @@ inline int gemm_choice(int M, int N, bool has_small, bool has_sparse)
   return has_sparse && tiles < kSparseRoundBelow ? 2 : 0;
 }
 
-// Few rows against a k-major B: the kernel that reads B once, straight into registers.  Us, tiles / this, 16 rows of bf16: 1024 x 1024
-// 11.3 / 10.5, 2048 x 4096 16.0 / 12.2, 4096 x 4096 16.0 / 12.3, 6144 x 4096 22.0 / 14.2, 8192 x 8192 33.2 / 25.8, 16384 x 4096 33.2 / 31.6; 1024 x
-// 8192 16.0 / 16.8 and 64 x 8192 14.2 / 16.7, where a workgroup's K is long and there are few of them; of 32 rows, which read A
-// twice as often, 8192 x 8192 34.3 / 34.5.
-inline bool takes_rows(int M, int N, int K, int trans_a, int trans_b, int bytes)
+// Few rows against a k-major B: columns of C per workgroup of the kernel that reads B once, straight into registers, or 0: tiles.
+// A workgroup reads its columns of B and all of A, which tell in rounds of one workgroup per CU: the least of rounds * (columns + 3/4 M), and 4 KB
+// of a row for a workgroup's start; wider where that is a thirtieth less (16 / 32 / 64 columns, us, bf16: 1 x 8576 x 6784 32 / 39 / 37, 16 x 8192 x 8192
+// 35 / 25 / 46, 16 x 16384 x 8192 68 / 58 / 52; over 2148 drawn products 1.004 of the best of the three).  Tiles / this: 16 x 1024 x 1024 12.0 / 4.6, 16 x 4096 x 4096 15.0 / 10.3, 16 x 8192 x 8192 33.2 / 25.3,
+// 16 x 16384 x 4096 33.4 / 27.8, 1 x 5120 x 8192 28.7 / 19.0.  Tiles are better
+//   where there is next to nothing to read: K of 256 bytes 4.4 / 5.0, of 384 4.5 / 5.0 (8 x 23040 x 432 of 8 bits 7.3 / 5.2);
+//   where K is long beside N: 1024 x 8192 16.0 / 16.8 (and 64 x 8192 14.2 / 16.7);
+//   of many columns, where they fill the chip without a split: 16 x 40960 x 8192 174 / 191 (from 2 KB a row on: 12 x 46912 x 544 15.4 / 13.1), 8 x 65536 x 6144 151 / 163;
+//   of more than eight rows, for which A is read often: 16 x 2048 x 6144 12.8 / 13.6, 16 x 5120 x 5120 18.1 / 20.7 (5120 x 4096 20.6 / 13.8, and of
+//   eight rows all that was drawn), 16 x 8448 x 10240 54 / 64.
+// Of 32 rows, which read A twice as often, 8192 x 8192 34.3 / 34.5.
+inline int rows_columns(int M, int N, int K, int trans_a, int trans_b, int bytes)
 {
-  return M <= 16 && !trans_a && trans_b && N >= 1024 && (N <= 4096 || N >= 6144) && K <= 4l * N && static_cast<long>(K) * bytes * 32 < (1l << 31) && static_cast<long>(N) * K < (1l << 31);
+  const long k_bytes = static_cast<long>(K) * bytes;
+  if (M > 16 || trans_a || !trans_b || N < 1024 || K > 4l * N || k_bytes <= (N <= 8192 ? 384 : 256) || 64 * k_bytes >= (1l << 31) || static_cast<long>(N) * K >= (1l << 31)) return 0;
+  if (N > (M > 8 && k_bytes > 2 << 10 ? 36864 : 49152)) return 0;
+  if (M > 8 && ((N < 2560 && k_bytes >= 11 << 10) || (N > 4096 && N < 6144 && k_bytes > 8 << 10) || (N > 8192 && N < 12288 && k_bytes > 16 << 10))) return 0;
+  int best = 0;
+  long least = 0;
+  for (const int columns : {16, 32, 64}) {
+    const long rounds = ((N + columns - 1) / columns + 255) / 256, cost = rounds * (k_bytes * (4 * columns + 3 * M) + (16 << 10));
+    if (best == 0 || 33 * cost < 32 * least) { best = columns; least = cost; }
+  }
+  return best;
 }
 
 int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, void* c, int M, int N, int K,
@@ -733,8 +750,8 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
     return ok_or(lego_gemm_any_launch(a, b, c, M, N, K, trans_a ? 1 : 0, trans_b ? 1 : 0, activation, element,
                                       as_stream(stream)));
   }
-  if (takes_rows(M, N, K, trans_a, trans_b, element == 2 || element == 3 ? 1 : 2))
-    return ok_or(lego_gemm_rows_launch(a, b, c, M, N, K, activation, element, as_stream(stream)));
+  if (const int columns = rows_columns(M, N, K, trans_a, trans_b, element == 2 || element == 3 ? 1 : 2))
+    return ok_or(lego_gemm_rows_launch(a, b, c, M, N, K, columns, activation, element, as_stream(stream)));
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
   const int choice = gemm_choice(M, N, k.small[layout] != nullptr, k.sparse[layout] != nullptr);
   const gemm_launcher* by_layout = choice == 1 ? k.small : choice == 2 ? k.sparse : k.big;
@@ -891,7 +908,7 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
   if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
   const auto product = [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK);
-    if (parts < 2 || takes_rows(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
+    if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
     return ok_or(parts_by_layout(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
   };
   if (tiled) return product(a, b, c, M, N, K, workspace);
@@ -931,7 +948,7 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
   if ((format != 0 && format != 1) || lego_hip_gemm_fp8_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) &&
                      (!trans_b || K % 16 == 0);
-  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need || takes_rows(M, N, K, trans_a, trans_b, 1))
+  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need || rows_columns(M, N, K, trans_a, trans_b, 1))
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
@@ -964,7 +981,7 @@ int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N
   return on_padded_copies(16, 1, a, b, c, M, N, K, trans_a, trans_b, workspace, stream,
                           [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK_8BIT);
-    if (parts < 2 || takes_rows(m, n, k, trans_a, trans_b, 1)) return whole(aa, bb, cc, m, n, k);
+    if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 1)) return whole(aa, bb, cc, m, n, k);
     return ok_or(fp8_parts(format)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums),
                                                                          as_stream(stream)));
   });
@@ -1433,6 +1450,13 @@ int lego_hip_gemm_plan(int M, int N, int K, int* plan2)
   const int choice = gemm_choice(M, N, true, true);
   plan2[0] = choice == 1 ? 128 : 256;
   plan2[1] = choice == 0 ? 16 : 32;
+  return 0;
+}
+
+int lego_hip_gemm_rows_plan(int M, int N, int K, int trans_a, int trans_b, int element_bytes, int* columns)
+{
+  if (columns == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
+  *columns = rows_columns(M, N, K, trans_a, trans_b, element_bytes);
   return 0;
 }
 

@@ -580,14 +580,14 @@ def emit_any(bm=64, bn=64, bk=32):
     return Emitted("gemm_any.hip", text, ["lego_gemm_any_launch"])
 
 
-def emit_rows(max_m=16, waves=8, wide_above=4096):
+def emit_rows(max_m=16, waves=8):
     """The kernel for few rows of A against a k-major B: B is read once, straight into MFMA operands."""
     M, N, K = size("M"), size("N"), size("K")
     row, col, kk = (idx(n) for n in ("row", "col", "kk"))
     rng = {row: (0, M), col: (0, N), kk: (0, K)}
     flat = lambda lay, i, j: tidy(lay.TileBy([lay.dims()[0], lay.dims()[1]])[i, j], rng)  # noqa: E731
     text = template("gemm_rows.hip.j2").render(
-        banner=BANNER, MAX_M=max_m, WAVES=waves, WIDE_ABOVE=wide_above,
+        banner=BANNER, MAX_M=max_m, WAVES=waves,
         a_layout="OrderBy(Row(M, K))[row, kk]", b_layout="OrderBy(Col(K, N))[kk, col]", c_layout="OrderBy(Row(M, N))[row, col]",
         a_off=code(flat(OrderBy(Row(M, K)), row, kk)), b_off=code(flat(OrderBy(Col(K, N)), kk, col)),
         c_off=code(flat(OrderBy(Row(M, N)), row, col)))
