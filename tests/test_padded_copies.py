@@ -85,6 +85,21 @@ def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
 
 
 @pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K,transposed_first", [(5, 520, 1023, False), (5, 521, 1024, False), (5, 520, 1024, True), (67, 520, 1023, True), (5, 520, 376, False)])
+def test_gpu_column_major_rows_of_no_whole_chunks(M, N, K, transposed_first, monkeypatch):
+    """A small column-major A is stored row-major first where the product would run by elements, not where copies take it."""
+    from lego_amd import ops
+    print(f"tn {M}x{N}x{K}", flush=True)
+    calls, transpose = [], ops.transpose
+    monkeypatch.setattr(ops, "transpose", lambda t: calls.append(t.shape) or transpose(t))
+    g = torch.Generator().manual_seed(M + N + K)
+    a = torch.randint(-1, 2, (M, K), generator=g).half()
+    b = torch.randint(-1, 2, (K, N), generator=g).half()
+    got = ops.matmul(a.t().contiguous().cuda().t(), b.cuda())
+    assert torch.equal(got.cpu().float(), a.float() @ b.float()) and bool(calls) == transposed_first
+
+
+@pytest.mark.gpu
 def test_gpu_grouped_in_runs_of_bounded_copies():
     """Copies of 680 MB in all, in two runs through the same room, with whole-chunk problems among them; nothing beyond the room is written."""
     from lego_amd import ops, runtime
