@@ -85,6 +85,8 @@ bool plain(const at::Tensor& t)
   return t.defined() && t.is_cuda() && !beyond(t.key_set(), known) && t.is_contiguous() && !t._fw_grad(0).defined();
 }
 
+bool on_its_element(const at::Tensor& t) { return reinterpret_cast<uintptr_t>(t.const_data_ptr()) % t.element_size() == 0; }
+
 // lego_layer_norm(x, (n,), weight, bias, eps), or None where the node in Python is to take the call
 py::object apply(const py::handle& x_, const py::handle& shape, const py::handle& weight_, const py::handle& bias_, const py::handle& eps)
 {
@@ -97,8 +99,9 @@ py::object apply(const py::handle& x_, const py::handle& shape, const py::handle
   PyObject* const length = PyTuple_GET_ITEM(shape.ptr(), 0);
   if (!PyLong_CheckExact(length) || PyLong_AsLongLong(length) != n) { PyErr_Clear(); return py::none(); }
   if (!entries_of(x.scalar_type()) || x.numel() / n > INT_MAX || n * (int64_t)x.element_size() > 65536) return py::none();
+  if (!((float)PyFloat_AS_DOUBLE(eps.ptr()) >= 0.0f) || !on_its_element(x)) return py::none();      // what the entry point refuses
   for (const at::Tensor& t : {weight, bias})
-    if (t.dim() != 1 || t.size(0) != n || t.scalar_type() != x.scalar_type() || t.device() != x.device()) return py::none();
+    if (t.dim() != 1 || t.size(0) != n || t.scalar_type() != x.scalar_type() || t.device() != x.device() || !on_its_element(t)) return py::none();
   at::Tensor y;
   {
     py::gil_scoped_release nothing_here_needs_it;

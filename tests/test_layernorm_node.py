@@ -88,3 +88,17 @@ def test_gpu_hooks_streams_versions_and_modes():
     for call in (ops.lego_layer_norm, ops.LEGOLayerNorm.apply):
         with pytest.raises(Exception):
             torch.vmap(lambda t: call(t, (256,), w.detach(), b.detach(), 1e-5))(x.detach()[None])
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("eps", [-1.0, -1e-3, float("nan")])
+def test_gpu_refused_eps_keeps_its_error(eps):
+    """An eps that the entry point refuses, before anything is launched, is the error of the call in Python: its entry and code."""
+    from lego_amd import ops, runtime
+    print(f"layernorm node, eps {eps}", flush=True)
+    x, w, b, _ = _inputs((4, 64), torch.float32)
+    assert runtime.layernorm_node().apply(x, (64,), w, b, eps) is None
+    with pytest.raises(runtime.LegoHipError) as refused:
+        ops.lego_layer_norm(x, (64,), w, b, eps)
+    assert refused.value.entry == "lego_hip_layernorm_fwd_f32" and refused.value.code == 1
+    assert runtime.layernorm_node().apply(x, (64,), w, b, 0.0) is not None
