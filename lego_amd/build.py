@@ -381,14 +381,13 @@ def _compile(src: Path, incremental: bool = False) -> Path:
 
 
 def build_node(incremental: bool = False) -> Path:
-    """Compile the LayerNorm node (C++ over torch's headers) beside liblego_hip.so, which it is linked with."""
+    """Compile the LayerNorm node (C++ over torch's headers) beside liblego_hip.so, which it is linked with.  The object is tied to
+    torch's C++ ABI: what it was built with is kept in a stamp beside it, and another torch or command builds it again."""
     import sysconfig
 
     import torch
     from torch.utils import cpp_extension
-    src = CSRC / f"{NODE_PATH.stem}.cpp"
-    if incremental and NODE_PATH.exists() and NODE_PATH.stat().st_mtime > max(p.stat().st_mtime for p in (src, ROOT / "include" / "lego_hip.h")):
-        return NODE_PATH
+    src, stamp = CSRC / "layernorm_node.cpp", NODE_PATH.with_suffix(".stamp")
     includes = [str(ROOT / "include"), *cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
     libs = cpp_extension.library_paths()
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
@@ -396,9 +395,15 @@ def build_node(incremental: bool = False) -> Path:
            *[a for i in includes for a in ("-I", i)], str(src), "-o", str(NODE_PATH),
            *[a for d in libs for a in ("-L", d, f"-Wl,-rpath,{d}")], "-L", str(LIB_DIR), "-Wl,-rpath,$ORIGIN", f"-l:{LIB_PATH.name}",
            "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-ltorch_hip"]
+    built_with = "\n".join([torch.__version__, sys.version, *cmd])
+    if (incremental and NODE_PATH.exists() and stamp.exists() and stamp.read_text() == built_with
+            and NODE_PATH.stat().st_mtime > max(p.stat().st_mtime for p in (src, ROOT / "include" / "lego_hip.h"))):
+        return NODE_PATH
+    stamp.unlink(missing_ok=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed on {src.name}:\n{res.stderr}")
+    stamp.write_text(built_with)
     return NODE_PATH
 
 
@@ -413,9 +418,12 @@ def build(verbose=True, incremental=False):
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"link failed:\n{res.stderr}")
-    build_node(incremental)
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} translation units")
+    try:
+        build_node(incremental)
+    except ModuleNotFoundError as missing:      # the library itself needs no torch
+        print(f"{NODE_PATH.name} is not built: {missing}")
     return LIB_PATH
 
 

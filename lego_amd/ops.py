@@ -14,6 +14,7 @@ only carriers of device pointers: every call goes through the C ABI of liblego_h
 from __future__ import annotations
 
 import ctypes
+import warnings
 
 import torch
 
@@ -164,12 +165,27 @@ class LEGOLayerNorm(torch.autograd.Function):
         return dx, None, dw, db, None
 
 
+_node_apply = None
+
+
+def _load_node():
+    """The node in C++, or, where it is not built or not for this torch, one that leaves every call to the node in Python (the same
+    kernels, some 50 us more of host time a step), and says so."""
+    global _node_apply
+    try:
+        _node_apply = runtime.layernorm_node().apply
+    except (FileNotFoundError, ImportError) as e:
+        warnings.warn(f"LayerNorm runs through its autograd node in Python: {e}", RuntimeWarning, stacklevel=3)
+        _node_apply = lambda *args: None      # noqa: E731
+    return _node_apply
+
+
 def lego_layer_norm(x, normalized_shape, weight, bias, eps):
     """LayerNorm with the reference's signature and gradients (triton_generated/layernorm/layernorm.py:323-407).  Plain GPU
     tensors go through the node in C++ (csrc/layernorm_node.cpp); subclasses, dual tensors, calls under a tracer, a mode or a
     transform, and calls that are refused, through the one above."""
     if not torch.compiler.is_compiling():
-        y = runtime.layernorm_node().apply(x, normalized_shape, weight, bias, eps)
+        y = (_node_apply or _load_node())(x, normalized_shape, weight, bias, eps)
         if y is not None:
             return y
     return LEGOLayerNorm.apply(x, normalized_shape, weight, bias, eps)

@@ -131,7 +131,7 @@ def layernorm_node():
         import importlib.util
         if not NODE_PATH.exists():
             raise FileNotFoundError(
-                f"{NODE_PATH} is missing: build it with `python -m lego_amd.build` (there is no fallback path)")
+                f"{NODE_PATH} is missing: build it with `python -m lego_amd.build`")
         loader = importlib.machinery.ExtensionFileLoader("layernorm_node", str(NODE_PATH))
         module = importlib.util.module_from_spec(importlib.util.spec_from_loader("layernorm_node", loader))
         loader.exec_module(module)

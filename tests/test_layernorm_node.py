@@ -13,6 +13,40 @@ def test_refused_calls_keep_their_errors():
         ops.lego_layer_norm(torch.ones(4, 8), (4,), w, w, 1e-5)
 
 
+@pytest.mark.parametrize("content", [None, "not a shared object"])
+def test_calls_go_on_without_the_node_in_cpp(tmp_path, monkeypatch, content):
+    """Not built, or an object that does not load (another torch's): one warning, and the node in Python takes the calls."""
+    from lego_amd import ops, runtime
+    monkeypatch.setattr(runtime, "_node", None)
+    monkeypatch.setattr(runtime, "NODE_PATH", tmp_path / "layernorm_node.so")
+    monkeypatch.setattr(ops, "_node_apply", None)
+    if content:
+        runtime.NODE_PATH.write_text(content)
+    w = torch.ones(8)
+    with pytest.warns(RuntimeWarning, match="in Python"), pytest.raises(ValueError, match="GPU"):
+        ops.lego_layer_norm(torch.ones(4, 8), (8,), w, w, 1e-5)
+
+
+def test_the_node_is_built_again_for_another_torch(tmp_path, monkeypatch):
+    import subprocess
+    from lego_amd import build
+    built = []
+
+    def run(cmd, **kwargs):
+        built.append(cmd)
+        build.NODE_PATH.write_text("")
+        return subprocess.CompletedProcess(cmd, 0, "", "")
+    monkeypatch.setattr(build, "NODE_PATH", tmp_path / "layernorm_node.so")
+    monkeypatch.setattr(build.subprocess, "run", run)
+    for _ in range(3):
+        build.build_node(incremental=True)
+    assert len(built) == 1
+    monkeypatch.setattr(torch, "__version__", "0.0")
+    build.build_node(incremental=True)
+    build.build_node(incremental=True)
+    assert len(built) == 2
+
+
 def _inputs(shape, dtype, seed=0):
     g = torch.Generator(device="cuda").manual_seed(seed)
     n = shape[-1]
