@@ -1,4 +1,6 @@
 """Needleman-Wunsch: the oracle is pinned on the CPU, the kernel against the oracle on the GPU."""
+from pathlib import Path
+
 import numpy as np
 import pytest
 import sympy as sp
@@ -102,6 +104,57 @@ def test_gpu_single_launch_agrees_with_a_launch_per_anti_diagonal(n):
     for _ in range(2):      # the second call finds the first one's workspace in the allocator
         got = ops.needleman_wunsch(ref.cuda(), m.cuda(), 3).cpu()
         assert torch.equal(got, want)
+
+
+_ONE_LANE = """
+#include <algorithm>
+#include <climits>
+using std::max;
+#define __device__
+#define __forceinline__ inline
+#define __builtin_amdgcn_mov_dpp(v, ...) (v)
+#define __builtin_amdgcn_update_dpp(edge, v, ...) (edge)      // lane 0: the column to its left
+typedef int int2v __attribute__((vector_size(8)));
+constexpr int kP = %(P)d;
+inline int slot_at(int slot, int) { return 2 * slot; }
+%(code)s
+int main()
+{
+  const int ends[] = {INT_MIN, INT_MIN + 1, -1, 0, 1, INT_MAX - 1, INT_MAX};
+  for (int penalty : ends) for (int score : ends) for (int edge : ends) {
+    int2v scores[kP];
+    for (auto& s : scores) s = int2v{plus(score, penalty), plus(minus(0, score), penalty)};
+    alignas(8) int out[2 * kP];
+    int ga = minus(edge, penalty), gb = ga, gnw = ga;
+    run_phase<false>(4, 0, penalty, scores, minus(edge, penalty), out, ga, gb, gnw);
+    // the recurrence as it is written down, modulo 2^32
+    int up_a = edge, up_b = edge, corner = edge;
+    for (int i = 0; i < kP; ++i) {
+      const int a = max(max(plus(corner, score), minus(up_a, penalty)), minus(edge, penalty));
+      const int b = max(max(plus(up_a, minus(0, score)), minus(up_b, penalty)), minus(a, penalty));
+      if (a != plus(out[2 * i], penalty) || b != plus(out[2 * i + 1], penalty)) return 1;
+      corner = edge, up_a = a, up_b = b;
+    }
+  }
+}
+"""
+
+
+def test_sums_wrap_as_the_language_promises(tmp_path):
+    """The recurrence of one lane, as the generator prints it, over the ends of the type: with a trap on signed overflow, which
+    the compiler may otherwise take as never happening, it runs through and gives the cells modulo 2^32."""
+    import re
+    import subprocess
+    from lego_amd.kernels import nw as gen
+    text = (Path(__file__).resolve().parents[1] / "lego_amd" / "csrc" / "generated" / "nw_i32.hip").read_text()
+    code = "\n".join(re.findall(r"^__device__ __forceinline__ int (?:plus|minus)\(.*$", text, re.M))
+    code += "\n" + re.search(r"template <bool kStart>\n.*?\n}\n", text, re.S).group(0)
+    src = tmp_path / "lane.cpp"
+    src.write_text(_ONE_LANE % {"P": gen.P, "code": code})
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-fsanitize=signed-integer-overflow", "-fsanitize-undefined-trap-on-error",
+                    str(src), "-o", str(tmp_path / "lane")], check=True)
+    assert subprocess.run([str(tmp_path / "lane")]).returncode == 0
+    assert not re.search(r"[-+] penalty|nw \+ ", re.sub(r"//.*", "", text))      # nor anywhere else in the kernels
 
 
 @pytest.mark.gpu
