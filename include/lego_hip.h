@@ -159,6 +159,9 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes);
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream);
+/* What lego_hip_gemm_ex_ws (element_bytes 2) or lego_hip_gemm_fp8_ex_ws (1) uses of that for operands of this layout: 0 too for products that
+ * run without (lego_hip_gemm_rows_plan), which the plain entry points compute as well. */
+int lego_hip_gemm_layout_workspace_bytes(int M, int N, int K, int trans_a, int trans_b, int element_bytes, unsigned long long* bytes);
 /* The product on zero-padded copies for operand rows that are not whole 16-byte chunks (lego_hip_gemm_fp8_padded_bytes gives the
  * size of the workspace, 0 where copies gain nothing): one launch for the copies, the product, one that copies the result back.
  * Without it (or 16-byte alignment of it) the call is lego_hip_gemm_fp8_ex. */

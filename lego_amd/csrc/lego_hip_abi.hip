@@ -956,6 +956,16 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
                                          static_cast<float*>(workspace), as_stream(stream)));
 }
 
+// The same sizes for operands of one layout: the kernel for few rows takes some of these products and needs no room for sums.
+int lego_hip_gemm_layout_workspace_bytes(int M, int N, int K, int trans_a, int trans_b, int element_bytes, unsigned long long* bytes)
+{
+  if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
+  const int chunk = 16 / element_bytes;
+  *bytes = 0;
+  if (N % chunk == 0 && K % chunk == 0 && rows_columns(M, N, K, trans_a, trans_b, element_bytes)) return 0;
+  return (element_bytes == 1 ? lego_hip_gemm_fp8_workspace_bytes : lego_hip_gemm_workspace_bytes)(M, N, K, bytes);
+}
+
 // Whether a product whose rows are not whole 16-byte chunks gains from copies that are; room for these and for the sums of their product.
 int lego_hip_gemm_fp8_padded_bytes(int M, int N, int K, int trans_a, int trans_b, unsigned long long* bytes)
 {

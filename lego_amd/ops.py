@@ -207,7 +207,7 @@ def _operand(t, name):
     raise ValueError(f"{name} must be contiguous or the transpose of a contiguous tensor")
 
 
-_gemm_workspace, _fp8_workspace, _fp8_padded = {}, {}, {}      # (M, N, K, ...) -> bytes of workspace that the product uses
+_gemm_workspace, _fp8_padded = {}, {}      # (M, N, K, ta, tb, ...) -> bytes of workspace that the product uses
 
 
 def _ask_workspace(entry, known, shape):
@@ -244,9 +244,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
                 need = _ask_workspace("lego_hip_gemm_fp8_padded_bytes", _fp8_padded, (M, N, K, ta, tb))
             entry = "lego_hip_gemm_fp8_padded"
         else:
-            need = _fp8_workspace.get((M, N, K))
+            need = _gemm_workspace.get((M, N, K, ta, tb, 1))
             if need is None:
-                need = _ask_workspace("lego_hip_gemm_fp8_workspace_bytes", _fp8_workspace, (M, N, K))
+                need = _ask_workspace("lego_hip_gemm_layout_workspace_bytes", _gemm_workspace, (M, N, K, ta, tb, 1))
             entry = "lego_hip_gemm_fp8_ex_ws"
         if need:
             workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
@@ -267,9 +267,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     c = torch.empty((M, N), device=a.device, dtype=out_dtype)
     # products of few tiles (a skinny operand, a long K) are split along K when there is room for the partial sums;
     # shapes whose operand rows are not whole 16-byte chunks run on zero-padded copies in the workspace
-    need = _gemm_workspace.get((M, N, K))
+    need = _gemm_workspace.get((M, N, K, ta, tb, 2))
     if need is None:
-        need = _ask_workspace("lego_hip_gemm_workspace_bytes", _gemm_workspace, (M, N, K))
+        need = _ask_workspace("lego_hip_gemm_layout_workspace_bytes", _gemm_workspace, (M, N, K, ta, tb, 2))
     if need:
         workspace = torch.empty(need // 4, dtype=torch.float32, device=a.device)
         element = 0 if a.dtype == torch.float16 else 4 if out_dtype == torch.float16 else 1

@@ -45,6 +45,7 @@ SIGNATURES = {
     "lego_hip_gemm_bf16_f16_ex": [_c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                                   _c_void_p],
     "lego_hip_gemm_workspace_bytes": [_c_int, _c_int, _c_int, ctypes.POINTER(ctypes.c_ulonglong)],
+    "lego_hip_gemm_layout_workspace_bytes": [_c_int] * 6 + [ctypes.POINTER(ctypes.c_ulonglong)],
     "lego_hip_gemm_ex_ws": [_c_int, _c_void_p, _c_void_p, _c_void_p, _c_int, _c_int, _c_int, _c_int, _c_int, _c_int,
                             _c_void_p, ctypes.c_ulonglong, _c_void_p],
     "lego_hip_gemm_fp8_workspace_bytes": [_c_int, _c_int, _c_int, ctypes.POINTER(ctypes.c_ulonglong)],

@@ -65,3 +65,20 @@ def test_gpu_row_past_the_matrix_reaches_nothing():
     c = torch.full((M * N + 256,), 7.0, dtype=torch.float16, device="cuda")
     runtime.call("lego_hip_gemm_f16_ex", ap, bp, c.data_ptr() + 256, M, N, K, 0, 1, 0, None)
     assert (c[128:128 + M * N] == K).all() and (c[:128] == 7).all() and (c[128 + M * N:] == 7).all()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float8_e5m2])
+def test_gpu_few_rows_allocate_the_result_alone(dtype):
+    """No room for partial sums that the kernel for few rows does not form; the same product against a row-major B still has it."""
+    from lego_amd import ops
+    print(f"gemm rows, memory, {dtype}", flush=True)
+    a, b = torch.zeros(16, 4096, device="cuda").to(dtype), torch.zeros(4096, 4096, device="cuda").to(dtype)
+
+    def peak(b):
+        before = torch.cuda.memory_allocated()
+        torch.cuda.reset_peak_memory_stats()
+        c = ops.matmul(a, b)
+        del c
+        return torch.cuda.max_memory_allocated() - before
+    assert peak(b.t()) == 2 * 16 * 4096 < peak(b)
