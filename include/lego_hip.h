@@ -198,11 +198,11 @@ int lego_hip_stencil_f32_plan(int n, int radius, int star, int bricks, int* plan
  * Two block steps of 64 per pair of launches, all on `stream`; nothing is kept between calls. */
 int lego_hip_lud_f32(float* m, int n, void* stream);
 
-/* What lego_hip_lud_f32 does to an n x n matrix in blocks of 64, in order, without touching a device: six ints per
- * record, {kind, 0, a, b, c, d}; a launch does one or more of them.
- *   kind 0 panels of step a (b blocks each);  1 block row and column a+1 against step a (b = blocks left in
- *   a block row);  3 trailing update of the square of side c from block b on against d/16 steps from a on (d%16 is 1);
- *   6 factors of the a diagonal blocks written.
+/* The launches of lego_hip_lud_f32 for an n x n matrix in blocks of 64, in order, without touching a device: seven ints per
+ * launch, {kind, workgroups, s, steps, q, side, run}, all as the launch itself has them.
+ *   kind 0: the first diagonal block, of `side` blocks a side, is factored;  1: the panels of the block steps s .. s+steps-1 are solved, q blocks
+ *   each beyond the diagonal block;  2: the square of side q behind them is updated against these steps, by the first workgroup the diagonal block of
+ *   the next `side` steps, which it factors too, by the others the rest in runs of `run` block rows of two block columns.
  * At most `capacity` records are written; *count receives how many there are.  No counterpart in the
  * reference (its host loop, lud_kernel_temp.cu:358-390, is three launches per step on one stream): it is
  * there so that the order of the work can be checked on the host. */

@@ -23,10 +23,7 @@ from .common import BANNER, Emitted, code, idx, size, template, tidy
 
 B, T, R = 64, 16, 4
 P = 2 * B      # two block steps between two passes over the trailing square
-# side (in blocks) of the trailing square from which the next panels are solved on a second stream meanwhile: none, the
-# trailing launch itself factors ahead (a matrix has at most 512 blocks a side)
-AHEAD_MIN = 512
-# the trailing square is walked in groups of up to GROUP block rows, column by column inside a group (the grouped launch
+# the trailing square is walked in groups of up to GROUP block rows, two block columns at a time inside a group (the grouped launch
 # order of the reference's matmul, matmul_sympy.py:57-65), and each of the XCDS L2 caches gets a contiguous run of it
 GROUP, XCDS, CUS = 8, 8, 256
 

@@ -52,122 +52,101 @@ def test_coarsening_places_every_block_element_once():
 
 
 def _plan(n):
-    """The launches of lego_hip_lud_f32 for an n x n matrix, as the library's own schedule records them."""
+    """The launches of lego_hip_lud_f32 for an n x n matrix: (kind, workgroups, s, steps, q, side, run) each."""
     import ctypes
     from lego_amd import runtime
     count = ctypes.c_int(0)
     runtime.call("lego_hip_lud_f32_plan", n, None, 0, ctypes.byref(count))
-    buf = (ctypes.c_int * (6 * count.value))()
+    buf = (ctypes.c_int * (7 * count.value))()
     runtime.call("lego_hip_lud_f32_plan", n, buf, count.value, ctypes.byref(count))
-    return [tuple(buf[6 * i:6 * i + 6]) for i in range(count.value)]
+    return [tuple(buf[7 * i:7 * i + 7]) for i in range(count.value)]
 
 
-def _replay(nb, plan):
-    """Replays a recorded schedule on block indices: every launch finds its inputs final, every block gets each
-    earlier step exactly once and in order, and what runs between a fork and the next join on the two streams
-    touches disjoint blocks (write/write and read/write).  Returns how many forks there were."""
-    applied = {(i, j): [] for i in range(nb) for j in range(nb)}
-    solved = {}
-
-    def update(block, steps, writes, reads):
-        i, j = block
-        assert block not in solved and block not in writes, block
-        for st in steps:
-            assert solved.get((i, st)) == st and solved.get((st, j)) == st, (block, st)
-            applied[block].append(st)
-            reads |= {(i, st), (st, j)}
-        writes.add(block)
-
-    forks, open_main, open_side = 0, None, None
-    for kind, stream, a, b, c, d in plan:
-        writes, reads = set(), set()
-        if kind == 0:       # panels of step a, b workgroups
-            assert b == nb - 1 - a
-            assert applied[(a, a)] == list(range(a))
-            reads.add((a, a))
-            for w in range(b):
-                for block in ((a, a + 1 + w), (a + 1 + w, a)):
-                    assert applied[block] == list(range(a)) and block not in solved, block
-                    solved[block] = a
-                    writes.add(block)
-        elif kind == 1:     # block row and column a+1 against step a
-            assert b == nb - 1 - a
-            for w in range(2 * b - 1):
-                update((a + 1, a + 1 + w) if w < b else (a + 2 + w - b, a + 1), [a], writes, reads)
-        elif kind == 2:     # two block rows and columns of the square of side c from block b on
-            for w in range(4 * c - 4):
-                block = (b + w // c, b + w % c) if w < 2 * c else (b + 2 + (w - 2 * c) // 2, b + (w - 2 * c) % 2)
-                update(block, [a, a + 1], writes, reads)
-        elif kind == 3:     # the square of side c from block b on
-            depth, run = d // 16, d % 16
-            assert run in (1, 2, 4, 8) and b + c == nb
-            for i in range(c):
-                for j in range(c):
-                    update((b + i, b + j), list(range(a, a + depth)), writes, reads)
-        elif kind == 4:
-            assert open_main is None
-            forks, open_main, open_side = forks + 1, (set(), set()), (set(), set())
-            continue
-        elif kind == 5:
-            assert open_main is not None
-            (mw, mr), (sw, sr) = open_main, open_side
-            assert not (mw & sw) and not (mw & sr) and not (mr & sw)
-            open_main = open_side = None
-            continue
-        else:
-            assert kind == 6 and a == nb and open_main is None
-            continue
-        if open_main is None:
-            assert stream == 0            # the side stream is only used between a fork and a join
-        else:
-            side = open_side if stream == 1 else open_main
-            side[0].update(writes)
-            side[1].update(reads)
-    assert open_main is None and plan[-1][0] == 6
-    for (i, j), steps in applied.items():
-        assert steps == list(range(min(i, j))), (i, j)
-    for i in range(nb):
-        for j in range(nb):
-            if i != j:
-                assert solved[(i, j)] == min(i, j)
-    return forks
+@pytest.mark.parametrize("nb", list(range(1, 14)) + [63, 64, 76, 77, 78, 79, 100, 129, 256, 511, 512])
+def test_launches_take_every_block_through_every_step_once(nb):
+    """What each launch reads is final when it starts, and every block has every step before its own once.  Panels of `steps` steps apply
+    the earlier of them to the later by substitution; the diagonal block that a launch factors is the next launch's."""
+    plan = _plan(64 * nb)
+    kind, workgroups, _, _, _, side, _ = plan[0]
+    assert (kind, workgroups) == (0, 1) and 1 <= side <= min(2, nb)
+    done, factored = 0, side               # steps applied to all blocks behind them; side of the factored diagonal block at `done`
+    for panels, trailing in zip(plan[1::2], plan[2::2]):
+        kind, workgroups, s, steps, q, _, _ = panels
+        assert kind == 1 and (s, steps) == (done, factored) and s + steps + q == nb and q > 0
+        assert workgroups * 2 * 16 == 64 * q                 # two wavefronts of sixteen columns, and two of sixteen rows
+        kind, workgroups, s2, steps2, q2, side, run = trailing
+        assert kind == 2 and (s2, steps2, q2) == (s, steps, q) and 1 <= side <= min(2, q) and 1 <= run <= lud_gen.GROUP
+        done, factored = done + steps, side
+        if q > side:
+            assert (workgroups - 1) % lud_gen.XCDS == 0 and workgroups - 1 >= -(-q // run) * -(-q // 2)
+    assert len(plan) % 2 == 1 and done + factored == nb
 
 
-@pytest.mark.parametrize("nb", list(range(1, 12)) + [63, 64, 76, 77, 78, 79, 100, 129, 256])
-def test_launch_order_updates_every_block_in_order_and_overlaps_only_disjoint_work(nb):
-    forks = _replay(nb, _plan(64 * nb))
-    assert (forks > 0) == (nb >= lud_gen.AHEAD_MIN + 5)
+_WALK = """
+#include <cstdio>
+#include <cstdlib>
+#include <vector>
+#define __host__
+#define __device__
+#define __forceinline__ inline
+%(code)s
+// every block of the square by one workgroup: the first has the diagonal block of `side` blocks, and beside a single one its neighbour
+bool covered_once(unsigned q, unsigned run, unsigned side, unsigned workgroups)
+{
+  std::vector<int> seen(q * q, 0);
+  for (unsigned r = 0; r < side; ++r) for (unsigned c = 0; c < 2 && c < q; ++c) ++seen[r * q + c];
+  for (unsigned wg = 0; wg + 1 < workgroups; ++wg) {
+    unsigned from = 0, to = 0, pair = 0;
+    if (!part_of(wg, workgroups - 1, q, run, side, from, to, pair)) continue;
+    if (to > q || to - from > run || 2 * pair >= q) return false;
+    for (unsigned r = from; r < to; ++r) for (unsigned c = 2 * pair; c < 2 * pair + 2 && c < q; ++c) ++seen[r * q + c];
+  }
+  for (int s : seen) if (s != 1) return false;
+  return true;
+}
+int main()
+{
+  for (unsigned q = 1; q <= 510; q = q < 40 ? q + 1 : q * 9 / 8) {
+    const unsigned chosen = trailing_rows(q);
+    if (chosen < 1 || chosen > %(group)d) return 1;
+    for (unsigned run = 1; run <= %(group)d; ++run)
+      for (unsigned side = 1; side <= 2 && side <= q; ++side)
+        if (!covered_once(q, run, side, trailing_grid(q, run))) { std::printf("q %%u run %%u side %%u\\n", q, run, side); return 2; }
+  }
+  return 0;
+}
+"""
 
 
-def test_trailing_walk_covers_the_square_once():
-    """The walk of the trailing update (groups of GROUP block rows, a column of a group in parts of `run` blocks)
-    after the remap onto the XCDs: the layouts that print the kernel's index expressions, evaluated for every
-    workgroup of the padded grid, give every block of a q x q square to exactly one workgroup, and one XCD
-    (every XCDS-th workgroup id) gets a contiguous piece of the walk."""
+def test_trailing_launch_covers_the_square_once(tmp_path):
+    """The decomposition of the trailing update as the generator prints it, compiled for the host: for squares of 1 to 510 blocks and every
+    length of run, each block is one workgroup's, the first one's part left out of the others'."""
+    import re
+    import subprocess
+    from pathlib import Path
+    text = (Path(__file__).resolve().parents[1] / "lego_amd" / "csrc" / "generated" / "lud_f32.hip").read_text()
+    code = "\n".join(re.search(p + r".*?\n}\n", text, re.S).group(0) for p in (
+        r"__host__ __device__ __forceinline__ bool part_of\(", r"inline unsigned trailing_rows\(", r"inline unsigned trailing_grid\("))
+    src = tmp_path / "walk.cpp"
+    src.write_text(_WALK % {"code": code, "group": lud_gen.GROUP})
+    subprocess.run(["g++", "-std=c++17", "-O1", str(src), "-o", str(tmp_path / "walk")], check=True)
+    res = subprocess.run([str(tmp_path / "walk")], capture_output=True, text=True)
+    assert res.returncode == 0, res.stdout
+
+
+def test_trailing_walk_gives_each_xcd_a_contiguous_piece():
+    """The layouts that print the kernel's index expressions: positions of the walk in group-major order, pairs of block columns inside a
+    group, and for every XCD (every XCDS-th workgroup id) consecutive ones."""
     import sympy as sp
-    ng, q, nsub, per, pid, wg = sp.symbols("ng q nsub per pid wg", integer=True, nonnegative=True)
-    order = sp.lambdify([ng, q, nsub, pid], lud_gen.block_order(ng, q, nsub, pid), "math")
+    ng, q2, per, pid, wg = sp.symbols("ng q2 per pid wg", integer=True, nonnegative=True)
+    order = sp.lambdify([ng, q2, pid], lud_gen.block_order(ng, q2, 1, pid), "math")
     remap = sp.lambdify([per, wg], lud_gen.xcd_remap(per, wg), "math")
-    G, X = lud_gen.GROUP, lud_gen.XCDS
-    for side in (1, 2, 7, 8, 9, 31, 64, 75, 124):
-        for run in (1, 2, 4, 8):
-            groups, parts = -(-side // G), G // run
-            positions = groups * side * parts
-            grid = -(-positions // X) * X
-            seen, by_xcd = set(), {}
-            for w in range(grid):
-                pos = int(remap(grid // X, w))
-                by_xcd.setdefault(w % X, []).append(pos)
-                if pos >= positions:
-                    continue
-                g, c, part = (int(v) for v in order(groups, side, parts, pos))
-                first = G * g + run * part
-                for r in range(first, min(first + run, side)):
-                    assert 0 <= c < side and (r, c) not in seen
-                    seen.add((r, c))
-            assert len(seen) == side * side, (side, run)
-            for x, got in by_xcd.items():
-                assert got == list(range(x * (grid // X), (x + 1) * (grid // X)))
+    X = lud_gen.XCDS
+    for groups, pairs in ((1, 1), (3, 2), (8, 31), (16, 62)):
+        assert [tuple(int(v) for v in order(groups, pairs, p)) for p in range(groups * pairs)] == [(g, c, 0) for g in range(groups) for c in range(pairs)]
+    for pieces in (1, 2, 31):
+        for x in range(X):
+            assert [int(remap(pieces, w)) for w in range(x, X * pieces, X)] == list(range(x * pieces, (x + 1) * pieces))
 
 
 @pytest.mark.gpu
@@ -186,13 +165,44 @@ def test_gpu_matches_oracle(n):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [192, 320, 576, 1088, 1152])
-def test_gpu_odd_block_counts_and_run_lengths(n):
-    """A last block that is no pair, a second column of blocks past the matrix, runs of one and more block rows with a short
-    last one: the factors against the oracle's, each rounded some n times at the size of the pivots."""
+def test_gpu_odd_block_counts(n):
+    """A last block that is no pair, a second column of blocks past the matrix: the factors against the oracle's, each rounded some n
+    times at the size of the pivots."""
     from lego_amd import ops
     print(f"lud n={n}", flush=True)
     a = _dominant(n, 300 + n).astype(np.float32)
     want = ok.lud(a)
+    got = ops.lud(torch.from_numpy(a.copy()).cuda()).cpu().numpy().astype(np.float64)
+    assert np.linalg.norm(got - want) <= n * 2.0 ** -24 * np.linalg.norm(want)
+    assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
+
+
+def _lud_by_blocks(a, b=128):
+    """The oracle's elimination on diagonal blocks, triangular solves and products in 64 bits around them."""
+    m = np.array(a, dtype=np.float64)
+    for k in range(0, len(m), b):
+        e = min(k + b, len(m))
+        m[k:e, k:e] = ok.lud(m[k:e, k:e])
+        m[k:e, e:] = scipy.linalg.solve_triangular(m[k:e, k:e], m[k:e, e:], lower=True, unit_diagonal=True)
+        m[e:, k:e] = scipy.linalg.solve_triangular(m[k:e, k:e], m[e:, k:e].T, trans=1).T
+        m[e:, e:] -= m[e:, k:e] @ m[k:e, e:]
+    return m
+
+
+def test_oracle_by_blocks_is_the_oracle():
+    a = _dominant(300, 4)
+    assert np.allclose(_lud_by_blocks(a, 64), ok.lud(a), rtol=1e-12, atol=1e-11)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n,runs", [(1600, {1, 2}), (2624, {1, 2, 3, 4}), (4160, {1, 2, 3, 4, 5, 6, 7, 8})])
+def test_gpu_run_lengths(n, runs):
+    """Trailing squares whose workgroups take runs of several block rows, the last ones short: bounds as for the odd block counts."""
+    from lego_amd import ops
+    print(f"lud n={n}", flush=True)
+    assert {record[6] for record in _plan(n) if record[0] == 2} == runs
+    a = _dominant(n, 500 + n).astype(np.float32)
+    want = _lud_by_blocks(a)
     got = ops.lud(torch.from_numpy(a.copy()).cuda()).cpu().numpy().astype(np.float64)
     assert np.linalg.norm(got - want) <= n * 2.0 ** -24 * np.linalg.norm(want)
     assert np.abs(got - want).max() <= 2e-5 * np.abs(want).max()
@@ -209,8 +219,7 @@ def test_gpu_rejects_bad_sizes():
 @pytest.mark.gpu
 @pytest.mark.parametrize("n", [4928, 8256, 16384, 32768])
 def test_gpu_large_matrix_reproduces_its_factors(n):
-    """Sizes at which the panels of the next pair of steps are solved on a second stream (77 and 129 blocks: odd
-    counts, the first the smallest that does), n = 16384, the largest size the reference publishes, and n = 32768, the
+    """77 and 129 blocks, odd counts, n = 16384, the largest size the reference publishes, and n = 32768, the
     largest the entry point takes (a 4 GiB matrix: offsets beyond 32 bits): L*U gives the
     matrix back (fp32, diagonally dominant)."""
     from lego_amd import ops
@@ -226,11 +235,9 @@ def test_gpu_large_matrix_reproduces_its_factors(n):
 
 
 @pytest.mark.gpu
-def test_gpu_call_with_second_stream_replays_from_a_hip_graph():
-    """At n = 8256 the call forks to a second stream of the library and joins it back with events; captured into a
-    graph on a stream that an eager call has used before (which made that stream's side stream), every replay
-    gives the bits of the eager result, with eager work and synchronisation between the replays.  Captured on a
-    stream the library has never seen, the call creates nothing and stays on the one stream: same bits."""
+def test_gpu_call_replays_from_a_hip_graph():
+    """Captured into a graph, on a stream that an eager call has used before and on a new one, every replay
+    gives the bits of the eager result, with eager work and synchronisation between the replays."""
     from lego_amd import ops
     print("lud n=8256 captured into a graph", flush=True)
     n = 8256
@@ -247,7 +254,7 @@ def test_gpu_call_with_second_stream_replays_from_a_hip_graph():
         ops.lud(w)                       # warm-up on a side stream, outside the capture
     torch.cuda.current_stream().wait_stream(side)
     torch.cuda.synchronize()
-    for capture_stream in (side, torch.cuda.Stream()):      # known to the library / never seen by it
+    for capture_stream in (side, torch.cuda.Stream()):
         graph = torch.cuda.CUDAGraph()
         with torch.cuda.graph(graph, stream=capture_stream):
             ops.lud(w)
