@@ -80,6 +80,7 @@ def test_launches_take_every_block_through_every_step_once(nb):
         if q > side:
             assert (workgroups - 1) % lud_gen.XCDS == 0 and workgroups - 1 >= -(-q // run) * -(-q // 2)
     assert len(plan) % 2 == 1 and done + factored == nb
+    assert factored == min(2, nb)          # a single block at the end would wait for panels of two steps
 
 
 _WALK = """
