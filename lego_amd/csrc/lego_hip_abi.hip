@@ -271,35 +271,49 @@ typedef unsigned u32x4w_any __attribute__((ext_vector_type(4), aligned(1)));    
 // Matrices on their way into, or out of, copies whose rows are whole 16-byte chunks on a 16-byte aligned base: up to kCopies of them
 // in one launch, told apart by the running total of workgroups (a launch of its own for each took 2-3 us, more than most of the
 // copies themselves).  One lane per 16-byte chunk; a chunk that lies inside the matrix as a whole is one access on either side.
-constexpr int kCopies = 64;
+// The list is kernel arguments, and the largest is 3 KB of them, a microsecond of each launch: a single product's copies, and those of a few,
+// have lists of their own.  Where a workgroup belongs takes one round of scalar loads of the list's totals, and none of a list of two (640 x
+// 1439 x 64, B and the result copied, with one list of 64 searched entry by entry 13.9 us, 13.4).
+constexpr int kCopies = 64, kSomeCopies = 12, kFewCopies = 2;
 struct Copy {
   const void* from;
   void* to;
   unsigned rows, row_bytes;        // of the matrix as it is
   unsigned rows_to, pitch;         // of the copy: rows beyond `rows` and bytes beyond `row_bytes` are zeros
-  unsigned end;                    // workgroups up to and including this one
+  unsigned first;                  // workgroup of the launch
 };
+template <int MAX>
 struct Copies {
-  Copy of[kCopies];
-  int count;
+  unsigned end[MAX];               // workgroups up to and including each one; ~0 past the last
+  Copy of[MAX];
 };
+static_assert(sizeof(Copies<kFewCopies>) <= 128, "what a single product's copies add to a launch");
 
-template <bool PAD>
-__global__ void __launch_bounds__(256) lego_copies_kernel(const Copies copies)
+template <bool PAD, int MAX>
+__global__ void __launch_bounds__(256) lego_copies_kernel(const Copies<MAX> copies)
 {
-  int i = 0;
-  while (i + 1 < copies.count && blockIdx.x >= copies.of[i].end) ++i;      // the same for the whole workgroup
-  const Copy c = copies.of[i];
-  const size_t chunk = static_cast<size_t>(blockIdx.x - (i ? copies.of[i - 1].end : 0u)) * 256 + threadIdx.x;
-  const unsigned per_row = c.pitch / 16, at = static_cast<unsigned>(chunk % per_row) * 16;
+  Copy c;      // the same for the whole workgroup
+  if constexpr (MAX == 2) {
+    c = copies.of[0];
+    const Copy& d = copies.of[1];
+    if (blockIdx.x >= copies.end[0]) c = d;
+  } else {
+    int i = 0;
+#pragma unroll
+    for (int j = 0; j + 1 < MAX; ++j) i += blockIdx.x >= copies.end[j] ? 1 : 0;
+    c = copies.of[i];
+  }
+  const unsigned chunk = (blockIdx.x - c.first) * 256 + threadIdx.x;      // of less than 2^32, as a launch has lanes
+  const unsigned per_row = c.pitch / 16, at = chunk % per_row * 16;
   const size_t r = chunk / per_row;
   if (PAD) {
     if (r >= c.rows_to) return;
     u32x4w v = {0u, 0u, 0u, 0u};
     if (r < c.rows && at < c.row_bytes) {
-      const uint8_t* p = static_cast<const uint8_t*>(c.from) + r * c.row_bytes + at;
+      const size_t offset = r * c.row_bytes + at;
+      const uint8_t* p = static_cast<const uint8_t*>(c.from) + offset;
       const unsigned valid = c.row_bytes - at;
-      if ((c.rows - r) * c.row_bytes - at >= 16) {      // the matrix has sixteen bytes from here on, this row's or the next one's
+      if (offset + 16 <= static_cast<size_t>(c.rows) * c.row_bytes) {      // the matrix has sixteen bytes from here on, this row's or the next one's
         v = *reinterpret_cast<const u32x4w_any*>(p);
 #pragma unroll
         for (unsigned e = 0; e < 4; ++e)
@@ -328,32 +342,47 @@ __global__ void __launch_bounds__(256) lego_copies_kernel(const Copies copies)
 // Collects copies of matrices that lie one after the other in a workspace and enqueues them, kCopies at a time.
 class Copier {
  public:
-  Copier(bool pad, hipStream_t stream) : pad_(pad), stream_(stream) { copies_.count = 0; }
+  Copier(bool pad, hipStream_t stream) : pad_(pad), stream_(stream) {}
   // rows x cols elements of `bytes` bytes each, copied to (pad) or from (otherwise) rows of cols_to elements
   void add(const void* from, void* to, long rows, long cols, long rows_to, long cols_to, int bytes)
   {
-    if (copies_.count == kCopies) (void)flush();      // its error is kept
+    if (count_ == kCopies) (void)flush();      // its error is kept
     const unsigned long long chunks = static_cast<unsigned long long>(pad_ ? rows_to : rows) * (cols_to * bytes / 16);
-    const unsigned before = copies_.count ? copies_.of[copies_.count - 1].end : 0u;
-    copies_.of[copies_.count++] = {from, to, static_cast<unsigned>(rows), static_cast<unsigned>(cols * bytes), static_cast<unsigned>(rows_to),
-                                   static_cast<unsigned>(cols_to * bytes), before + static_cast<unsigned>((chunks + 255) / 256)};
+    copies_[count_++] = {from, to, static_cast<unsigned>(rows), static_cast<unsigned>(cols * bytes), static_cast<unsigned>(rows_to),
+                            static_cast<unsigned>(cols_to * bytes), workgroups_};
+    workgroups_ += static_cast<unsigned>((chunks + 255) / 256);
   }
   hipError_t flush()
   {
-    if (copies_.count == 0) return err_;
-    const dim3 grid(copies_.of[copies_.count - 1].end);
-    if (pad_) hipLaunchKernelGGL(lego_copies_kernel<true>, grid, dim3(256), 0, stream_, copies_);
-    else hipLaunchKernelGGL(lego_copies_kernel<false>, grid, dim3(256), 0, stream_, copies_);
-    copies_.count = 0;
+    if (count_ == 0) return err_;
+    if (count_ <= kFewCopies) launch<kFewCopies>();
+    else if (count_ <= kSomeCopies) launch<kSomeCopies>();
+    else launch<kCopies>();
+    count_ = 0;
+    workgroups_ = 0;
     const hipError_t e = hipGetLastError();
     if (err_ == hipSuccess) err_ = e;
     return err_;
   }
 
  private:
+  template <int MAX>
+  void launch()
+  {
+    Copies<MAX> list;
+    for (int i = 0; i < MAX; ++i) {
+      list.of[i] = copies_[i < count_ ? i : 0];
+      list.end[i] = i + 1 < count_ ? copies_[i + 1].first : ~0u;
+    }
+    if (pad_) hipLaunchKernelGGL((lego_copies_kernel<true, MAX>), dim3(workgroups_), dim3(256), 0, stream_, list);
+    else hipLaunchKernelGGL((lego_copies_kernel<false, MAX>), dim3(workgroups_), dim3(256), 0, stream_, list);
+  }
+
   bool pad_;
   hipStream_t stream_;
-  Copies copies_;
+  Copy copies_[kCopies];
+  int count_ = 0;
+  unsigned workgroups_ = 0;
   hipError_t err_ = hipSuccess;
 };
 
