@@ -259,10 +259,11 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     if out_dtype not in (torch.float16, a.dtype):
         raise ValueError("out_dtype must be float16 or the operands' type")
     entry = "lego_hip_gemm_bf16_f16_ex" if (a.dtype, out_dtype) == (torch.bfloat16, torch.float16) else _GEMM_ENTRY[a.dtype]
-    if ta and M % 8 and (M * K >= 65536 or (K >= 384 and not (N % 8 or K % 8))):
+    if ta and M % 8 and (M * K >= 65536 or (K >= 384 and not (N % 8 or K % 8)) or (tb and M <= 16 and N >= 1024 and 1400 <= K <= 1984)):
         # a column-major A whose columns (M elements) are not whole 16-byte chunks is outside the tiled kernels unless the product
         # runs on copies anyway: store it row-major first (one pass with the transpose kernels; by elements / row-major first:
-        # 33 x 256 x 256 13 / 15 us, 7 x 512 x 512 22 / 16, 3 x 1024 x 8192 323 / 19; where copies take it, 5 x 8192 x 8191 75, 72 without)
+        # 33 x 256 x 256 13 / 15 us, 7 x 512 x 512 22 / 16, 3 x 1024 x 8192 323 / 19).  Where copies take it as well: first for the kernel for
+        # few rows where the chain of K is long and not yet split (2 x 2049 x 801 20 / 26, 1602 29 / 26, 1922 33 / 26, 2102 23 / 27)
         a_store, ta = transpose(a_store), 0
     c = torch.empty((M, N), device=a.device, dtype=out_dtype)
     # products of few tiles (a skinny operand, a long K) are split along K when there is room for the partial sums;

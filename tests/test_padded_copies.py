@@ -85,7 +85,8 @@ def test_gpu_8bit_products_of_any_shape(fp8, M, N, K):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K,transposed_first", [(5, 520, 1023, False), (5, 521, 1024, False), (5, 520, 1024, True), (67, 520, 1023, True), (5, 520, 376, False)])
+@pytest.mark.parametrize("M,N,K,transposed_first", [(5, 520, 1023, False), (5, 521, 1024, False), (5, 520, 1024, True), (67, 520, 1023, True), (5, 520, 376, False), (5, 1030, 1601, True),
+                                                      (5, 1030, 1201, False), (5, 1030, 2101, False), (5, 520, 1601, False)])
 def test_gpu_column_major_rows_of_no_whole_chunks(M, N, K, transposed_first, monkeypatch):
     """A small column-major A is stored row-major first where the product would run by elements, not where copies take it."""
     from lego_amd import ops
@@ -95,7 +96,7 @@ def test_gpu_column_major_rows_of_no_whole_chunks(M, N, K, transposed_first, mon
     g = torch.Generator().manual_seed(M + N + K)
     a = torch.randint(-1, 2, (M, K), generator=g).half()
     b = torch.randint(-1, 2, (K, N), generator=g).half()
-    got = ops.matmul(a.t().contiguous().cuda().t(), b.cuda())
+    got = ops.matmul(a.t().contiguous().cuda().t(), b.t().contiguous().cuda().t() if N > 1024 else b.cuda())
     assert torch.equal(got.cpu().float(), a.float() @ b.float()) and bool(calls) == transposed_first
 
 
