@@ -195,11 +195,12 @@ int lego_hip_stencil_f32_plan(int n, int radius, int star, int bricks, int* plan
  * strict lower triangle holds L (unit diagonal implied) and the upper triangle holds U, as
  * Rodinia's lud (the reference's thread-coarsening benchmark: benchmarks/cuda/lud.py:5-12,
  * kernels lud/lud_kernel_temp.cu:14-352, host loop :358-390).  n a multiple of 64, at most 32768.
- * Two block steps of 64 per pair of launches, all on `stream`; nothing is kept between calls. */
+ * Two block steps of 64 per pair of launches (one, before the last two, where their number is odd), all on `stream`; nothing is kept
+ * between calls. */
 int lego_hip_lud_f32(float* m, int n, void* stream);
 
-/* The launches of lego_hip_lud_f32 for an n x n matrix in blocks of 64, in order, without touching a device: seven ints per
- * launch, {kind, workgroups, s, steps, q, side, run}, all as the launch itself has them.
+/* The launches of lego_hip_lud_f32 for an n x n matrix in blocks of 64, in order, without touching a device: six ints per
+ * launch, {kind, workgroups, s, steps, side, run}, all as the launch itself has them; q = n/64 - s - steps blocks a side lie behind the steps.
  *   kind 0: the first diagonal block, of `side` blocks a side, is factored;  1: the panels of the block steps s .. s+steps-1 are solved, q blocks
  *   each beyond the diagonal block;  2: the square of side q behind them is updated against these steps, by the first workgroup the diagonal block of
  *   the next `side` steps, which it factors too, by the others the rest in runs of `run` block rows of two block columns.

@@ -817,7 +817,7 @@ typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int,
 // elements; the padding adds zeros to the sums) and the result is copied back: two more launches and three more passes over
 // the matrices, against the kernel that moves one element per access and whose chain of k-tiles is long.  8-bit operands, us by
 // elements / on copies: 320 x 1984 x 7959 829 / 35, 2000 x 2000 x 2001 276 / 27, 5000 x 3001 x 136 93 / 32, 6902 x 192 x 296 31 / 28, 1000 x
-// 1000 x 264 27 / 25, 33 x 100 x 200 16 / 23, 1000 x 1000 x 136 16 / 22: copies from K = 256 on, or from as many 64 x 64 tiles of the
+// 1001 x 264 38 / 14, 16 x 65 x 257 20 / 16, 33 x 100 x 200 16 / 23, 1000 x 1000 x 136 16 / 22: copies from K = 256 on, or from as many 64 x 64 tiles of the
 // result as keep the one-element kernel busy for 30 us.
 inline bool copies_gain_8bit(int M, int N, int K)
 {

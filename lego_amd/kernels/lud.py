@@ -14,7 +14,7 @@ in the ``n x n`` matrix are those of ``OrderBy(Row(n, n)).TileBy([n/64, n/64], [
 product itself runs on the fp32 matrix cores, whose accumulator layout is one more LEGO
 expression (``Row(4, 2, 4)``).  Block steps go in pairs: one launch solves the panels of both against a factored 128 x 128
 diagonal block, the next one updates the trailing blocks while its first workgroup factors the diagonal block of the next
-pair, in 16 x 16 tiles.
+pair, in 16 x 16 tiles.  Of an odd number of steps the one before the last two is by itself.
 """
 from __future__ import annotations
 

@@ -52,14 +52,14 @@ def test_coarsening_places_every_block_element_once():
 
 
 def _plan(n):
-    """The launches of lego_hip_lud_f32 for an n x n matrix: (kind, workgroups, s, steps, q, side, run) each."""
+    """The launches of lego_hip_lud_f32 for an n x n matrix: (kind, workgroups, s, steps, side, run) each."""
     import ctypes
     from lego_amd import runtime
     count = ctypes.c_int(0)
     runtime.call("lego_hip_lud_f32_plan", n, None, 0, ctypes.byref(count))
-    buf = (ctypes.c_int * (7 * count.value))()
+    buf = (ctypes.c_int * (6 * count.value))()
     runtime.call("lego_hip_lud_f32_plan", n, buf, count.value, ctypes.byref(count))
-    return [tuple(buf[7 * i:7 * i + 7]) for i in range(count.value)]
+    return [tuple(buf[6 * i:6 * i + 6]) for i in range(count.value)]
 
 
 @pytest.mark.parametrize("nb", list(range(1, 14)) + [63, 64, 76, 77, 78, 79, 100, 129, 256, 511, 512])
@@ -67,15 +67,16 @@ def test_launches_take_every_block_through_every_step_once(nb):
     """What each launch reads is final when it starts, and every block has every step before its own once.  Panels of `steps` steps apply
     the earlier of them to the later by substitution; the diagonal block that a launch factors is the next launch's."""
     plan = _plan(64 * nb)
-    kind, workgroups, _, _, _, side, _ = plan[0]
+    kind, workgroups, _, _, side, _ = plan[0]
     assert (kind, workgroups) == (0, 1) and 1 <= side <= min(2, nb)
     done, factored = 0, side               # steps applied to all blocks behind them; side of the factored diagonal block at `done`
     for panels, trailing in zip(plan[1::2], plan[2::2]):
-        kind, workgroups, s, steps, q, _, _ = panels
-        assert kind == 1 and (s, steps) == (done, factored) and s + steps + q == nb and q > 0
+        kind, workgroups, s, steps, _, _ = panels
+        q = nb - s - steps
+        assert kind == 1 and (s, steps) == (done, factored) and q > 0
         assert workgroups * 2 * 16 == 64 * q                 # two wavefronts of sixteen columns, and two of sixteen rows
-        kind, workgroups, s2, steps2, q2, side, run = trailing
-        assert kind == 2 and (s2, steps2, q2) == (s, steps, q) and 1 <= side <= min(2, q) and 1 <= run <= lud_gen.GROUP
+        kind, workgroups, s2, steps2, side, run = trailing
+        assert kind == 2 and (s2, steps2) == (s, steps) and 1 <= side <= min(2, q) and 1 <= run <= lud_gen.GROUP
         done, factored = done + steps, side
         if q > side:
             assert (workgroups - 1) % lud_gen.XCDS == 0 and workgroups - 1 >= -(-q // run) * -(-q // 2)
@@ -201,7 +202,7 @@ def test_gpu_run_lengths(n, runs):
     """Trailing squares whose workgroups take runs of several block rows, the last ones short: bounds as for the odd block counts."""
     from lego_amd import ops
     print(f"lud n={n}", flush=True)
-    assert {record[6] for record in _plan(n) if record[0] == 2} == runs
+    assert {record[5] for record in _plan(n) if record[0] == 2} == runs
     a = _dominant(n, 500 + n).astype(np.float32)
     want = _lud_by_blocks(a)
     got = ops.lud(torch.from_numpy(a.copy()).cuda()).cpu().numpy().astype(np.float64)
