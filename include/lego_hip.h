@@ -138,7 +138,8 @@ int lego_hip_gemm_bf16_f16_ex(const void* a, const void* b, void* c, int M, int 
  * fixed order (deterministic), applies the activation and stores C.  A product with N or K that is not a multiple
  * of 8 (operand rows that are not whole 16-byte chunks) runs on zero-padded copies of A, B and C in the workspace
  * instead of the one-element-per-access kernel, about ten times as fast; operands may then start at any element.
- * lego_hip_gemm_workspace_bytes gives the size the call uses for a shape (0: it gains nothing from a workspace).
+ * lego_hip_gemm_workspace_bytes gives room for all that the call uses for a shape, shallow products aside (0: none of 32 k-tiles and
+ * more, and no copies); lego_hip_gemm_layout_workspace_bytes gives what it uses.
  * The workspace is scratch: 16-byte aligned device memory, contents undefined on entry and exit, not to be shared
  * by calls that may overlap.  With a null or short workspace the call is lego_hip_gemm_*_ex.  No counterpart in
  * the reference, whose matmul has one program per tile (matmul_sympy.py:57-65). */
@@ -153,8 +154,7 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
 int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                          int activation, int format, void* stream);
 /* The same product with room for partial sums: a product of few tiles is split along K as lego_hip_gemm_ex_ws does it.
- * lego_hip_gemm_fp8_workspace_bytes gives the size the call uses for a shape (0: it stays whole); the workspace as
- * there.  With a null or short workspace, or a layout whose rows are not whole 16-byte chunks, the call is
+ * lego_hip_gemm_fp8_workspace_bytes gives room for it (as there); the workspace as there.  With a null or short workspace, or a layout whose rows are not whole 16-byte chunks, the call is
  * lego_hip_gemm_fp8_ex. */
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes);
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
@@ -284,6 +284,11 @@ int lego_hip_gemm_rows_plan(int M, int N, int K, int trans_a, int trans_b, int e
  * autotuner picks among tile configurations at run time, matmul_sympy.py:98-165); it is there so that the choice can be
  * checked on the host. */
 int lego_hip_gemm_plan(int M, int N, int K, int* plan2);
+
+/* For a product of that kind, of element_bytes = 1 or 2 per operand element: plan2[0] = parts along K, with room for their sums (1: none),
+ * plan2[1] = operand buffers of a workgroup in LDS: 4 (one workgroup per CU), or, of 128 x 128 tiles beyond one per CU and of all 256 x 256
+ * ones, 2.  Host only. */
+int lego_hip_gemm_parts_plan(int M, int N, int K, int element_bytes, int* plan2);
 
 /* The team that lego_hip_softmax_f16 and lego_hip_layernorm_fwd_f16 give a row of a matrix of M rows of N fp16
  * elements in whole 16-byte vectors on 16-byte aligned bases (N a multiple of 8, at most 32768): waves per row, the

@@ -158,8 +158,13 @@ def collect():
                 # 256x256 tiles to fill the chip
                 gs, _ = gemm.emit(**dict(GEMM, bk=GEMM_BK[dtype], bm=GEMM_SMALL_TILE, bn=GEMM_SMALL_TILE),
                                   trans_a=ta, trans_b=tb, dtype=dtype,
-                                  with_grouped=dtype == "f16" and not (ta or tb), with_splitk=True)
+                                  with_grouped=dtype == "f16" and not (ta or tb))
                 units.append(gs)
+                # ... and on four buffers of LDS, one workgroup per CU: for up to as many tiles, or parts of tiles along K, as there are CUs
+                gd, _ = gemm.emit(**dict(GEMM, bk=GEMM_BK[dtype], bm=GEMM_SMALL_TILE, bn=GEMM_SMALL_TILE),
+                                  trans_a=ta, trans_b=tb, dtype=dtype,
+                                  with_grouped=dtype == "f16" and not (ta or tb), suffix="_deep", stages=4, with_splitk=True)
+                units.append(gd)
     # The 256 x 256 tile on 32 x 32 accumulator blocks (v_mfma_f32_32x32x16), four waves of 128 x 128: behind at the
     # socket's power limit (8192^3: 1.29 against 1.36 PFLOP/s) and ahead away from it, so launches of one round that
     # leaves a third of the CUs idle take it (kSparseRoundBelow in lego_hip_abi.hip); the fp16 build for operands as
@@ -263,13 +268,15 @@ def collect():
           f"#define LEGO_LAYERNORM_BWD_MAX_N {mlb['MAX_N']}", ""]
     h += [f"hipError_t lego_gemm_{d}_{v}{t}_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);"
           for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")
-          for t in ("", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}")]
-    h += [f"hipError_t lego_gemm_{d}_{v}_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_splitk_launch(const void*, const void*, void*, int, int, int, int, "
+          for t in ("", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep")]
+    h += [f"hipError_t lego_gemm_{d}_{v}_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep_splitk_launch(const void*, const void*, void*, int, int, int, int, "
           "int, float*, hipStream_t);" for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")]
     h += [
           "hipError_t lego_grouped_gemm_f16_launch(const void* const*, const void* const*, void* const*, "
           "const int*, int, hipStream_t);",
           f"hipError_t lego_grouped_gemm_f16_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_launch(const void* const*, "
+          "const void* const*, void* const*, const int*, int, hipStream_t);",
+          f"hipError_t lego_grouped_gemm_f16_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep_launch(const void* const*, "
           "const void* const*, void* const*, const int*, int, hipStream_t);",
           "hipError_t lego_gemm_f16_nn_w2x4_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);",
           *[f"hipError_t lego_gemm_{d}_{v}_m32_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);"

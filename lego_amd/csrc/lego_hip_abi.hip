@@ -690,6 +690,7 @@ typedef hipError_t (*gemm_launcher)(const void*, const void*, void*, int, int, i
 struct GemmKernels {
   gemm_launcher big[4];     // 256 x 256 tiles, one workgroup per CU; index 2*trans_a + trans_b
   gemm_launcher small[4];   // 128 x 128 tiles, two workgroups per CU (null: not built for this type)
+  gemm_launcher deep[4];    // 128 x 128 tiles on four buffers of LDS, one workgroup per CU
   gemm_launcher sparse[4];  // 256 x 256 tiles on 32x32x16 MFMAs, for launches that leave many CUs idle (null: not built for this type)
 };
 // Fewer 256 x 256 tiles than this and the 128 x 128 kernel, with four times as many workgroups,
@@ -759,6 +760,18 @@ inline int rows_columns(int M, int N, int K, int trans_a, int trans_b, int bytes
   return best;
 }
 
+// Up to one 128 x 128 tile per CU runs on four buffers of LDS instead of two workgroups of two: what bounds such a launch is how far ahead
+// of a workgroup's k-tiles its operands are asked for.  us, two buffers / four, operands from memory (from the caches): e5m2 1000 x
+// 2048 x 2048 18.0 / 12.9 (10.4 / 9.1), fp16 2048^3 (256 tiles) 31.4 / 22.7 (25.3 / 20.1), 256 x 4096 x 1024 16.4 / 11.6 (8.6 / 8.5), 64 x 2800 x 128
+// 4.2 / 4.0.  Beyond, two workgroups per CU are ahead: 2304 x 2048 x 2048 (288 tiles) 32.5 / 35.3, 4096 x 2048 x 2048 42.6 / 44.5, 2496 x 2944 x 512
+// 14.9 / 22.5.  A lane's offset within a tile stays below a descriptor's 2 GiB.
+constexpr long kDeepTiles = 256;
+inline bool deep_offsets(int M, int N, int K, int bytes) { return 128l * bytes * std::max(M, std::max(N, K)) < (1l << 31); }
+inline bool deep_tiles(int M, int N, int K, int bytes)
+{
+  return static_cast<long>((M + 127) / 128) * ((N + 127) / 128) <= kDeepTiles && deep_offsets(M, N, K, bytes);
+}
+
 int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, void* c, int M, int N, int K,
             int trans_a, int trans_b, int activation, void* stream, int bk = LEGO_GEMM_BK, int chunk = 8)
 {
@@ -783,35 +796,33 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
     return ok_or(lego_gemm_rows_launch(a, b, c, M, N, K, columns, activation, element, as_stream(stream)));
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
   const int choice = gemm_choice(M, N, k.small[layout] != nullptr, k.sparse[layout] != nullptr);
-  const gemm_launcher* by_layout = choice == 1 ? k.small : choice == 2 ? k.sparse : k.big;
+  const gemm_launcher* by_layout = choice == 1 && deep_tiles(M, N, K, 16 / chunk) ? k.deep : choice == 1 ? k.small : choice == 2 ? k.sparse : k.big;
   return ok_or(by_layout[layout](a, b, c, M, N, K, activation, as_stream(stream)));
 }
 
-// Parts along K for a product of few tiles (1: one workgroup per tile does it all): enough parts for two
-// workgroups of 128 x 128 tiles per CU, at least four k-tiles each.  The second launch and the partial sums cost
-// about what 16 k-tiles take, so shallower products stay whole (1024^3: 8.6 us whole, 11.7 in four parts;
-// 512 x 512 x 2048: 13.7 whole, 8.2 in eight).  More workgroups also keep more loads in flight, so parts gain most where operands come
-// from memory, whatever the size of the result.  us whole / in parts, fp16, operands from memory, and in brackets from the
-// caches: 1024 x 1536 x 2048 27.5 / 26.2 (21.3 / 24.0), 1024 x 2048 x 3584 49.4 / 32.7 (34.8 / 30.8), 384 x 5120 x 3072 43.3 / 39.1 (30.6 /
-// 34.1), 256 x 8192 x 2304 33.2 / 28.1 (24.3 / 25.3), 8192 x 256 x 3584 49.1 / 34.5 (36.0 / 28.7), 1496 x 1144 x 3024 50.6 / 36.9 (38.9 / 35.7);
-// over 87 products of 2 to 4 tiles' worth of result per k-tile parts take 0.86 of the time from memory, 1.01 from the caches.
-// 8-bit operands are half as many bytes beside the same sums: a product whose result is more than two tiles' worth of
-// elements per k-tile stays whole, 21.6 against 24.3 from the caches at 384 x 4096 x 4096 with B transposed (28.4 / 26.7 from memory),
-// 24.1 / 27.6 at 4608 deep; below, k-tiles of 128: 16 x 8192 x 8192 41.4 / 18.0, 64 x 4096 x 4096 22.3 / 12.7, 256 x 256 x 16384 71.7 / 12.8,
-// 1024 x 1024 x 4096 21.7 / 18.8.
+// Parts along K for a product of few tiles (1: one workgroup per tile does it all): as many as the estimate of the launch's time is least
+// for, one round of workgroups of two k-tiles each at least.  In ns, whole 2400 + 420 per k-tile; parts 5200, the second launch in it, 420
+// per k-tile of a part, and the sums of every part, 24 for a tile's worth of them and 4 for each workgroup.  Fitted to 90 drawn products of up
+// to 128 tiles in each number of parts: the rule takes 1.016 times the best of them with operands from memory, 1.014 from the caches.  us
+// from memory (from the caches), whole / parts: fp16 512 x 512 x 512 5.8 / two 6.8, 512 x 512 x 1024 8.4 / four 7.4, 1024^3 9.0 / two 10.6, 1024 x 2048 x 3584
+// 35.0 (24.5) / two 29.0 (27.0), 1024 x 1024 x 4096 36.0 (24.8) / three 20.9 (18.4), four 20.7 (19.6), six, more than a round, 26.4 (23.5); 16 x 8192 x 8192
+// 54.6 / three 27.7, four 29.0; e5m2 1000 x 2048 x 2048 12.9 / two 15.2, 256 x 2048 x 4096 22.0 / four 12.5; e4m3 1024 x 1024 x 4096 19.6 / three 14.7.
 int splitk_parts(int M, int N, int K, int bk)
 {
   const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
-  if (tiles > 128 || depth < 32) return 1;
-  if (bk == LEGO_GEMM_BK_8BIT && static_cast<long>(M) * N > 2 * depth * 128 * 128) return 1;
-  long parts = (512 + tiles - 1) / tiles;
-  if (parts > depth / 4) parts = depth / 4;
-  if (parts > 64) parts = 64;
-  return parts < 2 ? 1 : static_cast<int>(parts);
+  if (tiles > kDeepTiles / 2 || !deep_offsets(M, N, K, 2 * LEGO_GEMM_BK / bk)) return 1;
+  const long most = std::min(std::min(kDeepTiles / tiles, depth / 2), 64l);
+  long best = 1, least = 2400 + 420 * depth;
+  for (long parts = 2; parts <= most; ++parts) {
+    const long sums = 24l * M * N / (128 * 128) + 4 * tiles;
+    const long time = 5200 + parts * sums + 420 * ((depth + parts - 1) / parts);
+    if (time < least) { best = parts; least = time; }
+  }
+  return static_cast<int>(best);
 }
 typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int, int, int, int, float*, hipStream_t);
-#define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_splitk_launch, lego_gemm_##DT##_nt_t128x128_splitk_launch, \
-                         lego_gemm_##DT##_tn_t128x128_splitk_launch, lego_gemm_##DT##_tt_t128x128_splitk_launch}
+#define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_deep_splitk_launch, lego_gemm_##DT##_nt_t128x128_deep_splitk_launch, \
+                         lego_gemm_##DT##_tn_t128x128_deep_splitk_launch, lego_gemm_##DT##_tt_t128x128_deep_splitk_launch}
 
 // Operand rows that are not whole 16-byte chunks: the tiled kernels run on zero-padded copies (every side a multiple of `chunk`
 // elements; the padding adds zeros to the sums) and the result is copied back: two more launches and three more passes over
@@ -868,12 +879,16 @@ int on_padded_copies(int chunk, int bytes, const void* a, const void* b, void* c
     lego_gemm_##DT##_tt_launch},                                                                       \
    {lego_gemm_##DT##_nn_t128x128_launch, lego_gemm_##DT##_nt_t128x128_launch,                         \
     lego_gemm_##DT##_tn_t128x128_launch, lego_gemm_##DT##_tt_t128x128_launch},                         \
+   {lego_gemm_##DT##_nn_t128x128_deep_launch, lego_gemm_##DT##_nt_t128x128_deep_launch,               \
+    lego_gemm_##DT##_tn_t128x128_deep_launch, lego_gemm_##DT##_tt_t128x128_deep_launch},               \
    {nullptr, nullptr, nullptr, nullptr}}
 #define LEGO_GEMM_KERNELS(DT)                                                                          \
   {{lego_gemm_##DT##_nn_launch, lego_gemm_##DT##_nt_launch, lego_gemm_##DT##_tn_launch,              \
     lego_gemm_##DT##_tt_launch},                                                                       \
    {lego_gemm_##DT##_nn_t128x128_launch, lego_gemm_##DT##_nt_t128x128_launch,                         \
     lego_gemm_##DT##_tn_t128x128_launch, lego_gemm_##DT##_tt_t128x128_launch},                         \
+   {lego_gemm_##DT##_nn_t128x128_deep_launch, lego_gemm_##DT##_nt_t128x128_deep_launch,               \
+    lego_gemm_##DT##_tn_t128x128_deep_launch, lego_gemm_##DT##_tt_t128x128_deep_launch},               \
    {lego_gemm_##DT##_nn_m32_launch, lego_gemm_##DT##_nt_m32_launch, lego_gemm_##DT##_tn_m32_launch,  \
     lego_gemm_##DT##_tt_m32_launch}}
 }  // namespace
@@ -899,17 +914,34 @@ int lego_hip_gemm_bf16_f16_ex(const void* a, const void* b, void* c, int M, int 
   return gemm_ex(k, 4, a, b, c, M, N, K, trans_a, trans_b, activation, stream);
 }
 
-int lego_hip_gemm_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
+namespace {
+// Room that a product of this kind uses: for zero-padded copies of both operands and of the result, N or K not being a multiple of 8 (M only
+// matters as the row length of a transposed A; that case alone stays with the one-element kernel), and for its sums, `parts(M, N, K)` of them.
+extern "C++" template <class Parts>
+unsigned long long room_16bit(int M, int N, int K, const Parts& parts)
 {
-  if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
-  // N or K not a multiple of 8: room for zero-padded copies of both operands and of the result.
-  // (M only matters as the row length of a transposed A; that case alone stays with the one-element kernel.)
   unsigned long long copies = 0;
   if (N % 8 || K % 8) {
     copies = padded_bytes(M, N, K, 8, 2);
     M = round_up(M, 8); N = round_up(N, 8); K = round_up(K, 8);     // the product that then runs
   }
-  *bytes = copies + parts_bytes(M, N, splitk_parts(M, N, K, LEGO_GEMM_BK));
+  return copies + parts_bytes(M, N, parts(M, N, K));
+}
+// What the entry points that know no layout ask for where there are no copies: the products they split are those of 32 k-tiles and more, of 8-bit operands those of up to two
+// tiles' worth of the result per k-tile.
+int stated_parts(int M, int N, int K, int bk)
+{
+  const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
+  if (tiles > kDeepTiles / 2 || depth < 32 || (bk == LEGO_GEMM_BK_8BIT && static_cast<long>(M) * N > 2 * depth * 128 * 128)) return 1;
+  return std::max(2, splitk_parts(M, N, K, bk));
+}
+}  // namespace
+
+int lego_hip_gemm_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
+{
+  if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
+  const bool copied = N % 8 || K % 8;
+  *bytes = room_16bit(M, N, K, [=](int m, int n, int k) { return (copied ? splitk_parts : stated_parts)(m, n, k, LEGO_GEMM_BK); });
   return 0;
 }
 
@@ -926,13 +958,12 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
       default: return lego_hip_gemm_bf16_f16_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, stream);
     }
   };
-  unsigned long long need = 0;
-  if (lego_hip_gemm_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
+  if (M <= 0 || N <= 0 || K <= 0) return kInvalid;
+  const unsigned long long need = room_16bit(M, N, K, [](int m, int n, int k) { return splitk_parts(m, n, k, LEGO_GEMM_BK); });
   if (need == 0 || workspace_bytes < need || !usable(workspace)) return whole(a, b, c, M, N, K);
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 8 == 0 && (trans_a ? M % 8 == 0 : K % 8 == 0) &&
                      (!trans_b || K % 8 == 0);
-  const bool copies = N % 8 || K % 8;      // and room for them
-  if (!tiled && !copies) return whole(a, b, c, M, N, K);
+  if (!tiled && N % 8 == 0 && K % 8 == 0) return whole(a, b, c, M, N, K);
   if (a == nullptr || b == nullptr || c == nullptr || (activation != 0 && activation != 1)) return kInvalid;
   if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
   const auto product = [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
@@ -958,7 +989,7 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0) return kInvalid;
-  *bytes = parts_bytes(M, N, N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT));
+  *bytes = parts_bytes(M, N, N % 16 ? 1 : stated_parts(M, N, K, LEGO_GEMM_BK_8BIT));
   return 0;
 }
 
@@ -973,26 +1004,28 @@ const splitk_launcher* fp8_parts(int format)
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream)
 {
-  unsigned long long need = 0;
-  if ((format != 0 && format != 1) || lego_hip_gemm_fp8_workspace_bytes(M, N, K, &need) != 0) return kInvalid;
+  if ((format != 0 && format != 1) || M <= 0 || N <= 0 || K <= 0) return kInvalid;
   const bool tiled = usable(a) && usable(b) && usable(c) && N % 16 == 0 && (trans_a ? M % 16 == 0 : K % 16 == 0) &&
                      (!trans_b || K % 16 == 0);
-  if (need == 0 || !tiled || !usable(workspace) || workspace_bytes < need || rows_columns(M, N, K, trans_a, trans_b, 1))
+  const int parts = splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT);
+  if (parts < 2 || !tiled || !usable(workspace) || workspace_bytes < parts_bytes(M, N, parts) || rows_columns(M, N, K, trans_a, trans_b, 1))
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
   const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
-  return ok_or(fp8_parts(format)[layout](a, b, c, M, N, K, activation, splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT),
-                                         static_cast<float*>(workspace), as_stream(stream)));
+  return ok_or(fp8_parts(format)[layout](a, b, c, M, N, K, activation, parts, static_cast<float*>(workspace), as_stream(stream)));
 }
 
-// The same sizes for operands of one layout: the kernel for few rows takes some of these products and needs no room for sums.
+// What is used for operands of one layout, shallow products that gain from parts among them; the kernel for few rows takes some and needs no
+// room for sums.
 int lego_hip_gemm_layout_workspace_bytes(int M, int N, int K, int trans_a, int trans_b, int element_bytes, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
   const int chunk = 16 / element_bytes;
   *bytes = 0;
   if (N % chunk == 0 && K % chunk == 0 && rows_columns(M, N, K, trans_a, trans_b, element_bytes)) return 0;
-  return (element_bytes == 1 ? lego_hip_gemm_fp8_workspace_bytes : lego_hip_gemm_workspace_bytes)(M, N, K, bytes);
+  if (element_bytes == 1) *bytes = parts_bytes(M, N, N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT));
+  else *bytes = room_16bit(M, N, K, [](int m, int n, int k) { return splitk_parts(m, n, k, LEGO_GEMM_BK); });
+  return 0;
 }
 
 // Whether a product whose rows are not whole 16-byte chunks gains from copies that are; room for these and for the sums of their product.
@@ -1170,7 +1203,7 @@ double grouped_makespan(const long* count, const double* cost, int batches, long
 }
 
 // What a grouped call launches: the kernel on 256 x 256 tiles with the last `split` tiles of its launch
-// order as two 128 x 256 halves each (kind 0), or the kernel on 128 x 128 tiles (kind 1).
+// order as two 128 x 256 halves each (kind 0), or the kernel on 128 x 128 tiles, two workgroups per CU (kind 1) or one (kind 2).
 struct GroupedPlan {
   int kind, tiles, split;
   double time;      // the estimate that chose it, in the units below
@@ -1179,8 +1212,11 @@ struct GroupedPlan {
 // Costs in units of one k-tile step of a 256 x 256 tile that has its CU to itself (about 1.8 us for
 // fp16), measured on MI355X: a tile pays a start-up and an epilogue on top of its steps (31.4 us for
 // 16 steps); a 128 x 256 half-tile takes 19.2 us for 16 steps; a 128 x 128 tile sharing its CU with
-// another one takes 0.66 of a whole tile of the same depth.
-constexpr double kTileOverhead = 1.6, kHalfStep = 0.58, kHalfOverhead = 1.5, kSmallCost = 0.66;
+// another one takes 0.66 of a whole tile of the same depth.  One on four buffers, alone on its CU, takes 0.38 of a step
+// per k-tile and two steps beside them: the choice between the two so estimated takes 1.0005 times the better one over 72
+// drawn calls of 1 to 16 problems (us, two workgroups per CU / one: 112 x 120 x 2816 and 128 x 184 x 512 30.5 / 19.7; 16 problems, 546 tiles of up to
+// 57 k-tiles, 68 / 45; nine of 565 tiles 71 / 52; 13 of 1056 tiles, deep ones among them in every round, 80 / 91; 14 of 762 tiles of up to 12 k-tiles 25.6 / 28.0).
+constexpr double kTileOverhead = 1.6, kHalfStep = 0.58, kHalfOverhead = 1.5, kSmallCost = 0.66, kDeepStep = 0.38, kDeepOverhead = 2.0;
 // Problems per call.  A launch carries its pointers and sizes as kernel arguments, LEGO_GROUPED_MAX_GROUPS problems
 // at most; a call with more is enqueued as several launches (below).
 constexpr int kGroupedMaxProblems = 1 << 20;
@@ -1197,8 +1233,9 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
     order[j] = o;
   }
   long big[LEGO_GROUPED_MAX_GROUPS], small[LEGO_GROUPED_MAX_GROUPS];
-  double depth[LEGO_GROUPED_MAX_GROUPS], small_cost[LEGO_GROUPED_MAX_GROUPS];
+  double depth[LEGO_GROUPED_MAX_GROUPS], small_cost[LEGO_GROUPED_MAX_GROUPS], deep_cost[LEGO_GROUPED_MAX_GROUPS];
   long total = 0;
+  bool deep = true;
   for (int s = 0; s < groups; ++s) {
     const int g = order[s];
     const int m = sizes3[3 * g], n = sizes3[3 * g + 1];
@@ -1206,6 +1243,8 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
     small[s] = static_cast<long>((m + 127) / 128) * ((n + 127) / 128);
     depth[s] = (sizes3[3 * g + 2] + LEGO_GEMM_BK - 1) / LEGO_GEMM_BK;
     small_cost[s] = kSmallCost * (depth[s] + kTileOverhead);
+    deep_cost[s] = kDeepStep * depth[s] + kDeepOverhead;
+    deep = deep && deep_offsets(m, n, sizes3[3 * g + 2], 2);
     total += big[s];
   }
   const long cus = 256;                 // MI355X
@@ -1235,10 +1274,11 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
     if (split == 0 || t <= best) { best = t; best_split = split; }
   }
   const double t_small = grouped_makespan(small, small_cost, groups, 2 * cus);
-  plan.kind = t_small < best ? 1 : 0;
+  const double t_deep = deep ? grouped_makespan(small, deep_cost, groups, cus) : t_small;
+  plan.kind = t_deep < t_small && t_deep < best ? 2 : t_small < best ? 1 : 0;
   plan.tiles = static_cast<int>(total);
   plan.split = plan.kind == 0 ? static_cast<int>(best_split) : 0;
-  plan.time = plan.kind == 1 ? t_small : best;
+  plan.time = plan.kind == 2 ? t_deep : plan.kind == 1 ? t_small : best;
   return plan;
 }
 
@@ -1342,18 +1382,17 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
   // depth, so the longest tiles start first.  (Splitting the problems over both tile sizes in two
   // launches was measured and never beat the better single launch.)
   const GroupedPlan plan = grouped_plan(sizes3, groups);
+  if (plan.kind == 2) return ok_or(lego_grouped_gemm_f16_t128x128_deep_launch(a, b, c, sizes3, groups, as_stream(stream)));
   if (plan.kind == 1) return ok_or(lego_grouped_gemm_f16_t128x128_launch(a, b, c, sizes3, groups, as_stream(stream)));
   if (plan.split == 0) return ok_or(lego_grouped_gemm_f16_launch(a, b, c, sizes3, groups, as_stream(stream)));
   return ok_or(lego_grouped_gemm_f16_split_launch(a, b, c, sizes3, groups, plan.split, as_stream(stream)));
 }
 
-// Ragged problems that a single product splits along K (more than 31 k-tiles): in the grouped launch they are chains of whole depth,
-// apart each is some four launches more.  Apart, then, where the launch without them is estimated shorter by more than 14 steps for
-// each and twice what it is of a step of the whole chip, and 2.5 for each of up to eight others, whose calls are enqueued all the same.  Us, together / apart: 64 x 64 x 4095 beside three of 64^3
-// 44 / 32, 512 x 512 x 4095 beside four of 512^3 50 / 35; 64 x 64 x 4095 beside sixteen of 1024^3 68 / 64, which the estimate keeps
-// together as it does 512 x 512 x 2577 beside eight of 512^3, 42 / 44; four of 64 x 64 x 4095 48 / 61, eight of 3001 x 2999 x
-// 3003 562 / 669.  Over 9831 drawn calls of 2 to 16 problems the rule takes 1.013 times the better of the two, all apart 1.19, all
-// together 1.11, by the number of problems 1.10.
+// Ragged problems that a single product splits along K: in the grouped launch they are chains of whole depth, apart each is some four
+// launches more.  Apart, then, where the launch without them is estimated shorter by more than 20 steps for each and twice what it is of a step of
+// the whole chip.  Us with what the host adds, together / apart: 64 x 64 x 4095 beside one of 64^3 31 / 28, beside two 32 / 32 (beside fifteen, which
+// the estimate cannot tell, 65 / 74), 512 x 512 x 4095 beside two of 512^3 36 / 34, which stay together, and beside eight 44 / 53; 64 x 64 x 2577 beside eight of
+// 1024^3 44 / 52, four of 64 x 64 x 4095 35 / 66.  Over 90 drawn calls with such problems the rule, and all together, take the better of the two.
 int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) try
 {
   if (sizes3 == nullptr || apart == nullptr || groups <= 0 || groups > kGroupedMaxProblems) return kInvalid;
@@ -1375,13 +1414,13 @@ int lego_hip_grouped_gemm_f16_apart(const int* sizes3, int groups, int* apart) t
     memcpy(all + 3 * i, size, sizeof(size));
     if (ragged && k > 31 * LEGO_GEMM_BK) {
       deep[deeps++] = g;
-      alone += 14.0 + 2.0 * m * n * k / (256.0 * 256 * 256 * LEGO_GEMM_BK);
+      alone += 20.0 + 2.0 * m * n * k / (256.0 * 256 * 256 * LEGO_GEMM_BK);
     } else {
       memcpy(rest + 3 * others++, size, sizeof(size));
     }
   }
   if (deeps == 0) return 0;
-  const double without = others ? grouped_plan(rest, others).time + 2.5 * (groups - 1 < 8 ? groups - 1 : 8) : 0.0;
+  const double without = others ? grouped_plan(rest, others).time : 0.0;
   if (grouped_plan(all, count).time > without + alone)
     for (int i = 0; i < deeps; ++i) apart[deep[i]] = 1;
   return 0;
@@ -1492,6 +1531,14 @@ int lego_hip_gemm_plan(int M, int N, int K, int* plan2)
   return 0;
 }
 
+int lego_hip_gemm_parts_plan(int M, int N, int K, int element_bytes, int* plan2)
+{
+  if (plan2 == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
+  plan2[0] = splitk_parts(M, N, K, element_bytes == 1 ? LEGO_GEMM_BK_8BIT : LEGO_GEMM_BK);
+  plan2[1] = plan2[0] > 1 || deep_tiles(M, N, K, element_bytes) ? 4 : 2;
+  return 0;
+}
+
 int lego_hip_gemm_rows_plan(int M, int N, int K, int trans_a, int trans_b, int element_bytes, int* columns)
 {
   if (columns == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
@@ -1505,7 +1552,7 @@ int lego_hip_grouped_gemm_f16_plan(const int* sizes3, int groups, int* plan3)
   for (int g = 0; g < groups; ++g)
     if (sizes3[3 * g] <= 0 || sizes3[3 * g + 1] <= 0 || sizes3[3 * g + 2] <= 0) return kInvalid;
   const GroupedPlan plan = grouped_plan(sizes3, groups);
-  plan3[0] = plan.kind == 1 ? 128 : 256;
+  plan3[0] = plan.kind == 0 ? 256 : 128;
   plan3[1] = plan.tiles;
   plan3[2] = plan.split;
   return 0;
@@ -1525,7 +1572,7 @@ int lego_hip_grouped_gemm_f16_stamps(const void* const* a, const void* const* b,
 {
   if (groups > LEGO_GROUPED_MAX_GROUPS || grouped_check(a, b, c, sizes3, groups) != 0) return kInvalid;
   const GroupedPlan plan = grouped_plan(sizes3, groups);
-  if (plan.kind == 1) return kInvalid;        // the measurement build exists for the 256 x 256 tiles only
+  if (plan.kind != 0) return kInvalid;        // the measurement build exists for the 256 x 256 tiles only
   if (plan.split == 0) return ok_or(lego_grouped_gemm_f16_stamps_launch(a, b, c, sizes3, groups, as_stream(stream)));
   return ok_or(lego_grouped_gemm_f16_stamps_split_launch(a, b, c, sizes3, groups, plan.split, as_stream(stream)));
 }

@@ -15,6 +15,8 @@ and then applies the grouped launch order inside that problem.
 """
 from __future__ import annotations
 
+import functools
+
 import sympy as sp
 
 from ..lego import BitXor, Col, GenP, OrderBy, Row
@@ -235,19 +237,32 @@ def last_ktile_schedule(TM, TN, NPH, WN, block=32, mps=1):
     return slots, tail
 
 
-def _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped, dtype, block=32, suffix="", stamps=False):
+_DTYPES = {"f16": ("_Float16", 2, "_Float16"), "bf16": ("__bf16", 2, "__bf16"), "bf16h": ("__bf16", 2, "_Float16"),
+           "e4m3": ("unsigned char", 1, "_Float16"), "e5m2": ("unsigned char", 1, "_Float16")}
+
+
+def _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped, dtype, block=32, suffix="", stamps=False, stages=2):
     """Everything the templates need for one tile shape.  ``block``: 32 = v_mfma_f32_32x32x16 (x64 for 8-bit operands),
-    16 = v_mfma_f32_16x16x32 (16-bit operands), the side of an accumulator block."""
-    # element type, bytes per element, k-depth of one MFMA, result type; the 8-bit types are the
+    16 = v_mfma_f32_16x16x32 (16-bit operands), the side of an accumulator block.  ``stages``: operand buffers in LDS."""
+    # element type, bytes per element, result type; the 8-bit types are the
     # OCP formats of v_mfma_f32_32x32x64_f8f6f4 (format code 0 = e4m3, 1 = e5m2)
     # "bf16h": bfloat16 operands with the fp16 result that the reference's matmul stores whatever its
     # operands' 16-bit type (matmul_sympy.py:129-145, 203)
-    elt, esize, mfma_k, out_elt = {"f16": ("_Float16", 2, 16, "_Float16"), "bf16": ("__bf16", 2, 16, "__bf16"),
-                                   "bf16h": ("__bf16", 2, 16, "_Float16"),
-                                   "e4m3": ("unsigned char", 1, 64, "_Float16"),
-                                   "e5m2": ("unsigned char", 1, 64, "_Float16")}[dtype]
-    EPC = 16 // esize                      # elements per 16-byte chunk
+    elt, esize, out_elt = _DTYPES[dtype]
     assert not (with_grouped and dtype != "f16"), "the grouped kernel is built for fp16 only"
+    variant = ("t" if trans_a else "n") + ("t" if trans_b else "n")
+    tag = ("" if (bm, bn) == (256, 256) else f"_t{bm}x{bn}") + ("" if tuple(waves) == (2, 2) else f"_w{waves[0]}x{waves[1]}") + suffix
+    return dict(_tile_geometry(bm, bn, bk, tuple(waves), max_group_m, trans_a, trans_b, esize, block),
+                banner=BANNER, elt=elt, out_elt=out_elt, FMT={"e4m3": 0, "e5m2": 1}.get(dtype, 0), dt=dtype,
+                mfma_dt={"bf16h": "bf16"}.get(dtype, dtype), variant=variant, tag=tag, with_grouped=with_grouped,
+                STAMPS=stamps, STAMP_ROWS=STAMP_ROWS, STAGES=stages)
+
+
+@functools.lru_cache(maxsize=None)
+def _tile_geometry(bm, bn, bk, waves, max_group_m, trans_a, trans_b, esize, block):
+    """The part of ``_tile_params`` that the layouts give, the same for all types of ``esize`` bytes."""
+    mfma_k = 16 if esize == 2 else 64
+    EPC = 16 // esize                      # elements per 16-byte chunk
     assert block in (32, 16) and (block == 32 or esize == 2)
     if block == 16:
         mfma_k = 32
@@ -455,16 +470,12 @@ def _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped,
                 f"{role}_kstep": code(sp.simplify(full.subs(k, k + 1) - full)),
                 f"{role}_frag_code": frag}
 
-    variant = ("t" if trans_a else "n") + ("t" if trans_b else "n")
-    tag = ("" if (bm, bn) == (256, 256) else f"_t{bm}x{bn}") + ("" if tuple(waves) == (2, 2) else f"_w{WAVES_M}x{WAVES_N}") + suffix
-    chunk_params = dict(WAVES=WAVES, variant=variant, tag=tag, with_grouped=with_grouped, **operand("a"), **operand("b"))
-
     shared = _rows_per_key(bn, 4 if esize == 2 else 8)
     params = dict(
         KEY="k%8" if shared == 1 else f"(k/{shared})%{8 // shared}",      # of an 8-bit [bk][bn] tile (lds_b_layout)
-        banner=BANNER, elt=elt, out_elt=out_elt, ESIZE=esize, EPC=EPC, MFMA_K=mfma_k, NPH=NPH,
-        FMT={"e4m3": 0, "e5m2": 1}.get(dtype, 0), dt=dtype, mfma_dt={"bf16h": "bf16"}.get(dtype, dtype), BM=bm, BN=bn, BK=bk, THREADS=THREADS, WAVES_M=WAVES_M, WAVES_N=WAVES_N,
-        WM=WM, WN=WN, TM=TM, TN=TN, A_ITERS=A_ITERS, B_ITERS=B_ITERS, DMA_LAST=DMA_LAST,
+        ESIZE=esize, EPC=EPC, MFMA_K=mfma_k, NPH=NPH,
+        BM=bm, BN=bn, BK=bk, THREADS=THREADS, WAVES_M=WAVES_M, WAVES_N=WAVES_N,
+        WM=WM, WN=WN, TM=TM, TN=TN, A_ITERS=A_ITERS, B_ITERS=B_ITERS, DMA_LAST=DMA_LAST, COPIES=COPIES,
         # s_waitcnt immediate: vmcnt in bits 3:0 and 15:14, expcnt and lgkmcnt left at their maxima
         WAIT_DMA_LAST="0x%04X" % (0x0F70 | (DMA_LAST % 16) | ((DMA_LAST // 16) << 14)),
         load_slots=load_slots, dma_last=dma_last, dma_first=dma_first, dma_none=none, XCDS=XCDS, MAX_GROUPS=MAX_GROUPS,
@@ -478,14 +489,14 @@ def _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped,
         c_layout=f"OrderBy(Row(M,N)).TileBy([M/{bm},N/{bn}],[{bm},{bn}])",
         wm=code(wm_e), wn=code(wn_e),
         # offset of a chunk = tile base (uniform) + position inside k-tile 0 (per lane) + k * step
-        **chunk_params,
+        WAVES=WAVES, **operand("a"), **operand("b"),
         # accumulator -> staging: row i*32 + l32, 8-byte chunk (j*32 + q*8 + lhi*4)/4 of the wave's block
         c_stage_store=code(stage_e),
         # staging -> memory: lane reads the pair of chunks (2p, 2p+1) of row cr; the XOR keeps a
         # pair together and (32 x 32 blocks) swaps its halves on odd rows
         c_out_row=code(c_out[0]), c_out_pair=code(c_out[1]),
         c_stage_load=code(tidy(4 * Cs_L[cr, 2 * cp], rng) - (4 * (cr % 2) if block == 32 else 0)),
-        BLOCK=block, MPS=MPS, ACC_REGS=block * block // 64, SWAP_ODD_ROWS=block == 32, STAMPS=stamps, STAMP_ROWS=STAMP_ROWS,
+        BLOCK=block, MPS=MPS, ACC_REGS=block * block // 64, SWAP_ODD_ROWS=block == 32,
         c_goff=code(tidy(C_L[pid_m, pid_n, wm * WM + cr, wn * WN + 8 * cp], rng)),
         c_stage_lane=code(stage_lane), c_back_lane=code(back_lane),
         c_wave=code(c_wave_e), c_lane=code(c_lane_e), c_it_step=code(c_it_e),
@@ -518,7 +529,7 @@ def split_order(split, wg):
 
 
 def emit(bm=256, bn=256, bk=64, waves=(2, 2), max_group_m=8, trans_a=False, trans_b=False, with_grouped=True,
-         dtype="f16", with_split=False, with_splitk=False, block=32, suffix="", stamps=False):
+         dtype="f16", with_split=False, with_splitk=False, block=32, suffix="", stamps=False, stages=2):
     """One translation unit: the GEMM kernel of one operand layout and element type on ``bm x bn``
     tiles, with ``with_grouped`` the grouped kernel on the same tiles, and with ``with_split`` a
     second grouped kernel that gives the last tiles of its launch to two workgroups each, as
@@ -527,7 +538,7 @@ def emit(bm=256, bn=256, bk=64, waves=(2, 2), max_group_m=8, trans_a=False, tran
     the names of the file and the launchers (a second build of one shape); ``stamps``: a measurement build whose
     workgroups record the real-time counter at fixed points of their tile (``lego_gemm_stamps_read``)."""
     assert not (with_splitk and block != 32), "partial sums along K are laid out for 32 x 32 accumulator blocks"
-    params = _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped, dtype, block, suffix, stamps)
+    params = _tile_params(bm, bn, bk, waves, max_group_m, trans_a, trans_b, with_grouped, dtype, block, suffix, stamps, stages)
     ns = f"t{bm}x{bn}"
     tiles = [dict(ns=ns, text=template("gemm_tile.hip.j2").render(**params))]
     params.update(main_ns=ns, with_split=with_split, with_splitk=with_splitk)
