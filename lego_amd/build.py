@@ -22,6 +22,7 @@ ROOT = Path(__file__).resolve().parents[1]
 LIB_DIR = Path(__file__).resolve().parent / "lib"
 LIB_PATH = LIB_DIR / "liblego_hip.so"
 NODE_PATH = LIB_DIR / "layernorm_node.so"
+CALLS_PATH = LIB_DIR / "host_calls.so"
 OBJ_DIR = LIB_DIR / "obj"
 
 # the tilings the library is built with
@@ -388,34 +389,44 @@ def _compile(src: Path, incremental: bool = False) -> Path:
 
 
 def build_node(incremental: bool = False) -> Path:
-    """Compile the LayerNorm node (C++ over torch's headers) beside liblego_hip.so, which it is linked with.  The object is tied to
+    """The LayerNorm node."""
+    return _build_extension(CSRC / "layernorm_node.cpp", NODE_PATH, incremental)
+
+
+def build_calls(incremental: bool = False) -> Path:
+    """The host side of the one-launch operators."""
+    return _build_extension(CSRC / "host_calls.cpp", CALLS_PATH, incremental)
+
+
+def _build_extension(src: Path, path: Path, incremental: bool) -> Path:
+    """Compile C++ over torch's headers beside liblego_hip.so, which it is linked with.  The object is tied to
     torch's C++ ABI: what it was built with is kept in a stamp beside it, and another torch or command builds it again."""
     import sysconfig
 
     import torch
     from torch.utils import cpp_extension
-    src, stamp = CSRC / "layernorm_node.cpp", NODE_PATH.with_suffix(".stamp")
+    stamp = path.with_suffix(".stamp")
     includes = [str(ROOT / "include"), *cpp_extension.include_paths(), "/opt/rocm/include", sysconfig.get_paths()["include"]]
     libs = cpp_extension.library_paths()
     cmd = ["g++", "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", "-DTORCH_API_INCLUDE_EXTENSION_H",
-           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DTORCH_EXTENSION_NAME={NODE_PATH.stem}",
-           *[a for i in includes for a in ("-I", i)], str(src), "-o", str(NODE_PATH),
+           f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", f"-DTORCH_EXTENSION_NAME={path.stem}",
+           *[a for i in includes for a in ("-I", i)], str(src), "-o", str(path),
            *[a for d in libs for a in ("-L", d, f"-Wl,-rpath,{d}")], "-L", str(LIB_DIR), "-Wl,-rpath,$ORIGIN", f"-l:{LIB_PATH.name}",
            "-ltorch", "-ltorch_cpu", "-ltorch_python", "-lc10", "-lc10_hip", "-ltorch_hip"]
     built_with = "\n".join([torch.__version__, sys.version, *cmd])
-    if (incremental and NODE_PATH.exists() and stamp.exists() and stamp.read_text() == built_with
-            and NODE_PATH.stat().st_mtime > max(p.stat().st_mtime for p in (src, ROOT / "include" / "lego_hip.h"))):
-        return NODE_PATH
+    if (incremental and path.exists() and stamp.exists() and stamp.read_text() == built_with
+            and path.stat().st_mtime > max(p.stat().st_mtime for p in (src, ROOT / "include" / "lego_hip.h"))):
+        return path
     stamp.unlink(missing_ok=True)
     res = subprocess.run(cmd, capture_output=True, text=True)
     if res.returncode != 0:
         raise RuntimeError(f"g++ failed on {src.name}:\n{res.stderr}")
     stamp.write_text(built_with)
-    return NODE_PATH
+    return path
 
 
 def build(verbose=True, incremental=False):
-    """Generate, compile every translation unit for gfx950 and link liblego_hip.so, then the LayerNorm node.  With
+    """Generate, compile every translation unit for gfx950 and link liblego_hip.so, then the two extension modules.  With
     ``incremental`` a translation unit whose object file is newer than its source is kept."""
     sources = generate() + [CSRC / "lego_hip_abi.hip"]
     OBJ_DIR.mkdir(parents=True, exist_ok=True)
@@ -429,8 +440,9 @@ def build(verbose=True, incremental=False):
         print(f"built {LIB_PATH} from {len(sources)} translation units")
     try:
         build_node(incremental)
+        build_calls(incremental)
     except ModuleNotFoundError as missing:      # the library itself needs no torch
-        print(f"{NODE_PATH.name} is not built: {missing}")
+        print(f"{NODE_PATH.name} and {CALLS_PATH.name} are not built: {missing}")
     return LIB_PATH
 
 

@@ -48,9 +48,36 @@ def _check(t, dtype, name, ndim=2):
         raise ValueError(f"{name} must be contiguous")
 
 
+class _InPython:
+    """In place of the module in C++: every call is Python's."""
+
+    transpose = softmax = stencil = matmul = group = staticmethod(lambda *args: None)
+
+
+_calls = None
+
+
+def _host():
+    """The operators' host side in C++ (csrc/host_calls.cpp); each gives None for what it leaves to Python: other than plain GPU tensors,
+    calls under a tracer, a mode or a transform, and calls that are refused."""
+    global _calls
+    if torch.compiler.is_compiling():
+        return _InPython
+    if _calls is None:
+        try:
+            _calls = runtime.host_calls()
+        except (FileNotFoundError, ImportError) as e:
+            warnings.warn(f"the operators' host side runs in Python, some 3 us more a call: {e}", RuntimeWarning, stacklevel=3)
+            _calls = _InPython
+    return _calls
+
+
 def transpose(x: torch.Tensor) -> torch.Tensor:
     """``x.T`` materialised: the ``rows x cols`` row-major input copied into the
     column-major layout of the same logical matrix."""
+    out = _host().transpose(x)
+    if out is not None:
+        return out
     if x.element_size() not in (2, 4):
         raise ValueError("transpose moves 2-byte and 4-byte elements (float16, bfloat16, float32, int32, ...)")
     _check(x, x.dtype, "x")
@@ -67,6 +94,10 @@ _ROW_TAG = {torch.float16: "f16", torch.bfloat16: "bf16", torch.float32: "f32"}
 
 def softmax(x: torch.Tensor, waves_per_row: int | None = None) -> torch.Tensor:
     """Row softmax of a 2-D fp16, bf16 or fp32 tensor."""
+    if waves_per_row is None:
+        y = _host().softmax(x)
+        if y is not None:
+            return y
     if x.dtype not in _ROW_TAG:
         raise ValueError("softmax supports float16, bfloat16 and float32")
     _check(x, x.dtype, "x")
@@ -225,6 +256,9 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     column-major (a ``.T`` view), fp32 accumulation, row-major fp16 result: the reference's ``matmul``
     allocates a float16 result whatever its operands' type (matmul_sympy.py:129-145, its fp8 path
     :346-364).  ``out_dtype=torch.bfloat16`` with bfloat16 operands keeps their type instead."""
+    c = _host().matmul(a, b, activation, out_dtype)
+    if c is not None:
+        return c
     if activation not in ("", "leaky_relu"):
         raise NotImplementedError(f"activation {activation!r} is not generated by this build")
     a_store, ta = _operand(a, "a")
@@ -297,6 +331,9 @@ def _problems_apart(sizes):
 
 def lego_group_gemm_fn(group_A, group_B):
     """One launch for a list of independent GEMMs; returns the list of results."""
+    group_C = _host().group(group_A, group_B)
+    if group_C is not None:
+        return group_C
     if len(group_A) != len(group_B):
         raise ValueError("group_A and group_B must have the same length")
     # Problems whose rows are not whole 16-byte chunks run on zero-padded copies in a workspace; those whose long chains the other
@@ -365,6 +402,10 @@ def needleman_wunsch(reference: torch.Tensor, matrix: torch.Tensor, penalty: int
 
 
 def _stencil(entry, x, c, radius, bricks, out):
+    if out is None:
+        got = _host().stencil(x, c, radius, bricks, c.dim() == 3)
+        if got is not None:
+            return got
     _check(x, torch.float32, "x", ndim=3)
     _check(c, torch.float32, "c", ndim=c.dim())
     n = x.shape[0]

@@ -11,6 +11,7 @@ from pathlib import Path
 
 LIB_PATH = Path(__file__).resolve().parent / "lib" / "liblego_hip.so"
 NODE_PATH = LIB_PATH.with_name("layernorm_node.so")
+CALLS_PATH = LIB_PATH.with_name("host_calls.so")
 
 _c_int, _c_void_p, _c_float = ctypes.c_int, ctypes.c_void_p, ctypes.c_float
 _PTR_ARRAY = ctypes.POINTER(ctypes.c_void_p)
@@ -123,22 +124,34 @@ def load_library(path=None):
 
 
 _node = None
+_calls = None
+
+
+def _extension(path):
+    import importlib.machinery
+    import importlib.util
+    if not path.exists():
+        raise FileNotFoundError(f"{path} is missing: build it with `python -m lego_amd.build`")
+    loader = importlib.machinery.ExtensionFileLoader(path.stem, str(path))
+    module = importlib.util.module_from_spec(importlib.util.spec_from_loader(path.stem, loader))
+    loader.exec_module(module)
+    return module
 
 
 def layernorm_node():
     """The extension module with LayerNorm's autograd node, prebuilt beside the library."""
     global _node
     if _node is None:
-        import importlib.machinery
-        import importlib.util
-        if not NODE_PATH.exists():
-            raise FileNotFoundError(
-                f"{NODE_PATH} is missing: build it with `python -m lego_amd.build`")
-        loader = importlib.machinery.ExtensionFileLoader("layernorm_node", str(NODE_PATH))
-        module = importlib.util.module_from_spec(importlib.util.spec_from_loader("layernorm_node", loader))
-        loader.exec_module(module)
-        _node = module
+        _node = _extension(NODE_PATH)
     return _node
+
+
+def host_calls():
+    """The extension module with the host side of the one-launch operators, prebuilt beside the library."""
+    global _calls
+    if _calls is None:
+        _calls = _extension(CALLS_PATH)
+    return _calls
 
 
 _entry_points = {}
