@@ -31,7 +31,7 @@ from .common import BANNER, Emitted, code, idx, size, template, tidy
 B = 64
 # the single launch: strips of STRIP columns, STRIPS of them per workgroup, in phases of P steps; an LDS ring of RING blocks of
 # P slots per strip, scores requested AHEAD blocks before they are needed, the column to the left WEST_AHEAD blocks before
-STRIP, STRIPS, P, RING, AHEAD, WEST_AHEAD, LAG = 128, 2, 16, 9, 4, 1, 6
+STRIP, STRIPS, P, RING, AHEAD, WEST_AHEAD, LAG = 128, 2, 16, 9, 4, 2, 6
 
 
 def tile_layout(b=B):

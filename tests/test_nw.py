@@ -199,3 +199,47 @@ def test_gpu_maximum_size_closed_form():
     for rows in (slice(0, 130), slice(16000, 16130), slice(n - 129, n + 1)):
         want = -(idx[rows, None] - idx[None, :]).abs() * penalty
         assert torch.equal(m[rows], want)
+
+
+def _wrapped(ref, m, penalty):
+    """The recurrence modulo 2^32 over any borders, one anti-diagonal at a time."""
+    ref, m = ref.numpy(), m.numpy().copy()
+    p = np.array([penalty], dtype=np.int32)
+    for d in range(2, 2 * len(m) - 1):
+        i = np.arange(max(1, d - len(m) + 1), min(d - 1, len(m) - 1) + 1)
+        j = d - i
+        m[i, j] = np.maximum(np.maximum(m[i - 1, j - 1] + ref[i, j], m[i, j - 1] - p), m[i - 1, j] - p)
+    return torch.from_numpy(m)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [128, 192, 256, 320, 576])
+@pytest.mark.parametrize("where", ["near", "score", "score last", "top", "left", "penalty", "negative"])
+def test_gpu_values_beyond_the_near_form(n, where):
+    """The kernel leaves its shorter form of the recurrence where a value is too far from zero for it: at the bounds themselves, and where
+    the first one beyond is a score in any strip, a border's cell, or the penalty."""
+    from lego_amd import ops
+    print(f"needleman-wunsch n={n}, {where}", flush=True)
+    g = torch.Generator().manual_seed(7 * n)
+    limit, penalty = (1 << 28) // (n + 256), 9
+    ref = torch.randint(-4, 12, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    m = torch.randint(-99, 99, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    if where == "near":              # scores and penalty as large as the shorter form takes them
+        ref = torch.where(ref > 4, limit, -limit).to(torch.int32)
+        penalty = (1 << 27) // (n + 256)
+        m[n // 3, 0] = -(1 << 27)
+    elif where == "score":
+        ref[n // 2, n // 3], ref[n // 2 + 1, n - 5] = limit + 1, 2 ** 31 - 1
+    elif where == "score last":
+        ref[n, n], ref[n - 20, 1] = -(2 ** 31), -limit - 1
+    elif where == "top":
+        m[0, n - 3], m[0, 1] = 2 ** 31 - 1, (1 << 28) + 1000
+    elif where == "left":
+        m[n // 2, 0], m[n // 2 + 40, 0] = 2 ** 31 - 5, -(2 ** 31)
+    elif where == "penalty":
+        penalty = (1 << 27) // (n + 256) + 1
+    else:
+        penalty = -3
+    want = _wrapped(ref, m, penalty)
+    got = ops.needleman_wunsch(ref.cuda(), m.cuda(), penalty)
+    assert torch.equal(got.cpu(), want)
