@@ -245,6 +245,10 @@ int lego_hip_grouped_gemm_f16(const void* const* a, const void* const* b, void* 
 int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, unsigned long long* bytes);
 int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
                                  void* workspace, unsigned long long workspace_bytes, void* stream);
+/* What lego_hip_grouped_gemm_f16_ws has a use for: room for those copies and for the partial sums of deep problems, which are computed in parts along
+ * K where their chains are what the launch waits for (0: for neither).  *limit receives the most k-tiles of 64 that a workgroup then takes, or
+ * 0 where there are no parts.  With room for the copies alone, all problems stay whole. */
+int lego_hip_grouped_gemm_f16_room(const int* sizes3, int groups, unsigned long long* bytes, int* limit);
 /* Which problems of a grouped call are better apart, apart[g] = 1: those that need copies and that lego_hip_gemm_ex_ws would split
  * along K, where the other problems do not fill the time of their chains.  Host only; lego_hip_grouped_gemm_f16_ws itself takes
  * any of them. */

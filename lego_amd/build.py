@@ -279,6 +279,8 @@ def collect():
           "const void* const*, void* const*, const int*, int, hipStream_t);",
           f"hipError_t lego_grouped_gemm_f16_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep_launch(const void* const*, "
           "const void* const*, void* const*, const int*, int, hipStream_t);",
+          f"hipError_t lego_grouped_gemm_f16_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep_parts_launch(const void* const*, "
+          "const void* const*, void* const*, const int*, int, int, float*, hipStream_t);",
           "hipError_t lego_gemm_f16_nn_w2x4_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);",
           *[f"hipError_t lego_gemm_{d}_{v}_m32_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);"
             for d in GEMM_SPARSE_ROUND_DTYPES for v in ("nn", "nt", "tn", "tt")],

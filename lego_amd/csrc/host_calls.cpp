@@ -155,18 +155,22 @@ PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t count)
   if (groups == 0 || groups > kMost || PyList_GET_SIZE(args[1]) != groups) return nothing();
   std::vector<at::Tensor> as, bs, cs;       // held while the interpreter's lock is not
   std::vector<int> sizes;
-  bool ragged = false;
+  bool ragged = false, deep = false;
   for (Py_ssize_t g = 0; g < groups; ++g) {
     const at::Tensor *const a = plain(PyList_GET_ITEM(args[0], g), 2), *const b = plain(PyList_GET_ITEM(args[1], g), 2);
     if (!a || !b || a->scalar_type() != at::kHalf || b->scalar_type() != at::kHalf || !a->is_contiguous() || !b->is_contiguous() || a->size(1) != b->size(0))
       return nothing();
     const int N = (int)b->size(1), K = (int)a->size(1);
     ragged = ragged || N % 8 || K % 8;
-    if (ragged && (groups == 1 || ((N % 8 || K % 8) && K > 1984))) return nothing();       // those that may be products of their own
+    if (ragged && groups == 1) return nothing();       // a product of its own
+    deep = deep || ((N % 8 || K % 8) && K > 1984);
     as.push_back(*a);
     bs.push_back(*b);
     sizes.insert(sizes.end(), {(int)a->size(0), N, K});
   }
+  unsigned long long need = 0;
+  int limit = 0;
+  if (lego_hip_grouped_gemm_f16_room(sizes.data(), (int)groups, &need, &limit) != 0 || (deep && limit == 0)) return nothing();      // some may be products of their own
   HANDLE_TH_ERRORS
   {
     pybind11::gil_scoped_release nothing_here_needs_it;
@@ -178,14 +182,10 @@ PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t count)
       pb[g] = bs[g].const_data_ptr();
       pc[g] = cs[g].mutable_data_ptr();
     }
-    unsigned long long need = 0;
-    int code = ragged ? lego_hip_grouped_gemm_f16_workspace_bytes(sizes.data(), (int)groups, &need) : 0;
-    if (code == 0) {
-      at::Tensor workspace;
-      if (ragged) workspace = at::empty({(int64_t)((need + 3) / 4)}, options_of(cs.back()).dtype(at::kFloat));
-      code = ragged ? lego_hip_grouped_gemm_f16_ws(pa, pb, pc, sizes.data(), (int)groups, workspace.mutable_data_ptr(), need, current_stream())
-                    : lego_hip_grouped_gemm_f16(pa, pb, pc, sizes.data(), (int)groups, current_stream());
-    }
+    at::Tensor workspace;
+    if (need) workspace = at::empty({(int64_t)((need + 3) / 4)}, options_of(cs.back()).dtype(at::kFloat));
+    const int code = need ? lego_hip_grouped_gemm_f16_ws(pa, pb, pc, sizes.data(), (int)groups, workspace.mutable_data_ptr(), need, current_stream())
+                          : lego_hip_grouped_gemm_f16(pa, pb, pc, sizes.data(), (int)groups, current_stream());
     if (code != 0) cs.clear();
   }
   if (cs.empty()) return nothing();

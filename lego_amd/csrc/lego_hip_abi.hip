@@ -1207,6 +1207,8 @@ double grouped_makespan(const long* count, const double* cost, int batches, long
 struct GroupedPlan {
   int kind, tiles, split;
   double time;      // the estimate that chose it, in the units below
+  int limit;        // k-tiles of a unit where the call is shorter with deep problems in parts, given room for their sums (0: nowhere), ...
+  int sums;         // ... and the tiles of those
 };
 
 // Costs in units of one k-tile step of a 256 x 256 tile that has its CU to itself (about 1.8 us for
@@ -1216,6 +1218,12 @@ struct GroupedPlan {
 // per k-tile and two steps beside them: the choice between the two so estimated takes 1.0005 times the better one over 72
 // drawn calls of 1 to 16 problems (us, two workgroups per CU / one: 112 x 120 x 2816 and 128 x 184 x 512 30.5 / 19.7; 16 problems, 546 tiles of up to
 // 57 k-tiles, 68 / 45; nine of 565 tiles 71 / 52; 13 of 1056 tiles, deep ones among them in every round, 80 / 91; 14 of 762 tiles of up to 12 k-tiles 25.6 / 28.0).
+// In parts along K: the same per k-tile and a little more for the sums that a workgroup stores, the second launch, and for each tile of sums its
+// way to memory and back; parts where that is less than 0.9 of the best whole launch.  Over 36 drawn calls of 1 to 16 problems this takes 0.94 of
+// the whole launches' time, the best of eight limits for each call 0.93, and over 60 others 0.92 (us, whole / parts: five problems of 43 to 8 k-tiles 34.1 / 20.1, six
+// 42 / 23, thirteen of 13 GFLOP 48 / 28; without the margin thirteen of 34.7 took 37.7).
+constexpr double kPartOverhead = 2.3, kPartLaunch = 2.2, kPartSum = 0.035, kPartGain = 0.9;
+constexpr int kPartTiles = 1024;       // partial sums of a call, 64 KiB each
 constexpr double kTileOverhead = 1.6, kHalfStep = 0.58, kHalfOverhead = 1.5, kSmallCost = 0.66, kDeepStep = 0.38, kDeepOverhead = 2.0;
 // Problems per call.  A launch carries its pointers and sizes as kernel arguments, LEGO_GROUPED_MAX_GROUPS problems
 // at most; a call with more is enqueued as several launches (below).
@@ -1279,6 +1287,25 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
   plan.tiles = static_cast<int>(total);
   plan.split = plan.kind == 0 ? static_cast<int>(best_split) : 0;
   plan.time = plan.kind == 2 ? t_deep : plan.kind == 1 ? t_small : best;
+  plan.limit = plan.sums = 0;
+  double least = kPartGain * plan.time;
+  for (const int limit : {4, 6, 8, 12, 16, 24, 32, 48}) {
+    if (!deep || limit >= depth[0]) break;      // the deepest problem is the first
+    long count[LEGO_GROUPED_MAX_GROUPS], units = 0, sums = 0;
+    double length[LEGO_GROUPED_MAX_GROUPS], cost[LEGO_GROUPED_MAX_GROUPS];
+    for (int s = 0; s < groups; ++s) {
+      const long d = static_cast<long>(depth[s]), parts = (d + limit - 1) / limit, per = (d + parts - 1) / parts, used = (d + per - 1) / per;
+      if (used > 1) sums += used * small[s];
+      units += used * small[s];
+      const double t = kDeepStep * per + (used > 1 ? kPartOverhead : kDeepOverhead);
+      int j = s;
+      while (j > 0 && length[j - 1] < per) { length[j] = length[j - 1]; cost[j] = cost[j - 1]; count[j] = count[j - 1]; --j; }
+      length[j] = per; cost[j] = t; count[j] = used * small[s];
+    }
+    if (sums > kPartTiles) continue;
+    const double t = grouped_makespan(count, cost, groups, cus) + kPartLaunch + kPartSum * sums;
+    if (t < least) { least = t; plan.limit = limit; plan.sums = static_cast<int>(sums); }
+  }
   return plan;
 }
 
@@ -1477,17 +1504,63 @@ int lego_hip_grouped_gemm_f16_workspace_bytes(const int* sizes3, int groups, uns
   return ok_or(hipErrorOutOfMemory);
 }
 
+namespace {
+constexpr unsigned long long kSumBytes = 128 * 128 * sizeof(float);
+// The launch of a call in parts, its problems on whole chunks: as the plan for their sizes has it.  One launch's problems, in one run of copies.
+inline GroupedPlan parts_plan(const int* sizes3, int groups, unsigned long long copies)
+{
+  GroupedPlan none{};
+  if (groups > LEGO_GROUPED_MAX_GROUPS || copies > kCopyRoom) return none;
+  int sizes[3 * LEGO_GROUPED_MAX_GROUPS];
+  for (int g = 0; g < groups; ++g) {
+    const int m = sizes3[3 * g], n = sizes3[3 * g + 1], k = sizes3[3 * g + 2];
+    const bool ragged = n % 8 || k % 8;
+    const int size[3] = {m, ragged ? round_up(n, 8) : n, ragged ? round_up(k, 8) : k};
+    memcpy(sizes + 3 * g, size, sizeof(size));
+  }
+  return grouped_plan(sizes, groups);
+}
+inline unsigned long long all_copies(const int* sizes3, int groups)
+{
+  unsigned long long total = 0;
+  for (int g = 0; g < groups; ++g) total += copies_of(sizes3 + 3 * g);
+  return total;
+}
+}  // namespace
+
+int lego_hip_grouped_gemm_f16_room(const int* sizes3, int groups, unsigned long long* bytes, int* limit)
+{
+  if (limit == nullptr) return kInvalid;
+  const int rc = lego_hip_grouped_gemm_f16_workspace_bytes(sizes3, groups, bytes);
+  if (rc != 0) return rc;
+  const GroupedPlan plan = parts_plan(sizes3, groups, all_copies(sizes3, groups));
+  *limit = plan.limit;
+  *bytes += plan.sums * kSumBytes;
+  return 0;
+}
+
 int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups,
                                  void* workspace, unsigned long long workspace_bytes, void* stream) try
 {
   const int checked = grouped_check(a, b, c, sizes3, groups);
   unsigned long long need = 0;
+  // the products, their copies in the first `used` bytes of the workspace: with deep ones in parts where there is room for the sums
+  const auto products = [&](const void* const* aa, const void* const* bb, void* const* cc, const int* sizes, int count, unsigned long long used) {
+    if (count == groups && used <= workspace_bytes && usable(workspace) && grouped_check(aa, bb, cc, sizes, count) == 0) {
+      const GroupedPlan plan = parts_plan(sizes, count, used);
+      if (plan.limit && workspace_bytes - used >= plan.sums * kSumBytes)
+        return ok_or(lego_grouped_gemm_f16_t128x128_deep_parts_launch(aa, bb, cc, sizes, count, plan.limit,
+                                                                      reinterpret_cast<float*>(static_cast<uint8_t*>(workspace) + used), as_stream(stream)));
+    }
+    return lego_hip_grouped_gemm_f16(aa, bb, cc, sizes, count, stream);
+  };
+  if (checked == 0) return products(a, b, c, sizes3, groups, 0);
   if (checked != 2 || lego_hip_grouped_gemm_f16_workspace_bytes(sizes3, groups, &need) != 0 || need == 0 || workspace_bytes < need || !usable(workspace))
     return lego_hip_grouped_gemm_f16(a, b, c, sizes3, groups, stream);
   std::vector<const void*> aa, bb;
   std::vector<void*> cc;
   std::vector<int> sizes, copied;
-  return grouped_copy_runs(sizes3, groups, [&](const int* problems, int count, unsigned long long) {
+  return grouped_copy_runs(sizes3, groups, [&](const int* problems, int count, unsigned long long used) {
     aa.clear(); bb.clear(); cc.clear(); sizes.clear(); copied.clear();
     Copier pads(true, as_stream(stream)), back(false, as_stream(stream));
     uint8_t* at = static_cast<uint8_t*>(workspace);
@@ -1506,7 +1579,7 @@ int lego_hip_grouped_gemm_f16_ws(const void* const* a, const void* const* b, voi
     }
     const hipError_t err = pads.flush();
     if (err != hipSuccess) return ok_or(err);
-    const int rc = lego_hip_grouped_gemm_f16(aa.data(), bb.data(), cc.data(), sizes.data(), count, stream);
+    const int rc = products(aa.data(), bb.data(), cc.data(), sizes.data(), count, used);
     if (rc != 0) return rc;
     for (const int i : copied) back.add(cc[i], c[problems[i]], sizes[3 * i], sizes3[3 * problems[i] + 1], sizes[3 * i], sizes[3 * i + 1], 2);
     return ok_or(back.flush());

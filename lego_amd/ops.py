@@ -322,7 +322,10 @@ def _problems_apart(sizes):
     """Asked once for a list of sizes: the answer is a function of the sizes alone."""
     groups = len(sizes) // 3
     flags = (ctypes.c_int * groups)()
-    runtime.call("lego_hip_grouped_gemm_f16_apart", (ctypes.c_int * len(sizes))(*sizes), groups, flags)
+    sz, size, limit = (ctypes.c_int * len(sizes))(*sizes), ctypes.c_ulonglong(0), ctypes.c_int(0)
+    runtime.call("lego_hip_grouped_gemm_f16_room", sz, groups, ctypes.byref(size), ctypes.byref(limit))
+    if not limit.value:      # otherwise in parts, in the one launch
+        runtime.call("lego_hip_grouped_gemm_f16_apart", sz, groups, flags)
     if len(_group_apart) >= 1024:
         _group_apart.clear()
     apart = _group_apart[sizes] = frozenset(g for g in range(groups) if flags[g])
@@ -374,9 +377,9 @@ def _grouped(group_A, group_B, sizes):
     pb = arr(*[t.data_ptr() for t in group_B])
     pc = arr(*[t.data_ptr() for t in group_C])
     sz = (ctypes.c_int * (3 * groups))(*sizes)
-    if any(s % 8 for s in sizes[1::3]) or any(s % 8 for s in sizes[2::3]):
-        size = ctypes.c_ulonglong(0)
-        runtime.call("lego_hip_grouped_gemm_f16_workspace_bytes", sz, groups, ctypes.byref(size))
+    size, limit = ctypes.c_ulonglong(0), ctypes.c_int(0)
+    runtime.call("lego_hip_grouped_gemm_f16_room", sz, groups, ctypes.byref(size), ctypes.byref(limit))
+    if size.value:
         workspace = torch.empty(size.value // 2, dtype=torch.float16, device=group_C[0].device)
         runtime.call("lego_hip_grouped_gemm_f16_ws", pa, pb, pc, sz, groups, _ptr(workspace), size.value, _stream())
         return group_C

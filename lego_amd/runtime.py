@@ -70,6 +70,7 @@ SIGNATURES = {
     "lego_hip_grouped_gemm_f16": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_void_p],
     "lego_hip_grouped_gemm_f16_workspace_bytes": [_INT_ARRAY, _c_int, ctypes.POINTER(ctypes.c_ulonglong)],
     "lego_hip_grouped_gemm_f16_ws": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_void_p, ctypes.c_ulonglong, _c_void_p],
+    "lego_hip_grouped_gemm_f16_room": [_INT_ARRAY, _c_int, ctypes.POINTER(ctypes.c_ulonglong), ctypes.POINTER(_c_int)],
     "lego_hip_grouped_gemm_f16_apart": [_INT_ARRAY, _c_int, _INT_ARRAY],
     "lego_hip_grouped_gemm_f16_plan": [_INT_ARRAY, _c_int, _INT_ARRAY],
     "lego_hip_grouped_gemm_f16_split": [_PTR_ARRAY, _PTR_ARRAY, _PTR_ARRAY, _INT_ARRAY, _c_int, _c_int, _c_void_p],

@@ -92,7 +92,7 @@ def test_gpu_groups_and_stencils(monkeypatch):
     print("host calls, groups and stencils", flush=True)
     made = lambda sizes: ([torch.randint(-2, 3, (m, k), device="cuda").half() for m, _, k in sizes], [torch.randint(-2, 3, (k, n), device="cuda").half() for _, n, k in sizes])
     for sizes, taken in (([(64, 64, 64)], True), ([(33, 16, 72), (128, 128, 64)], True), ([(33, 17, 65), (128, 128, 64)], True), ([(33, 17, 65)], False),
-                         ([(8, 8, 8)] * 65, False), ([(8, 8, 2001), (8, 8, 8)], False)):
+                         ([(8, 8, 8)] * 65, False), ([(8, 8, 2001), (8, 8, 8)], True), ([(64, 64, 2577)] + [(1024, 1024, 1024)] * 16, False)):
         a, b = made(sizes)
         _both(monkeypatch, lambda: ops.lego_group_gemm_fn(a, b), taken)
     x, c = torch.rand(16, 16, 16, device="cuda"), torch.rand(8, 8, 8, device="cuda")
