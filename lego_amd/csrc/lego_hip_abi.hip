@@ -967,7 +967,9 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
   if (a == nullptr || b == nullptr || c == nullptr || (activation != 0 && activation != 1)) return kInvalid;
   if ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 1u) return kInvalid;
   const auto product = [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
-    const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK);
+    // as many parts as there is room for: that of a product on copies is asked for with M rounded up, and the estimate of a smaller M
+    // may want more of them (130 x 136 x 8200 43, 136 x 136 x 8200 33)
+    const int parts = N % 8 || K % 8 ? splitk_parts(round_up(m, 8), n, round_up(k, 8), LEGO_GEMM_BK) : splitk_parts(m, n, k, LEGO_GEMM_BK);
     if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
     return ok_or(parts_by_layout(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
   };
