@@ -111,7 +111,7 @@ int lego_hip_layernorm_bwd_bf16(const void* dy, const void* x, const void* w, co
  * last k-tile where need be, take every shape whose operand rows are whole 16-byte chunks on 16-byte
  * aligned bases: N a multiple of 8, and K (operands as given) or M (A transposed) a multiple of 8 as
  * well.  Any other shape or alignment (bases need only element alignment then) takes a kernel that
- * moves one element per access, about a tenth as fast.  Shapes in whole tiles take a kernel without
+ * reads vectors at any element.  Shapes in whole tiles take a kernel without
  * edge tests. */
 int lego_hip_gemm_f16(const void* a, const void* b, void* c, int M, int N, int K, void* stream);
 /* The same with the reference's fused epilogue (matmul(a, b, activation="leaky_relu"),
@@ -137,7 +137,7 @@ int lego_hip_gemm_bf16_f16_ex(const void* a, const void* b, void* c, int M, int 
  * of every tile are dealt to several workgroups, which leave fp32 sums there, and a second kernel adds them in a
  * fixed order (deterministic), applies the activation and stores C.  A product with N or K that is not a multiple
  * of 8 (operand rows that are not whole 16-byte chunks) runs on zero-padded copies of A, B and C in the workspace
- * instead of the one-element-per-access kernel, about ten times as fast; operands may then start at any element.
+ * instead of the kernel that takes any shape, faster where K is long; operands may then start at any element.
  * lego_hip_gemm_workspace_bytes gives room for all that the call uses for a shape, shallow products aside (0: none of 32 k-tiles and
  * more, and no copies); lego_hip_gemm_layout_workspace_bytes gives what it uses.
  * The workspace is scratch: 16-byte aligned device memory, contents undefined on entry and exit, not to be shared
@@ -159,8 +159,9 @@ int lego_hip_gemm_fp8_ex(const void* a, const void* b, void* c, int M, int N, in
 int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* bytes);
 int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                             int activation, int format, void* workspace, unsigned long long workspace_bytes, void* stream);
-/* What lego_hip_gemm_ex_ws (element_bytes 2) or lego_hip_gemm_fp8_ex_ws (1) uses of that for operands of this layout: 0 too for products that
- * run without (lego_hip_gemm_rows_plan), which the plain entry points compute as well. */
+/* What lego_hip_gemm_ex_ws (element_bytes 2) or lego_hip_gemm_fp8_ex_ws (1; lego_hip_gemm_fp8_padded where rows are not whole 16-byte chunks)
+ * uses of that for operands of this layout: 0 too for products that run best without (lego_hip_gemm_rows_plan, and small ones of ragged
+ * rows), which the plain entry points compute. */
 int lego_hip_gemm_layout_workspace_bytes(int M, int N, int K, int trans_a, int trans_b, int element_bytes, unsigned long long* bytes);
 /* The product on zero-padded copies for operand rows that are not whole 16-byte chunks (lego_hip_gemm_fp8_padded_bytes gives the
  * size of the workspace, 0 where copies gain nothing): one launch for the copies, the product, one that copies the result back.

@@ -780,8 +780,8 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
   // The tiled kernels move 16-byte chunks (`chunk` elements): bases 16-byte aligned and every operand row
   // in whole chunks -- rows of C and of B as given run along N, rows of A as given and of a transposed B
   // along K, rows of a transposed A along M.  Tiles may be ragged in M, N and K.  Everything else -- the
-  // reference keeps M, N, K symbolic (matmul_sympy.py:69-70) -- goes to the kernel that moves one element
-  // per access.
+  // reference keeps M, N, K symbolic (matmul_sympy.py:69-70) -- goes to the kernel that reads vectors at any
+  // element.
   (void)bk;
   const bool tiled = usable(a) && usable(b) && usable(c) && N % chunk == 0 &&
                      (trans_a ? M % chunk == 0 : K % chunk == 0) && (!trans_b || K % chunk == 0);
@@ -826,10 +826,10 @@ typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int,
 
 // Operand rows that are not whole 16-byte chunks: the tiled kernels run on zero-padded copies (every side a multiple of `chunk`
 // elements; the padding adds zeros to the sums) and the result is copied back: two more launches and three more passes over
-// the matrices, against the kernel that moves one element per access and whose chain of k-tiles is long.  8-bit operands, us by
+// the matrices, against the kernel that takes any shape, here when it moved one element per access.  8-bit operands, us by
 // elements / on copies: 320 x 1984 x 7959 829 / 35, 2000 x 2000 x 2001 276 / 27, 5000 x 3001 x 136 93 / 32, 6902 x 192 x 296 31 / 28, 1000 x
 // 1001 x 264 38 / 14, 16 x 65 x 257 20 / 16, 33 x 100 x 200 16 / 23, 1000 x 1000 x 136 16 / 22: copies from K = 256 on, or from as many 64 x 64 tiles of the
-// result as keep the one-element kernel busy for 30 us.
+// result as kept it busy for 30 us; of these the rule below sends to that kernel what it now does sooner.
 inline bool copies_gain_8bit(int M, int N, int K)
 {
   const double tiles = static_cast<double>((M + 63) / 64) * ((N + 63) / 64);
@@ -840,6 +840,21 @@ inline unsigned long long padded_bytes(int M, int N, int K, int chunk, int bytes
 {
   const unsigned long long m = round_up(M, chunk), n = round_up(N, chunk), k = round_up(K, chunk);
   return bytes * (m * k + k * n) + 2ull * m * n;
+}
+// Whether a product whose rows are not whole 16-byte chunks is better off with the kernel that takes any than on padded copies, one or two
+// launches more.  In us: there 3.7 and the longer of one tile's chain of k-tiles and the tiles' work over the chip's CUs; here 9.5, or 8.2 where
+// the result is not copied back, and the copies' bytes, read and written, at 2 TB/s.  Over 203 drawn ragged products of all types and layouts the
+// rule takes 0.80 of the time on copies, the better of the two each time 0.78.  us direct / on copies: fp16 64 x 852 x 64 4.5 / 10.5, 55 x 512 x 93
+// 5.6 / 15.3, 64 x 3594 x 314 6.6 / 10.9, 3039 x 336 x 518 10.8 / 13.0; 6 x 383 x 1688 16.4 / 14.4, 1152 x 5120 x 113 19.2 / 10.5, 1618 x 2024 x 485
+// 22.3 / 14.6, 496 x 135 x 3878 24.4 / 18.6.
+inline bool direct_gains(int M, int N, int K, int trans_a, int trans_b, int chunk, int bytes)
+{
+  const double tiles = static_cast<double>((M + 63) / 64) * ((N + 63) / 64), depth = (K + 63) / 64;
+  const double step = !trans_a && trans_b && K % 8 == 0 ? 0.25 : 0.42;      // both operands k-major: four accesses a lane and k-tile instead of eight
+  const double direct = 3.7 + std::max(step * depth, (1 + 0.9 * step * depth) * tiles / 256);
+  const bool back = N % chunk || (trans_a && M % chunk);
+  const double results = back ? 0.0 : 2.0 * round_up(M, chunk) * N;
+  return direct <= (back ? 9.5 : 8.2) + (padded_bytes(M, N, K, chunk, bytes) - results) / 2e6;
 }
 inline unsigned long long parts_bytes(int M, int N, int parts)
 {
@@ -1017,15 +1032,18 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
   return ok_or(fp8_parts(format)[layout](a, b, c, M, N, K, activation, parts, static_cast<float*>(workspace), as_stream(stream)));
 }
 
-// What is used for operands of one layout, shallow products that gain from parts among them; the kernel for few rows takes some and needs no
-// room for sums.
+// What is used for operands of one layout, shallow products that gain from parts among them; the kernels for few rows and for any shape take
+// some and need no room.
 int lego_hip_gemm_layout_workspace_bytes(int M, int N, int K, int trans_a, int trans_b, int element_bytes, unsigned long long* bytes)
 {
   if (bytes == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
   const int chunk = 16 / element_bytes;
   *bytes = 0;
   if (N % chunk == 0 && K % chunk == 0 && rows_columns(M, N, K, trans_a, trans_b, element_bytes)) return 0;
-  if (element_bytes == 1) *bytes = parts_bytes(M, N, N % 16 ? 1 : splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT));
+  const bool ragged = N % chunk || (trans_a ? M : K) % chunk || (trans_b && K % chunk);
+  if (ragged && direct_gains(M, N, K, trans_a, trans_b, chunk, element_bytes)) return 0;
+  if (element_bytes == 1 && ragged) return lego_hip_gemm_fp8_padded_bytes(M, N, K, trans_a, trans_b, bytes);
+  if (element_bytes == 1) *bytes = parts_bytes(M, N, splitk_parts(M, N, K, LEGO_GEMM_BK_8BIT));
   else *bytes = room_16bit(M, N, K, [](int m, int n, int k) { return splitk_parts(m, n, k, LEGO_GEMM_BK); });
   return 0;
 }

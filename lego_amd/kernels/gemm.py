@@ -569,23 +569,22 @@ def emit(bm=256, bn=256, bk=64, waves=(2, 2), max_group_m=8, trans_a=False, tran
     return Emitted(f"gemm_{dtype}_{variant}{tag}.hip", text, launchers), meta
 
 
-def emit_any(bm=64, bn=64, bk=32):
-    """The kernel for shapes the tiled kernels do not take (any M, N, K and alignment): one element per
-    global access, operands staged k-major in LDS with zero fill past the edges."""
-    assert bm == 64 and bn == 64 and bk % 16 == 0 and 256 * 8 == bm * bk == bn * bk
+def emit_any(bm=64, bn=64, bk=64):
+    """The kernel for shapes the tiled kernels do not take (any M, N, K and alignment): vectors at any
+    element, operands staged k-major in LDS with zero fill past K."""
+    assert bm == 64 and bn == 64 and bk == 64      # sixteen elements of an operand per lane
     M, N, K = size("M"), size("N"), size("K")
     row, col, kk, sr, sk = (idx(n) for n in ("row", "col", "kk", "sr", "sk"))
     rng = {row: (0, M), col: (0, N), kk: (0, K)}
     flat = lambda lay, i, j: tidy(lay.TileBy([lay.dims()[0], lay.dims()[1]])[i, j], rng)  # noqa: E731
-    pitch = bk + 8        # 80-byte rows: eight-k reads of 32 consecutive rows cover every 16-byte bank group evenly
+    pitch = bk + 8        # 144-byte rows: eight-k reads of 16 consecutive rows cover every 16-byte bank group once
     S = OrderBy(Row(bm, pitch)).TileBy([bm, pitch])
+    rows = size("rows")     # of A, or columns of B: an operand is rows x K, row-major (A as given, B transposed) or column-major
     text = template("gemm_any.hip.j2").render(
         banner=BANNER, BM=bm, BN=bn, BK=bk, PITCH=pitch,
-        a_row_layout="OrderBy(Row(M, K))[row, kk]", a_col_layout="OrderBy(Col(M, K))[row, kk]",
-        b_row_layout="OrderBy(Row(K, N))[kk, col]", b_col_layout="OrderBy(Col(K, N))[kk, col]",
+        k_major_layout="OrderBy(Row(rows, K))[row, kk]", row_major_layout="OrderBy(Col(rows, K))[row, kk]",
         c_layout="OrderBy(Row(M, N))[row, col]", s_layout=f"OrderBy(Row({bm}, {pitch}))[sr, sk]",
-        a_row=code(flat(OrderBy(Row(M, K)), row, kk)), a_col=code(flat(OrderBy(Col(M, K)), row, kk)),
-        b_row=code(flat(OrderBy(Row(K, N)), kk, col)), b_col=code(flat(OrderBy(Col(K, N)), kk, col)),
+        k_major=code(flat(OrderBy(Row(rows, K)), row, kk)), row_major=code(flat(OrderBy(Col(rows, K)), row, kk)),
         c_off=code(flat(OrderBy(Row(M, N)), row, col)),
         s_off=code(tidy(S[sr, sk], {sr: (0, bm), sk: (0, pitch)})))
     return Emitted("gemm_any.hip", text, ["lego_gemm_any_launch"])

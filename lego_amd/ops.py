@@ -238,7 +238,7 @@ def _operand(t, name):
     raise ValueError(f"{name} must be contiguous or the transpose of a contiguous tensor")
 
 
-_gemm_workspace, _fp8_padded = {}, {}      # (M, N, K, ta, tb, ...) -> bytes of workspace that the product uses
+_gemm_workspace = {}      # (M, N, K, ta, tb, ...) -> bytes of workspace that the product uses
 
 
 def _ask_workspace(entry, known, shape):
@@ -272,16 +272,12 @@ def matmul(a: torch.Tensor, b: torch.Tensor, activation: str = "", out_dtype=tor
     if a.dtype in _FP8_FORMAT:
         c = torch.empty((M, N), device=a.device, dtype=torch.float16)
         if N % 16 or (M if ta else K) % 16 or (tb and K % 16):
-            # rows that are not whole 16-byte chunks: zero-padded copies where they gain
-            need = _fp8_padded.get((M, N, K, ta, tb))
-            if need is None:
-                need = _ask_workspace("lego_hip_gemm_fp8_padded_bytes", _fp8_padded, (M, N, K, ta, tb))
-            entry = "lego_hip_gemm_fp8_padded"
+            entry = "lego_hip_gemm_fp8_padded"      # rows that are not whole 16-byte chunks: zero-padded copies where they gain
         else:
-            need = _gemm_workspace.get((M, N, K, ta, tb, 1))
-            if need is None:
-                need = _ask_workspace("lego_hip_gemm_layout_workspace_bytes", _gemm_workspace, (M, N, K, ta, tb, 1))
             entry = "lego_hip_gemm_fp8_ex_ws"
+        need = _gemm_workspace.get((M, N, K, ta, tb, 1))
+        if need is None:
+            need = _ask_workspace("lego_hip_gemm_layout_workspace_bytes", _gemm_workspace, (M, N, K, ta, tb, 1))
         if need:
             workspace = torch.empty(need, dtype=torch.uint8, device=a.device)
             runtime.call(entry, _ptr(a_store), _ptr(b_store), _ptr(c), M, N, K, ta, tb,
