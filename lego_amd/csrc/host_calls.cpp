@@ -127,9 +127,9 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t count)
   if (activation < 0 || !(eight || half || brain) || (!eight && out_type != at::kHalf && out_type != type)) return nothing();
   const int M = (int)a->size(0), N = (int)b->size(1), K = (int)a->size(1);
   unsigned long long need = 0;
+  const bool ragged = eight && (N % 16 || (ta ? M : K) % 16 || (tb && K % 16));      // copies, where they gain
   if (eight) {
-    // products in parts, and rows that are not whole 16-byte chunks, are Python's
-    if (N % 16 || (ta ? M : K) % 16 || (tb && K % 16) || lego_hip_gemm_layout_workspace_bytes(M, N, K, ta, tb, 1, &need) != 0 || need != 0) return nothing();
+    if (lego_hip_gemm_layout_workspace_bytes(M, N, K, ta, tb, 1, &need) != 0) return nothing();
   } else if ((ta && M % 8) || lego_hip_gemm_layout_workspace_bytes(M, N, K, ta, tb, 2, &need) != 0) {
     return nothing();       // a column-major A of such columns may be stored row-major first
   }
@@ -139,7 +139,9 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t count)
     const void *const pa = a->const_data_ptr(), *const pb = b->const_data_ptr();
     void *const pc = out.mutable_data_ptr(), *const stream = current_stream();
     const bool mixed = brain && out_type == at::kHalf;
-    const int code = eight ? lego_hip_gemm_fp8_ex(pa, pb, pc, M, N, K, ta, tb, activation, type == at::kFloat8_e5m2, stream)
+    const int code = eight && need ? (ragged ? lego_hip_gemm_fp8_padded : lego_hip_gemm_fp8_ex_ws)(pa, pb, pc, M, N, K, ta, tb, activation, type == at::kFloat8_e5m2,
+                                                                                                   workspace.mutable_data_ptr(), need, stream)
+                     : eight ? lego_hip_gemm_fp8_ex(pa, pb, pc, M, N, K, ta, tb, activation, type == at::kFloat8_e5m2, stream)
                      : need ? lego_hip_gemm_ex_ws(half ? 0 : mixed ? 4 : 1, pa, pb, pc, M, N, K, ta, tb, activation, workspace.mutable_data_ptr(), need, stream)
                             : (half ? lego_hip_gemm_f16_ex : mixed ? lego_hip_gemm_bf16_f16_ex : lego_hip_gemm_bf16_ex)(pa, pb, pc, M, N, K, ta, tb, activation, stream);
     return code == 0 ? out : at::Tensor();

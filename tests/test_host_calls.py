@@ -72,16 +72,15 @@ def test_gpu_rows_and_transposes(monkeypatch, dtype):
 def test_gpu_products(monkeypatch, dtype, out):
     from lego_amd import ops
     eight = torch.finfo(dtype).bits == 8
-    for M, N, K in ((16, 64, 32), (1, 16, 16), (64, 48, 1), (1, 1, 64), (130, 136, 96), (16, 64, 4096), (33, 17, 65), (64, 1024, 512)):
+    for M, N, K in ((16, 64, 32), (1, 16, 16), (64, 48, 1), (1, 1, 64), (130, 136, 96), (16, 64, 4096), (33, 17, 65), (33, 17, 4097), (64, 1024, 512)):
         for ta in (0, 1):
             for tb in (0, 1):
                 a = torch.randint(-2, 3, (K, M) if ta else (M, K), device="cuda").to(dtype)
                 b = torch.randint(-2, 3, (N, K) if tb else (K, N), device="cuda").to(dtype)
                 a, b = a.t() if ta else a, b.t() if tb else b
                 # of one row or column either layout is the other, and the first one is what is seen
-                la, lb = int(not a.is_contiguous()), int(not b.is_contiguous())
-                whole = N % 16 == 0 and (M if la else K) % 16 == 0 and not (lb and K % 16)
-                taken = (whole and K < 4096) if eight else not (la and M % 8)
+                la = int(not a.is_contiguous())
+                taken = eight or not (la and M % 8)
                 print(f"host calls {dtype} {M}x{N}x{K} {ta}{tb}", flush=True)
                 _both(monkeypatch, lambda: ops.matmul(a, b, activation="leaky_relu" if M == 16 else "", out_dtype=out), taken)
 
