@@ -844,7 +844,7 @@ inline unsigned long long padded_bytes(int M, int N, int K, int chunk, int bytes
 // Whether a product whose rows are not whole 16-byte chunks is better off with the kernel that takes any than on padded copies, one or two
 // launches more.  In us: there 3.7 and the longer of one tile's chain of k-tiles and the tiles' work over the chip's CUs; here 9.5, or 8.2 where
 // the result is not copied back, and the copies' bytes, read and written, at 2 TB/s.  Over 203 drawn ragged products of all types and layouts the
-// rule takes 0.80 of the time on copies, the better of the two each time 0.78.  us direct / on copies: fp16 64 x 852 x 64 4.5 / 10.5, 55 x 512 x 93
+// rule takes 0.80 of the time on copies, the better of the two each time 0.78.  us direct / on copies, 16 bits: 64 x 852 x 64 4.5 / 10.5, 55 x 512 x 93
 // 5.6 / 15.3, 64 x 3594 x 314 6.6 / 10.9, 3039 x 336 x 518 10.8 / 13.0; 6 x 383 x 1688 16.4 / 14.4, 1152 x 5120 x 113 19.2 / 10.5, 1618 x 2024 x 485
 // 22.3 / 14.6, 496 x 135 x 3878 24.4 / 18.6.
 inline bool direct_gains(int M, int N, int K, int trans_a, int trans_b, int chunk, int bytes)
