@@ -55,13 +55,15 @@ class _InPython:
 
 
 _calls = None
+_call = runtime.call
 
 
 def _host():
     """The operators' host side in C++ (csrc/host_calls.cpp); each gives None for what it leaves to Python: other than plain GPU tensors,
-    calls under a tracer, a mode or a transform, and calls that are refused."""
+    calls under a tracer, a mode or a transform, and calls that are refused.  A program that puts a function of its own in the place of
+    ``runtime.call``, to record or time what is called, sees these operators' calls in it: they are all made in Python then."""
     global _calls
-    if torch.compiler.is_compiling():
+    if torch.compiler.is_compiling() or runtime.call is not _call:
         return _InPython
     if _calls is None:
         try:

@@ -31,6 +31,16 @@ def test_refused_calls_keep_their_errors():
         ops.lego_group_gemm_fn([x], [])
 
 
+def test_a_function_in_the_place_of_the_call_sees_the_calls(monkeypatch):
+    from lego_amd import ops, runtime
+    monkeypatch.setattr(ops, "_calls", in_cpp := object())
+    assert ops._host() is in_cpp
+    monkeypatch.setattr(runtime, "call", lambda entry, *args: None)
+    assert ops._host() is ops._InPython
+    monkeypatch.undo()
+    assert ops._host() is not ops._InPython
+
+
 def _both(monkeypatch, call, taken=True):
     """What the call gives through C++ and in Python; whether C++ took it."""
     from lego_amd import ops, runtime
@@ -83,6 +93,37 @@ def test_gpu_products(monkeypatch, dtype, out):
                 taken = eight or not (la and M % 8)
                 print(f"host calls {dtype} {M}x{N}x{K} {ta}{tb}", flush=True)
                 _both(monkeypatch, lambda: ops.matmul(a, b, activation="leaky_relu" if M == 16 else "", out_dtype=out), taken)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("in_cpp", [True, False])
+@pytest.mark.parametrize("dtype,M,N,K,ta,tb,uses", [
+    (torch.float8_e5m2, 16, 64, 4096, 0, 0, "parts"), (torch.float8_e5m2, 24, 64, 4096, 0, 1, "parts"), (torch.float8_e4m3fn, 32, 64, 4104, 1, 0, "parts"),
+    (torch.float8_e5m2, 24, 64, 4096, 1, 0, "copies"), (torch.float8_e4m3fn, 32, 64, 4104, 0, 0, "copies"), (torch.float8_e5m2, 32, 64, 4104, 1, 1, "copies"),
+    (torch.float8_e5m2, 33, 17, 65, 0, 0, "nothing"), (torch.float8_e4m3fn, 64, 64, 64, 0, 1, "nothing"), (torch.float16, 16, 64, 4104, 0, 0, "parts"),
+    (torch.float16, 33, 17, 65, 0, 1, "nothing"), (torch.bfloat16, 496, 135, 3878, 0, 0, "copies"), (torch.float16, 16, 4096, 4096, 0, 1, "nothing")])
+def test_gpu_products_bring_a_workspace_only_where_it_is_used(monkeypatch, in_cpp, dtype, M, N, K, ta, tb, uses):
+    """What a call allocates besides its result, on either route: room for sums of whole tiles, for copies of operands with ragged rows, or nothing."""
+    import ctypes
+    from lego_amd import ops, runtime
+    print(f"workspace {dtype} {M}x{N}x{K} {ta}{tb} {'C++' if in_cpp else 'Python'}", flush=True)
+    need, size = ctypes.c_ulonglong(0), torch.finfo(dtype).bits // 8
+    runtime.call("lego_hip_gemm_layout_workspace_bytes", M, N, K, ta, tb, size, ctypes.byref(need))
+    need = need.value
+    assert {"parts": need > 0 and need % 65536 == 0, "copies": need >= size * (M * K + K * N) + 2 * M * N, "nothing": need == 0}[uses]
+    # some two hundred products of -4 .. 4 a sum: below 2048, exact in fp16
+    a = (torch.randint(-2, 3, (K, M) if ta else (M, K), device="cuda") * (torch.rand((K, M) if ta else (M, K), device="cuda") < 200.0 / K)).to(dtype)
+    b = torch.randint(-2, 3, (N, K) if tb else (K, N), device="cuda").to(dtype)
+    a, b = a.t() if ta else a, b.t() if tb else b
+    monkeypatch.setattr(ops, "_calls", runtime.host_calls() if in_cpp else ops._InPython)
+
+    def allocated():
+        stats = torch.cuda.memory_stats()
+        return stats["allocation.all.allocated"], stats["requested_bytes.all.allocated"]
+    before = allocated()
+    c = ops.matmul(a, b)
+    assert tuple(after - first for after, first in zip(allocated(), before)) == (1 + (need > 0), 2 * M * N + need)
+    assert c.shape == (M, N) and torch.equal(c.double(), a.double() @ b.double())
 
 
 @pytest.mark.gpu
