@@ -846,12 +846,17 @@ inline unsigned long long padded_bytes(int M, int N, int K, int chunk, int bytes
 // the result is not copied back, and the copies' bytes, read and written, at 2 TB/s.  Over 203 drawn ragged products of all types and layouts the
 // rule takes 0.80 of the time on copies, the better of the two each time 0.78.  us direct / on copies, 16 bits: 64 x 852 x 64 4.5 / 10.5, 55 x 512 x 93
 // 5.6 / 15.3, 64 x 3594 x 314 6.6 / 10.9, 3039 x 336 x 518 10.8 / 13.0; 6 x 383 x 1688 16.4 / 14.4, 1152 x 5120 x 113 19.2 / 10.5, 1618 x 2024 x 485
-// 22.3 / 14.6, 496 x 135 x 3878 24.4 / 18.6.
+// 22.3 / 14.6, 496 x 135 x 3878 24.4 / 18.6.  Those had sides
+// of up to 8192; taller ones are bound by memory, 2 TB/s there too, and an A beyond the L2s' 32 MB is read again for every column of tiles: 4194305 x 63 x 63
+// 657 / 755, 4194241 x 9 x 130 516 / 789, 1000000 x 63 x 63 137 / 185; 5000000 x 100 x 60 989 / 880, 1000000 x 100 x 60 201 / 196, 100000 x 66 x 200 with B
+// transposed 28.4 / 26.2; 20000 x 1001 x 50, whose A stays in the L2s, 29.4 / 32.5.  (7778 x 110 x 2114 with B transposed is 17.3 / 32.0.)
 inline bool direct_gains(int M, int N, int K, int trans_a, int trans_b, int chunk, int bytes)
 {
   const double tiles = static_cast<double>((M + 63) / 64) * ((N + 63) / 64), depth = (K + 63) / 64;
   const double step = !trans_a && trans_b && K % 8 == 0 ? 0.25 : 0.42;      // both operands k-major: four accesses a lane and k-tile instead of eight
-  const double direct = 3.7 + std::max(step * depth, (1 + 0.9 * step * depth) * tiles / 256);
+  const double a_bytes = static_cast<double>(bytes) * M * K, reads = a_bytes > 32e6 ? (N + 63) / 64 : 1;
+  const double memory = M > 8192 ? (reads * a_bytes + 2.0 * M * N) / 2e6 : 0.0;
+  const double direct = 3.7 + std::max(std::max(step * depth, (1 + 0.9 * step * depth) * tiles / 256), memory);
   const bool back = N % chunk || (trans_a && M % chunk);
   const double results = back ? 0.0 : 2.0 * round_up(M, chunk) * N;
   return direct <= (back ? 9.5 : 8.2) + (padded_bytes(M, N, K, chunk, bytes) - results) / 2e6;

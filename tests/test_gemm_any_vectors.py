@@ -24,13 +24,43 @@ def test_small_ragged_products_need_no_copies_and_deep_ones_do():
     assert _room(64, 64, 64, 0, 0, 2) == 0 and _room(16, 16, 8192, 0, 0, 2) > 0       # whole chunks: parts as before
 
 
-def _entry(dtype, a, b, c, M, N, K, ta, tb, activation=0):
+def _entry(dtype, a, b, c, M, N, K, ta, tb, activation=0, stream=0):
     from lego_amd import runtime
-    stream = torch.cuda.current_stream().cuda_stream
+    stream = torch.cuda.current_stream().cuda_stream if stream == 0 else stream
     if dtype in (E5M2, E4M3):
         runtime.call("lego_hip_gemm_fp8_ex", a, b, c, M, N, K, ta, tb, activation, int(dtype == E5M2), stream)
     else:
         runtime.call("lego_hip_gemm_f16_ex" if dtype == F16 else "lego_hip_gemm_bf16_f16_ex", a, b, c, M, N, K, ta, tb, activation, stream)
+
+
+_TALL = [(F16, 4194305, 63, 63, 0), (BF16, 4194241, 9, 130, 0), (E4M3, 4194310, 60, 33, 1), (E5M2, 4200000, 63, 41, 0)]
+
+
+@pytest.mark.parametrize("dtype,M,N,K,ta", _TALL)
+def test_more_rows_of_tiles_than_a_grid_dimension_has_are_taken(dtype, M, N, K, ta):
+    """Without a GPU a call that is taken gets as far as the launch, which finds no device; one that is refused does not."""
+    from lego_amd import runtime
+    if torch.cuda.is_available():
+        pytest.skip("the operands are addresses of nothing")
+    assert _room(M, N, K, ta, 0, torch.finfo(dtype).bits // 8) == 0 < _room(5000000, 100, 60, 0, 0, 2)      # A of 600 MB in two columns of tiles
+    with pytest.raises(runtime.LegoHipError) as refused:
+        _entry(dtype, 1 << 20, 1 << 21, 1 << 22, M, N, K, ta, 0, stream=None)
+    assert refused.value.code == 100      # hipErrorNoDevice
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,M,N,K,ta", _TALL)
+def test_gpu_more_rows_of_tiles_than_a_grid_dimension_has(dtype, M, N, K, ta):
+    """Whole numbers, exact in every type: every row of a product of 65537 rows of tiles and more, the last one ragged."""
+    from lego_amd import ops
+    print(f"tall {dtype} {M}x{N}x{K} {ta}", flush=True)
+    a = torch.randint(-2, 3, (K, M) if ta else (M, K), device="cuda", dtype=torch.int8).to(dtype)
+    b = torch.randint(-2, 3, (K, N), device="cuda").to(dtype)
+    a = a.t() if ta else a
+    got = ops.matmul(a, b)
+    for first in range(0, M, 1 << 20):
+        rows = slice(first, first + (1 << 20))
+        assert torch.equal(got[rows].float(), a[rows].float() @ b.float()), first
 
 
 def _between(t, dtype, before, after=16):
