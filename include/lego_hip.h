@@ -292,7 +292,8 @@ int lego_hip_gemm_plan(int M, int N, int K, int* plan2);
 
 /* For a product of that kind, of element_bytes = 1 or 2 per operand element: plan2[0] = parts along K, with room for their sums (1: none),
  * plan2[1] = operand buffers of a workgroup in LDS: 4 (one workgroup per CU), or, of 128 x 128 tiles beyond one per CU and of all 256 x 256
- * ones, 2.  Host only. */
+ * ones, 2.  Where 128 rows or columns of a side are 2 GiB and more (K from 2^24 / element_bytes on) the answer is {1, 2}: with room, products of
+ * up to 128 tiles then run in parts of their own rule, two workgroups of two buffers per CU and at most 64 parts a tile.  Host only. */
 int lego_hip_gemm_parts_plan(int M, int N, int K, int element_bytes, int* plan2);
 
 /* The team that lego_hip_softmax_f16 and lego_hip_layernorm_fwd_f16 give a row of a matrix of M rows of N fp16

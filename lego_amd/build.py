@@ -159,7 +159,7 @@ def collect():
                 # 256x256 tiles to fill the chip
                 gs, _ = gemm.emit(**dict(GEMM, bk=GEMM_BK[dtype], bm=GEMM_SMALL_TILE, bn=GEMM_SMALL_TILE),
                                   trans_a=ta, trans_b=tb, dtype=dtype,
-                                  with_grouped=dtype == "f16" and not (ta or tb))
+                                  with_grouped=dtype == "f16" and not (ta or tb), with_splitk=True)
                 units.append(gs)
                 # ... and on four buffers of LDS, one workgroup per CU: for up to as many tiles, or parts of tiles along K, as there are CUs
                 gd, _ = gemm.emit(**dict(GEMM, bk=GEMM_BK[dtype], bm=GEMM_SMALL_TILE, bn=GEMM_SMALL_TILE),
@@ -270,8 +270,8 @@ def collect():
     h += [f"hipError_t lego_gemm_{d}_{v}{t}_launch(const void*, const void*, void*, int, int, int, int, hipStream_t);"
           for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")
           for t in ("", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}", f"_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep")]
-    h += [f"hipError_t lego_gemm_{d}_{v}_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}_deep_splitk_launch(const void*, const void*, void*, int, int, int, int, "
-          "int, float*, hipStream_t);" for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt")]
+    h += [f"hipError_t lego_gemm_{d}_{v}_t{GEMM_SMALL_TILE}x{GEMM_SMALL_TILE}{t}_splitk_launch(const void*, const void*, void*, int, int, int, int, "
+          "int, float*, hipStream_t);" for d in GEMM_DTYPES for v in ("nn", "nt", "tn", "tt") for t in ("", "_deep")]
     h += [
           "hipError_t lego_grouped_gemm_f16_launch(const void* const*, const void* const*, void* const*, "
           "const int*, int, hipStream_t);",

@@ -810,7 +810,9 @@ int gemm_ex(const GemmKernels& k, int element, const void* a, const void* b, voi
 int splitk_parts(int M, int N, int K, int bk)
 {
   const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
-  if (tiles > kDeepTiles / 2 || !deep_offsets(M, N, K, 2 * LEGO_GEMM_BK / bk)) return 1;
+  if (tiles > kDeepTiles / 2) return 1;
+  // chains of 65537 k-tiles and more, past the reach of a descriptor: two workgroups per CU on two buffers
+  if (!deep_offsets(M, N, K, 2 * LEGO_GEMM_BK / bk)) return static_cast<int>(std::min((512 + tiles - 1) / tiles, 64l));
   const long most = std::min(std::min(kDeepTiles / tiles, depth / 2), 64l);
   long best = 1, least = 2400 + 420 * depth;
   for (long parts = 2; parts <= most; ++parts) {
@@ -821,8 +823,17 @@ int splitk_parts(int M, int N, int K, int bk)
   return static_cast<int>(best);
 }
 typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int, int, int, int, float*, hipStream_t);
-#define LEGO_SPLITK(DT) {lego_gemm_##DT##_nn_t128x128_deep_splitk_launch, lego_gemm_##DT##_nt_t128x128_deep_splitk_launch, \
-                         lego_gemm_##DT##_tn_t128x128_deep_splitk_launch, lego_gemm_##DT##_tt_t128x128_deep_splitk_launch}
+struct SplitkKernels {
+  splitk_launcher deep[4], far[4];      // on four buffers; on two, whose instructions have bases of their own and reach 4 GiB from there: index 2*trans_a + trans_b
+  splitk_launcher of(int M, int N, int K, int trans_a, int trans_b, int bytes) const
+  {
+    return (deep_offsets(M, N, K, bytes) ? deep : far)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)];
+  }
+};
+#define LEGO_SPLITK(DT) {{lego_gemm_##DT##_nn_t128x128_deep_splitk_launch, lego_gemm_##DT##_nt_t128x128_deep_splitk_launch,  \
+                          lego_gemm_##DT##_tn_t128x128_deep_splitk_launch, lego_gemm_##DT##_tt_t128x128_deep_splitk_launch}, \
+                         {lego_gemm_##DT##_nn_t128x128_splitk_launch, lego_gemm_##DT##_nt_t128x128_splitk_launch,            \
+                          lego_gemm_##DT##_tn_t128x128_splitk_launch, lego_gemm_##DT##_tt_t128x128_splitk_launch}}
 
 // Operand rows that are not whole 16-byte chunks: the tiled kernels run on zero-padded copies (every side a multiple of `chunk`
 // elements; the padding adds zeros to the sums) and the result is copied back: two more launches and three more passes over
@@ -968,9 +979,9 @@ int lego_hip_gemm_workspace_bytes(int M, int N, int K, unsigned long long* bytes
 int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int M, int N, int K, int trans_a, int trans_b,
                         int activation, void* workspace, unsigned long long workspace_bytes, void* stream)
 {
-  static const splitk_launcher f16[4] = LEGO_SPLITK(f16), bf16[4] = LEGO_SPLITK(bf16), bf16h[4] = LEGO_SPLITK(bf16h);
+  static const SplitkKernels f16 = LEGO_SPLITK(f16), bf16 = LEGO_SPLITK(bf16), bf16h = LEGO_SPLITK(bf16h);
   if (element != 0 && element != 1 && element != 4) return kInvalid;
-  const splitk_launcher parts_by_layout = (element == 0 ? f16 : element == 1 ? bf16 : bf16h)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)];
+  const SplitkKernels& kernels = element == 0 ? f16 : element == 1 ? bf16 : bf16h;
   const auto whole = [&](const void* aa, const void* bb, void* cc, int m, int n, int k) {
     switch (element) {
       case 0: return lego_hip_gemm_f16_ex(aa, bb, cc, m, n, k, trans_a, trans_b, activation, stream);
@@ -991,7 +1002,7 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
     // may want more of them (130 x 136 x 8200 43, 136 x 136 x 8200 33)
     const int parts = N % 8 || K % 8 ? splitk_parts(round_up(m, 8), n, round_up(k, 8), LEGO_GEMM_BK) : splitk_parts(m, n, k, LEGO_GEMM_BK);
     if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
-    return ok_or(parts_by_layout(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
+    return ok_or(kernels.of(m, n, k, trans_a, trans_b, 2)(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
   };
   if (tiled) return product(a, b, c, M, N, K, workspace);
   return on_padded_copies(8, 2, a, b, c, M, N, K, trans_a, trans_b, workspace, stream, product);
@@ -1016,9 +1027,9 @@ int lego_hip_gemm_fp8_workspace_bytes(int M, int N, int K, unsigned long long* b
 }
 
 namespace {
-const splitk_launcher* fp8_parts(int format)
+const SplitkKernels& fp8_parts(int format)
 {
-  static const splitk_launcher e4m3[4] = LEGO_SPLITK(e4m3), e5m2[4] = LEGO_SPLITK(e5m2);
+  static const SplitkKernels e4m3 = LEGO_SPLITK(e4m3), e5m2 = LEGO_SPLITK(e5m2);
   return format == 0 ? e4m3 : e5m2;
 }
 }  // namespace
@@ -1033,8 +1044,7 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
   if (parts < 2 || !tiled || !usable(workspace) || workspace_bytes < parts_bytes(M, N, parts) || rows_columns(M, N, K, trans_a, trans_b, 1))
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
-  const int layout = (trans_a ? 2 : 0) + (trans_b ? 1 : 0);
-  return ok_or(fp8_parts(format)[layout](a, b, c, M, N, K, activation, parts, static_cast<float*>(workspace), as_stream(stream)));
+  return ok_or(fp8_parts(format).of(M, N, K, trans_a, trans_b, 1)(a, b, c, M, N, K, activation, parts, static_cast<float*>(workspace), as_stream(stream)));
 }
 
 // What is used for operands of one layout, shallow products that gain from parts among them; the kernels for few rows and for any shape take
@@ -1079,8 +1089,7 @@ int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N
                           [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK_8BIT);
     if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 1)) return whole(aa, bb, cc, m, n, k);
-    return ok_or(fp8_parts(format)[(trans_a ? 2 : 0) + (trans_b ? 1 : 0)](aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums),
-                                                                         as_stream(stream)));
+    return ok_or(fp8_parts(format).of(m, n, k, trans_a, trans_b, 1)(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
   });
 }
 
@@ -1632,7 +1641,7 @@ int lego_hip_gemm_plan(int M, int N, int K, int* plan2)
 int lego_hip_gemm_parts_plan(int M, int N, int K, int element_bytes, int* plan2)
 {
   if (plan2 == nullptr || M <= 0 || N <= 0 || K <= 0 || (element_bytes != 1 && element_bytes != 2)) return kInvalid;
-  plan2[0] = splitk_parts(M, N, K, element_bytes == 1 ? LEGO_GEMM_BK_8BIT : LEGO_GEMM_BK);
+  plan2[0] = deep_offsets(M, N, K, element_bytes) ? splitk_parts(M, N, K, element_bytes == 1 ? LEGO_GEMM_BK_8BIT : LEGO_GEMM_BK) : 1;
   plan2[1] = plan2[0] > 1 || deep_tiles(M, N, K, element_bytes) ? 4 : 2;
   return 0;
 }
