@@ -243,3 +243,34 @@ def test_gpu_values_beyond_the_near_form(n, where):
     want = _wrapped(ref, m, penalty)
     got = ops.needleman_wunsch(ref.cuda(), m.cuda(), penalty)
     assert torch.equal(got.cpu(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("n", [192, 320, 1088])
+@pytest.mark.parametrize("where", ["highest", "above", "lowest", "below", "growing", "border", "left", "penalty", "penalty above"])
+def test_gpu_bounds_of_the_near_form(n, where):
+    """Either side of each bound up to which the kernel keeps its shorter form, and values that pass the bound, or the type's end, in the course of it."""
+    from lego_amd import ops
+    print(f"needleman-wunsch n={n}, bound: {where}", flush=True)
+    g = torch.Generator().manual_seed(11 * n)
+    penalty = 10
+    ref = torch.randint(-4, 12, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    m = torch.randint(-99, 99, (n + 1, n + 1), generator=g, dtype=torch.int32)
+    some = torch.rand(n + 1, n + 1, generator=g) < 0.3
+    if where in ("highest", "above"):
+        ref = torch.where(some, (1 << 23) + (where == "above"), ref)
+    elif where in ("lowest", "below"):
+        ref = torch.where(some, -(1 << 30) - (where == "below"), ref)
+        m[n // 2:, 0] -= 1 << 29      # a sum with the lowest score that is still inside the type
+    elif where == "growing":          # a whole diagonal of matches from 2^28 on: past 2^29 after 128 rows, past the type's end after 896
+        ref, m = torch.full_like(ref, 1 << 21), m + (1 << 28)
+    elif where == "border":
+        m[0, n // 2], m[0, n - 1] = (1 << 29) - penalty * n, (1 << 29) + 1
+    elif where == "left":
+        m[n // 3, 0], m[n - 40, 0], m[n - 20, 0] = -(1 << 29), (1 << 29) - penalty * n, (1 << 29) + 1
+    else:
+        penalty = (1 << 27) // (n + 256) + (where == "penalty above")
+        m[:, 0] = m[0, :] = -penalty * torch.arange(n + 1, dtype=torch.int32)
+    want = _wrapped(ref, m, penalty)
+    got = ops.needleman_wunsch(ref.cuda(), m.cuda(), penalty)
+    assert torch.equal(got.cpu(), want)
