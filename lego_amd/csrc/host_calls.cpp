@@ -151,7 +151,8 @@ PyObject* matmul(PyObject*, PyObject* const* args, Py_ssize_t count)
 // group(as, bs): the grouped launch of two lists of row-major fp16 matrices
 PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t count)
 {
-  constexpr int kMost = 64;       // as many as a launch carries
+  HANDLE_TH_ERRORS
+  constexpr int kMost = 64;       // pointers kept on the stack; longer lists are Python's
   if (count != 2 || !nothing_in_between() || !PyList_CheckExact(args[0]) || !PyList_CheckExact(args[1])) return nothing();
   const Py_ssize_t groups = PyList_GET_SIZE(args[0]);
   if (groups == 0 || groups > kMost || PyList_GET_SIZE(args[1]) != groups) return nothing();
@@ -165,7 +166,7 @@ PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t count)
     const int N = (int)b->size(1), K = (int)a->size(1);
     ragged = ragged || N % 8 || K % 8;
     if (ragged && groups == 1) return nothing();       // a product of its own
-    deep = deep || ((N % 8 || K % 8) && K > 1984);
+    deep = deep || ((N % 8 || K % 8) && K > 1984);      // 31 k-tiles: lego_hip_grouped_gemm_f16_apart looks at none of fewer
     as.push_back(*a);
     bs.push_back(*b);
     sizes.insert(sizes.end(), {(int)a->size(0), N, K});
@@ -173,7 +174,6 @@ PyObject* group(PyObject*, PyObject* const* args, Py_ssize_t count)
   unsigned long long need = 0;
   int limit = 0;
   if (lego_hip_grouped_gemm_f16_room(sizes.data(), (int)groups, &need, &limit) != 0 || (deep && limit == 0)) return nothing();      // some may be products of their own
-  HANDLE_TH_ERRORS
   {
     pybind11::gil_scoped_release nothing_here_needs_it;
     const void *pa[kMost], *pb[kMost];
