@@ -947,7 +947,7 @@ int lego_hip_gemm_bf16_f16_ex(const void* a, const void* b, void* c, int M, int 
 
 namespace {
 // Room that a product of this kind uses: for zero-padded copies of both operands and of the result, N or K not being a multiple of 8 (M only
-// matters as the row length of a transposed A; that case alone stays with the one-element kernel), and for its sums, `parts(M, N, K)` of them.
+// matters as the row length of a transposed A; that case alone stays with the kernel for any shape), and for its sums, `parts(M, N, K)` of them.
 extern "C++" template <class Parts>
 unsigned long long room_16bit(int M, int N, int K, const Parts& parts)
 {
@@ -1325,12 +1325,11 @@ GroupedPlan grouped_plan_uncached(const int* sizes3, int groups)
   double least = kPartGain * plan.time;
   for (const int limit : {4, 6, 8, 12, 16, 24, 32, 48}) {
     if (!deep || limit >= depth[0]) break;      // the deepest problem is the first
-    long count[LEGO_GROUPED_MAX_GROUPS], units = 0, sums = 0;
+    long count[LEGO_GROUPED_MAX_GROUPS], sums = 0;
     double length[LEGO_GROUPED_MAX_GROUPS], cost[LEGO_GROUPED_MAX_GROUPS];
     for (int s = 0; s < groups; ++s) {
       const long d = static_cast<long>(depth[s]), parts = (d + limit - 1) / limit, per = (d + parts - 1) / parts, used = (d + per - 1) / per;
       if (used > 1) sums += used * small[s];
-      units += used * small[s];
       const double t = kDeepStep * per + (used > 1 ? kPartOverhead : kDeepOverhead);
       int j = s;
       while (j > 0 && length[j - 1] < per) { length[j] = length[j - 1]; cost[j] = cost[j - 1]; count[j] = count[j - 1]; --j; }
@@ -1370,7 +1369,7 @@ GroupedPlan grouped_plan(const int* sizes3, int groups)
 }
 
 // 0: every problem fits the tiled kernels (one launch); 2: the arguments are valid but some problem needs
-// the element-wise kernel (N or K not in whole 16-byte chunks, a base that is not 16-byte aligned);
+// the kernel for any shape (N or K not in whole 16-byte chunks, a base that is not 16-byte aligned);
 // kInvalid otherwise
 int grouped_check(const void* const* a, const void* const* b, void* const* c, const int* sizes3, int groups)
 {
