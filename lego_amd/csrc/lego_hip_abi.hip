@@ -822,6 +822,17 @@ int splitk_parts(int M, int N, int K, int bk)
   }
   return static_cast<int>(best);
 }
+// As many of those parts as a launch takes: three quarters where all would put a workgroup on every CU, each reading rows of a k-major operand of up to 64
+// rows or columns against a large one from a multiple of 32 k-tiles on: they are then a multiple of 4 KiB apart in every row, and what they ask memory for at a time
+// falls on few of its channels.  us from memory (from the caches), 256 workgroups / 192: fp16 24 x 8192 x 8192 with B transposed 39.0 (24.5) / 33.2 (24.5),
+// 64 x 8192 x 8192 42.0 (27.5) / 35.0 (27.2), 8192 x 64 x 8192 39.8 (26.3) / 33.2 (26.0), e5m2 24 x 8192 x 16384 38.9 / 33.3; parts of 20 k-tiles, 40 x 8192 x 5120, 22.0 / 23.0, of 16,
+// 24 x 4096 x 8192, 17.8 / 18.4, and 128 rows, 128 x 8192 x 16384, 61.6 / 65.2 from the caches, stay whole rounds.
+int launched_parts(int parts, int M, int N, int K, int trans_a, int trans_b, int bk)
+{
+  const long tiles = static_cast<long>((M + 127) / 128) * ((N + 127) / 128), depth = (K + bk - 1) / bk;
+  const bool few = (M <= 64 && trans_b) || (N <= 64 && !trans_a);
+  return few && parts >= 4 && parts * tiles == kDeepTiles && (depth + parts - 1) / parts % 32 == 0 ? parts - parts / 4 : parts;
+}
 typedef hipError_t (*splitk_launcher)(const void*, const void*, void*, int, int, int, int, int, float*, hipStream_t);
 struct SplitkKernels {
   splitk_launcher deep[4], far[4];      // on four buffers; on two, whose instructions have bases of their own and reach 4 GiB from there: index 2*trans_a + trans_b
@@ -1002,7 +1013,7 @@ int lego_hip_gemm_ex_ws(int element, const void* a, const void* b, void* c, int 
     // may want more of them (130 x 136 x 8200 43, 136 x 136 x 8200 33)
     const int parts = N % 8 || K % 8 ? splitk_parts(round_up(m, 8), n, round_up(k, 8), LEGO_GEMM_BK) : splitk_parts(m, n, k, LEGO_GEMM_BK);
     if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 2)) return whole(aa, bb, cc, m, n, k);
-    return ok_or(kernels.of(m, n, k, trans_a, trans_b, 2)(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
+    return ok_or(kernels.of(m, n, k, trans_a, trans_b, 2)(aa, bb, cc, m, n, k, activation, launched_parts(parts, m, n, k, trans_a, trans_b, LEGO_GEMM_BK), static_cast<float*>(sums), as_stream(stream)));
   };
   if (tiled) return product(a, b, c, M, N, K, workspace);
   return on_padded_copies(8, 2, a, b, c, M, N, K, trans_a, trans_b, workspace, stream, product);
@@ -1044,7 +1055,7 @@ int lego_hip_gemm_fp8_ex_ws(const void* a, const void* b, void* c, int M, int N,
   if (parts < 2 || !tiled || !usable(workspace) || workspace_bytes < parts_bytes(M, N, parts) || rows_columns(M, N, K, trans_a, trans_b, 1))
     return lego_hip_gemm_fp8_ex(a, b, c, M, N, K, trans_a, trans_b, activation, format, stream);
   if (activation != 0 && activation != 1) return kInvalid;
-  return ok_or(fp8_parts(format).of(M, N, K, trans_a, trans_b, 1)(a, b, c, M, N, K, activation, parts, static_cast<float*>(workspace), as_stream(stream)));
+  return ok_or(fp8_parts(format).of(M, N, K, trans_a, trans_b, 1)(a, b, c, M, N, K, activation, launched_parts(parts, M, N, K, trans_a, trans_b, LEGO_GEMM_BK_8BIT), static_cast<float*>(workspace), as_stream(stream)));
 }
 
 // What is used for operands of one layout, shallow products that gain from parts among them; the kernels for few rows and for any shape take
@@ -1089,7 +1100,7 @@ int lego_hip_gemm_fp8_padded(const void* a, const void* b, void* c, int M, int N
                           [&](const void* aa, const void* bb, void* cc, int m, int n, int k, void* sums) {
     const int parts = splitk_parts(m, n, k, LEGO_GEMM_BK_8BIT);
     if (parts < 2 || rows_columns(m, n, k, trans_a, trans_b, 1)) return whole(aa, bb, cc, m, n, k);
-    return ok_or(fp8_parts(format).of(m, n, k, trans_a, trans_b, 1)(aa, bb, cc, m, n, k, activation, parts, static_cast<float*>(sums), as_stream(stream)));
+    return ok_or(fp8_parts(format).of(m, n, k, trans_a, trans_b, 1)(aa, bb, cc, m, n, k, activation, launched_parts(parts, m, n, k, trans_a, trans_b, LEGO_GEMM_BK_8BIT), static_cast<float*>(sums), as_stream(stream)));
   });
 }
 

@@ -41,3 +41,17 @@ def test_gpu_far_products(dtype, M, N, K, ta, tb):
     a, b = a.t() if ta else a, b.t() if tb else b
     want = sum(a[:, k:k + (1 << 20)].float() @ b[k:k + (1 << 20)].float() for k in range(0, K, 1 << 20))
     assert torch.equal(ops.matmul(a, b).float(), want)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("dtype,M,N,K,ta,tb", [(F16, 24, 8192, 8192, 0, 1), (F16, 64, 8192, 8160, 1, 1), (F16, 8192, 40, 8192, 0, 0), (E5M2, 24, 8192, 16384, 0, 1),
+                                               (F16, 24, 8191, 8185, 0, 1)])
+def test_gpu_three_quarters_of_the_parts(dtype, M, N, K, ta, tb):
+    """Parts of a multiple of 32 k-tiles along k-major operands: the launch takes fewer of them than there is room for."""
+    from lego_amd import ops
+    print(f"parts {dtype} {M}x{N}x{K} {ta}{tb}", flush=True)
+    shape = (K, M) if ta else (M, K)
+    a = (torch.randint(-1, 2, shape, device="cuda", dtype=torch.int8) * (torch.rand(shape, device="cuda") < 300.0 / K)).to(dtype)
+    b = torch.randint(-2, 3, (N, K) if tb else (K, N), device="cuda", dtype=torch.int8).to(dtype)
+    a, b = a.t() if ta else a, b.t() if tb else b
+    assert torch.equal(ops.matmul(a, b).float(), a.float() @ b.float())
