@@ -877,11 +877,16 @@ inline bool direct_gains(int M, int N, int K, int trans_a, int trans_b, int chun
   const double tiles = static_cast<double>((M + 63) / 64) * ((N + 63) / 64), depth = (K + 63) / 64;
   const double step = !trans_a && trans_b && K % 8 == 0 ? 0.25 : 0.42;      // both operands k-major: four accesses a lane and k-tile instead of eight
   const double a_bytes = static_cast<double>(bytes) * M * K, reads = a_bytes > 32e6 ? (N + 63) / 64 : 1;
+  // A large A in whole chunks is no copy: the product reads it where it is, at 4.5 TB/s, and here its tiles are bound by how often it is read.  us direct / on copies
+  // from memory: bf16 6174 x 68 x 5808 with B transposed 41.9 / 31.2, f16 7452 x 277 x 5680 115 / 68, bf16 6831 x 315 x 3176 with A stored row-major first 89 / 61.
+  const bool in_place = a_bytes > 32e6 && K % chunk == 0 && !(trans_a && M % chunk);
+  const double work = in_place && step < 0.42 ? 0.45 : 0.9 * step;
   const double memory = M > 8192 ? (reads * a_bytes + 2.0 * M * N) / 2e6 : 0.0;
-  const double direct = 3.7 + std::max(std::max(step * depth, (1 + 0.9 * step * depth) * tiles / 256), memory);
+  const double direct = 3.7 + std::max(std::max(step * depth, (1 + work * depth) * tiles / 256), memory);
   const bool back = N % chunk || (trans_a && M % chunk);
   const double results = back ? 0.0 : 2.0 * round_up(M, chunk) * N;
-  return direct <= (back ? 9.5 : 8.2) + (padded_bytes(M, N, K, chunk, bytes) - results) / 2e6;
+  const double copied = padded_bytes(M, N, K, chunk, bytes) - results - (in_place ? static_cast<double>(bytes) * round_up(M, chunk) * K : 0.0);
+  return direct <= (back ? 9.5 : 8.2) + copied / 2e6 + (in_place ? a_bytes / 4.5e6 : 0.0);
 }
 inline unsigned long long parts_bytes(int M, int N, int parts)
 {

@@ -24,3 +24,12 @@ def test_sums_stay_in_the_workspace(M, N, K):
                      torch.cuda.current_stream().cuda_stream)
         assert torch.equal(c.cpu().double(), a.double() @ b.double().t())
         assert (ws[need.value:] == 85).all()
+
+
+def test_a_large_operand_in_whole_chunks_is_no_copy():
+    """Ragged columns against a large A that is read where it is: on copies of the rest, not by the kernel for any shape; a ragged K keeps that one."""
+    from lego_amd import runtime
+    need = ctypes.c_ulonglong(0)
+    for M, N, K, copies in ((6174, 68, 5808, True), (7452, 277, 5680, True), (6831, 315, 3176, True), (7778, 110, 2114, False), (1073, 427, 2368, False)):
+        runtime.call("lego_hip_gemm_layout_workspace_bytes", M, N, K, 0, 1, 2, ctypes.byref(need))
+        assert (need.value > 0) == copies, (M, N, K)
